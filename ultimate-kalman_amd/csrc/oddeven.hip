@@ -129,7 +129,6 @@ __global__ void __launch_bounds__(((2 * NB + 63) / 64) * 64)
     }
     if (tid < n) xout[oj * n + tid] = r;
   }
-  if (!cov) return;
 
   /* ---- W = T Sigma: lane q < 2n owns column q (NB rows, zero beyond n) ---- */
   const int q = tid;
@@ -267,6 +266,31 @@ __device__ __forceinline__ double lane_bcast(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
+/* R^{-1} r on one wave: lane i < n holds r_i and rinv_i = 1 / R_ii, R upper
+ * triangular in LDS (rows 0 .. n-1 of the first n columns read, ld). The
+ * solved entries go from lane to lane by readlane, and R's entries, which do
+ * not depend on them, are read ahead in groups; a shuffle through LDS and an
+ * LDS read per step made the chain several times as long. */
+template <int NB>
+__device__ __forceinline__ double wave_back_solve(double r, const double* R, int ld, double rinv, int n, int i) {
+  constexpr int PF = 8;
+  const int ii = i < n ? i : 0;
+  for (int q0 = (n - 1) / PF * PF; q0 >= 0; q0 -= PF) {
+    double rr[PF];
+#pragma unroll
+    for (int t = 0; t < PF; ++t) rr[t] = R[ii + (q0 + t < n ? q0 + t : n - 1) * ld];
+#pragma unroll
+    for (int t = PF - 1; t >= 0; --t) {
+      const int q = q0 + t;
+      if (q < n) {
+        const double xq = lane_bcast(r * rinv, q);
+        r = (i == q) ? xq : (i < q ? fma(-rr[t], xq, r) : r);
+      }
+    }
+  }
+  return r;
+}
+
 /*
  * x_j = R^{-1} (cf - Bt x_{j-1} - Y x_{j+1}) for one even step per wave: lane
  * i owns row i. Bt and Y stream column by column (coalesced), the
@@ -291,28 +315,38 @@ __global__ void __launch_bounds__(64) k_estimate(uk_level_t lv, uk_factors_t fac
   const double* Rg = fac.R + ev * nn;
   const double* Bg = fac.Bt + ev * nn;
   const double* Yg = fac.Y + ev * nn;
+  /* lanes beyond the block re-read its last row; the absent neighbours' blocks
+   * are stored as zeros (j = 0: B~, a lone step: Y) and their estimates read
+   * as zero: no branch stands between the loads */
   const bool row = i < n;
-  double rrow[NB];
-#pragma unroll
-  for (int q = 0; q < NB; ++q) rrow[q] = (row && q < n && q >= i) ? Rg[i + (int64_t)q * n] : 0.0;
-  const double rinv = row ? 1.0 / Rg[i + (int64_t)i * n] : 0.0;
+  const int ii = row ? i : n - 1;
   const double xm = (has_m && row) ? xout[om * n + i] : 0.0;
   const double xp = (has_p && row) ? xout[op * n + i] : 0.0;
-  double r = row ? fac.cf[ev * n + i] : 0.0;
-#pragma unroll 8
-  for (int q = 0; q < NB; ++q) {
-    if (q < n) {
-      const double b = (has_m && row) ? Bg[i + (int64_t)q * n] : 0.0;
-      const double y = (has_p && row) ? Yg[i + (int64_t)q * n] : 0.0;
-      r = fma(-b, lane_bcast(xm, q), r);
-      r = fma(-y, lane_bcast(xp, q), r);
+  double r = fac.cf[ev * n + ii];
+  double rrow[NB];
+#pragma unroll
+  for (int q = 0; q < NB; ++q) rrow[q] = Rg[ii + (int64_t)(q < n ? q : n - 1) * n];
+  const double rinv = 1.0 / Rg[ii + (int64_t)ii * n];
+  constexpr int PF = 8;
+  for (int q0 = 0; q0 < n; q0 += PF) {
+    double b[PF], y[PF];
+#pragma unroll
+    for (int t = 0; t < PF; ++t) {
+      const int64_t at = ii + (int64_t)(q0 + t < n ? q0 + t : n - 1) * n;
+      b[t] = Bg[at];
+      y[t] = Yg[at];
+    }
+#pragma unroll
+    for (int t = 0; t < PF; ++t) { /* xm and xp are zero in the lanes from n on */
+      r = fma(-b[t], lane_bcast(xm, q0 + t), r);
+      r = fma(-y[t], lane_bcast(xp, q0 + t), r);
     }
   }
 #pragma unroll
   for (int q = NB - 1; q >= 0; --q) {
     if (q < n) {
       const double xq = lane_bcast(r * rinv, q);
-      r = (i == q) ? xq : fma(-rrow[q], xq, r);
+      r = (i == q) ? xq : (i < q ? fma(-rrow[q], xq, r) : r); /* rows beyond q are solved */
     }
   }
   if (row) xout[oj * n + i] = r;
@@ -406,43 +440,61 @@ __global__ void __launch_bounds__(NB * 8, (NB == 48 ? 3 : 1))
   {
     const int rb = w / TB;             /* row block of Sigma: 0 (u_{j-1}) or 1 (u_{j+1}) */
     const int ri = (w % TB) * 16 + li; /* row within the block */
-    const double* src0 = rb == 0 ? Sout + om * nn : XTup + sup * nn; /* S_mm | S_pm */
-    const double* src1 = rb == 0 ? Xup + sup * nn : Sout + op * nn;  /* S_mp | S_pp */
-    const bool live0 = rb == 0 ? has_m : (has_m && has_p);
-    const bool live1 = rb == 0 ? (has_m && has_p) : has_p;
+    const bool both = has_m && has_p;
+    const bool live0 = rb == 0 ? has_m : both;
+    const bool live1 = rb == 0 ? both : has_p;
+    /* S_mm | S_pm, and S_mp | S_pp; what is absent or outside the block reads
+     * R's first entry and becomes zero, without a branch */
+    const double* src0 = !live0 ? Rg : (rb == 0 ? Sout + om * nn : XTup + sup * nn);
+    const double* src1 = !live1 ? Rg : (rb == 0 ? Xup + sup * nn : Sout + op * nn);
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
       const int cb = t * 4 / NB, ci = t * 4 + lk - cb * NB;
-      sig[t] = 0.0;
-      if ((cb == 0 ? live0 : live1) && ri < n && ci < n) sig[t] = (cb == 0 ? src0 : src1)[ri + (int64_t)ci * n];
+      const bool in = (cb == 0 ? live0 : live1) && ri < n && ci < n;
+      const double x = (cb == 0 ? src0 : src1)[in ? ri + (int64_t)ci * n : 0];
+      sig[t] = in ? x : 0.0;
     }
   }
   constexpr int RPER = (NB * NB + NT - 1) / NT;
-  double rpre[RPER];
+  static_assert(RPER * NT == NB * NB, "the workgroup covers a block in whole passes");
+  double rpre[RPER], bpre[RPER], ypre[RPER];
 #pragma unroll
   for (int e = 0; e < RPER; ++e) {
     const int idx = tid + e * NT;
     const int i = idx % NB, c = idx / NB;
-    rpre[e] = (idx < NB * NB && i < n && c < n) ? Rg[i + c * n] : (i == c ? 1.0 : 0.0);
-  }
-  for (int idx = tid; idx < NB * NB; idx += NT) {
-    const int i = idx % NB, c = idx / NB;
     const bool in = i < n && c < n;
-    T[i + c * LD] = (in && has_m) ? Bg[i + c * n] : 0.0;
-    T[NB * LD + i + c * LD] = (in && has_p) ? Yg[i + c * n] : 0.0;
+    const int at = in ? i + c * n : 0;
+    const double x = Rg[at], b = Bg[at], y = Yg[at];
+    rpre[e] = in ? x : (i == c ? 1.0 : 0.0);
+    bpre[e] = in && has_m ? b : 0.0;
+    ypre[e] = in && has_p ? y : 0.0;
   }
-  for (int i = tid; i < NB; i += NT) {
-    sh.xm[i] = (has_m && i < n) ? xout[om * n + i] : 0.0;
-    sh.xp[i] = (has_p && i < n) ? xout[op * n + i] : 0.0;
+  double cf = 0.0, xmv = 0.0, xpv = 0.0;
+  if (tid < n) {
+    cf = fac.cf[ev * n + tid];
+    xmv = has_m ? xout[om * n + tid] : 0.0;
+    xpv = has_p ? xout[op * n + tid] : 0.0;
+  }
+#pragma unroll
+  for (int e = 0; e < RPER; ++e) {
+    const int idx = tid + e * NT;
+    const int i = idx % NB, c = idx / NB;
+    T[i + c * LD] = bpre[e];
+    T[NB * LD + i + c * LD] = ypre[e];
+  }
+  if (tid < NB) {
+    sh.xm[tid] = xmv;
+    sh.xp[tid] = xpv;
   }
   __syncthreads();
-  if (tid < NB) {
-    double r = 0.0;
-    if (tid < n) {
-      r = fac.cf[ev * n + tid];
-      for (int q = 0; q < n; ++q) r -= T[tid + q * LD] * sh.xm[q] + T[NB * LD + tid + q * LD] * sh.xp[q];
+  if (tid < NB) { /* rows from n on are zero */
+    double r0 = cf, r1 = 0.0;
+#pragma unroll 8
+    for (int q = 0; q < NB; ++q) {
+      r0 = fma(-T[tid + q * LD], sh.xm[q], r0);
+      r1 = fma(-T[NB * LD + tid + q * LD], sh.xp[q], r1);
     }
-    sh.r[tid] = r;
+    sh.r[tid] = r0 + r1;
   }
 
   /* ---- W^T = Sigma T^T: wave w owns rows [16w, 16w + 16) of W^T ---- */
@@ -529,12 +581,8 @@ __global__ void __launch_bounds__(NB * 8, (NB == 48 ? 3 : 1))
       }
     }
     if (w == 1) {
-      double r = lane < n ? sh.r[lane] : 0.0;
-      for (int q = n - 1; q >= 0; --q) {
-        const double xq = __shfl(r, q) * sh.rinv[q];
-        if (lane == q) r = xq;
-        else if (lane < q) r -= Rs[lane + q * LD] * xq;
-      }
+      const int ll = lane < n ? lane : 0;
+      const double r = wave_back_solve<NB>(lane < n ? sh.r[ll] : 0.0, Rs, LD, sh.rinv[ll], n, lane);
       if (lane < n) xout[oj * n + lane] = r;
     }
     __syncthreads(); /* R's diagonal blocks consumed */
@@ -661,6 +709,205 @@ __global__ void __launch_bounds__(NB * 8, (NB == 48 ? 3 : 1))
       for (int r = 0; r < 4; ++r) {
         const int i = ti * 16 + 4 * r + lk;
         if (i < n && jc < n) S[jc + (int64_t)i * n] = acc[r]; /* S symmetric: S[i][jc] stored as its transpose */
+      }
+    }
+  }
+}
+
+/*
+ * The back substitution with covariances for n <= 16: one even step per wave,
+ * four waves per workgroup that share nothing, KS = ceil(n / 4). Every block
+ * is one 16 x 16 matrix-core tile, and the products are ordered so that an
+ * accumulator (lane (li, lk) holds rows 4 r + lk of column li) is the next
+ * product's operand as it stands: as B for itself, as A for its transpose.
+ *   W^T = Sigma T^T (two tiles), N = I + T W^T,
+ *   K^T = N R^{-T} (N symmetric: its accumulator is the A operand),
+ *   S = R^{-1} K^T, U_1 = R^{-1} W_1, U_2^T = W_2^T R^{-T}.
+ * Blocks are read from HBM straight into fragments, S and X are written from
+ * accumulators. Only R (for the substitution), R^{-1} and, where cross
+ * covariances are wanted, W^T turn round in LDS, within the wave: there is no
+ * barrier. Lanes 0..15 substitute the unit vectors and lane 16 the
+ * estimate's right-hand side in the same instructions.
+ * Only X[s] = Cov(u_s, u_{s+1}) is kept between levels; its transpose is read
+ * across rows of a 2 KB block instead of being stored a second time.
+ * Most levels of a smoothing have few steps, and there the kernel's length is
+ * one step's chain: at n = 16 it was 25.8 us in the vector form (one column
+ * per lane and three 16-step substitutions one after another).
+ */
+template <int KS>
+struct BackSmallShared {
+  static constexpr int LD = 18; /* even: pairs of a column are read in 16 bytes */
+  double R[4 * KS * LD];        /* R, then R^{-1}, column-major */
+  double W[2][16 * LD];         /* W^T's halves, column by column */
+  double rinv[16];
+  double r[16];                 /* cf - Bt x_{j-1} - Y x_{j+1}, then x_j */
+};
+
+template <int KS, bool DIAG>
+__global__ void __launch_bounds__(256)
+    k_backsub_small(uk_level_t lv, uk_factors_t fac, double* __restrict__ xout, double* __restrict__ Sout,
+                    const double* __restrict__ Xup, double* __restrict__ Xcur, int n) {
+  constexpr int LD = BackSmallShared<KS>::LD, NK = 4 * KS;
+  __shared__ __align__(16) BackSmallShared<KS> shw[4];
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  BackSmallShared<KS>& sh = shw[threadIdx.x >> 6];
+  const int64_t ev = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (ev >= lv.evens) return; /* the same for the whole wave; no barrier follows */
+  const int p = (int)find_problem(lv.even_start, lv.nprob, ev);
+  const int64_t u = ev - lv.even_start[p];
+  const int64_t j = 2 * u;
+  const int64_t L = lv.L[p];
+  const bool has_m = j > 0, has_p = j + 1 < L;
+  const int64_t nn = (int64_t)n * n;
+  const int64_t ob = lv.orig_start[lv.prob[p]];
+  const int64_t stride = (int64_t)1 << lv.level;
+  const int64_t oj = ob + (j + 1) * stride - 1;
+  const int64_t om = has_m ? ob + j * stride - 1 : oj; /* an absent neighbour's loads go to valid places and read as 0 */
+  const int64_t op = has_p ? ob + (j + 2) * stride - 1 : oj;
+  const int64_t sj = lv.step_start[p] + j;
+  const int64_t sup = lv.next_start[p] + (j >> 1) - 1;
+  const double* Rg = fac.R + ev * nn;
+  const double* Xg = (has_m && has_p) ? Xup + sup * nn : Rg;
+
+  /* fragment ks of a block: element (li, 4 ks + lk), or its transpose's */
+  int at[KS], att[KS];
+  bool in[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int c = 4 * ks + lk;
+    in[ks] = li < n && c < n;
+    at[ks] = in[ks] ? li + c * n : 0;
+    att[ks] = in[ks] ? c + li * n : 0;
+  }
+  double fR[KS], fB[KS], fY[KS], fm[KS], fp[KS], fx[KS], fxt[KS], xm[KS], xp[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int c = 4 * ks + lk, cc = c < n ? c : 0;
+    fR[ks] = Rg[at[ks]];
+    fB[ks] = fac.Bt[ev * nn + at[ks]];
+    fY[ks] = fac.Y[ev * nn + at[ks]];
+    xm[ks] = xout[om * n + cc];
+    xp[ks] = xout[op * n + cc];
+    fm[ks] = Sout[om * nn + at[ks]];
+    fp[ks] = Sout[op * nn + at[ks]];
+    fx[ks] = Xg[at[ks]];
+    fxt[ks] = Xg[att[ks]];
+  }
+  const double cf = fac.cf[ev * n + (li < n ? li : 0)];
+  const bool both = has_m && has_p;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int c = 4 * ks + lk;
+    fR[ks] = in[ks] ? fR[ks] : (li == c ? 1.0 : 0.0);
+    fB[ks] = in[ks] && has_m ? fB[ks] : 0.0;
+    fY[ks] = in[ks] && has_p ? fY[ks] : 0.0;
+    fm[ks] = in[ks] && has_m ? fm[ks] : 0.0;
+    fp[ks] = in[ks] && has_p ? fp[ks] : 0.0;
+    fx[ks] = in[ks] && both ? fx[ks] : 0.0;
+    fxt[ks] = in[ks] && both ? fxt[ks] : 0.0;
+    xm[ks] = c < n && has_m ? xm[ks] : 0.0;
+    xp[ks] = c < n && has_p ? xp[ks] : 0.0;
+  }
+
+  /* R and its diagonal's reciprocals to LDS; the right-hand side */
+  double r = 0.0;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int c = 4 * ks + lk;
+    if (li < NK) sh.R[c * LD + li] = fR[ks];
+    if (li == c) sh.rinv[c] = 1.0 / fR[ks];
+    r = fma(fB[ks], xm[ks], r);
+    r = fma(fY[ks], xp[ks], r);
+  }
+  r += __shfl_xor(r, 16);
+  r += __shfl_xor(r, 32);
+  if (lane < 16) sh.r[li] = li < n ? cf - r : 0.0;
+  wave_lds_sync();
+
+  /* W^T = Sigma T^T: rows of u_{j-1}, then rows of u_{j+1} */
+  dx4 wt = dx4{0.0, 0.0, 0.0, 0.0}, wb = wt;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    wt = mfma16(fm[ks], fB[ks], wt);
+    wb = mfma16(fxt[ks], fB[ks], wb);
+  }
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    wt = mfma16(fx[ks], fY[ks], wt);
+    wb = mfma16(fp[ks], fY[ks], wb);
+  }
+
+  /* lanes 0..15: columns of R^{-1}; lane 16: the estimate */
+  double v[NK];
+#pragma unroll
+  for (int i = 0; i < NK; ++i) v[i] = lane == 16 ? sh.r[i] : (i == lane ? 1.0 : 0.0);
+#pragma unroll
+  for (int q = NK - 1; q >= 0; --q) {
+    const double xq = v[q] * sh.rinv[q];
+    v[q] = xq;
+    const double2* Rq = reinterpret_cast<const double2*>(&sh.R[q * LD]);
+#pragma unroll
+    for (int i = 0; i < q; i += 2) {
+      const double2 t = Rq[i / 2];
+      v[i] = fma(-t.x, xq, v[i]);
+      if (i + 1 < q) v[i + 1] = fma(-t.y, xq, v[i + 1]);
+    }
+  }
+
+  /* N = I + T W^T */
+  dx4 nacc;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) nacc[i] = (4 * i + lk == li && li < n) ? 1.0 : 0.0;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) nacc = mfma16(fB[ks], wt[ks], nacc);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) nacc = mfma16(fY[ks], wb[ks], nacc);
+
+  wave_lds_sync(); /* R consumed */
+  if (lane < NK) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) sh.R[lane * LD + i] = v[i];
+  }
+  if (lane == 16) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) sh.r[i] = v[i];
+  }
+  if (Xcur) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sh.W[0][li * LD + 4 * i + lk] = wt[i];
+      sh.W[1][li * LD + 4 * i + lk] = wb[i];
+    }
+  }
+  wave_lds_sync();
+  if (lane < n) xout[oj * n + lane] = sh.r[lane];
+  double ri[KS]; /* R^{-1}(li, 4 ks + lk): A of R^{-1}, B of R^{-T} */
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) ri[ks] = li < NK ? sh.R[(4 * ks + lk) * LD + li] : 0.0;
+
+  dx4 kt = dx4{0.0, 0.0, 0.0, 0.0}, S = kt;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) kt = mfma16(nacc[ks], ri[ks], kt);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) S = mfma16(ri[ks], kt[ks], S);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { /* S symmetric: element (4 i + lk, li) stored as its transpose */
+    const int c = 4 * i + lk;
+    if (DIAG ? (c == li && li < n) : (c < n && li < n)) Sout[oj * nn + li + (int64_t)c * n] = S[i];
+  }
+  if (Xcur) { /* X[j-1] = Cov(u_{j-1}, u_j) = -U_1^T, X[j] = Cov(u_j, u_{j+1}) = -U_2 */
+    dx4 u1 = dx4{0.0, 0.0, 0.0, 0.0}, u2 = u1;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u1 = mfma16(ri[ks], sh.W[0][(4 * ks + lk) * LD + li], u1);
+      u2 = mfma16(sh.W[1][(4 * ks + lk) * LD + li], ri[ks], u2);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = 4 * i + lk;
+      if (c < n && li < n) {
+        if (has_m) Xcur[(sj - 1) * nn + li + (int64_t)c * n] = -u1[i];
+        if (has_p) Xcur[sj * nn + li + (int64_t)c * n] = -u2[i];
       }
     }
   }
@@ -932,13 +1179,11 @@ __global__ void __launch_bounds__((QRGeom<NB, NB + 1, 3>::NT))
                    double* __restrict__ C, double* __restrict__ o) {
   using G = QRGeom<NB, NB + 1, 3>;
   constexpr int SL = G::SL;
-  constexpr int NT = G::NT;
   __shared__ Refl<NB, SL, double> refl;
   const int tid = threadIdx.x, sub = tid & (SL - 1), c = tid / SL;
   const int64_t s = blockIdx.x;
   const int64_t nn = (int64_t)n * n;
   const int hi = mr > NB ? mr - NB : 0; /* rows in block 1 */
-  refl_clear<NB, SL, NT, double>(refl, tid);
   Col<NB, SL, double> col;
   const double* src = c < n ? wC + s * (int64_t)mr * n + (int64_t)c * mr : wo + s * mr;
   if (c <= n) {
@@ -1012,14 +1257,12 @@ template <int NB>
 struct FilterShared {
   double R[NB * NB];
   double y[NB];
-  double rinv[NB];
 };
 
 template <int NB>
 __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1>::NT))
     k_filter_step(uk_filter_t st, uk_filter_in_t in, int n, int first) {
   constexpr int SL = QRGeom<NB, 2 * NB + 1, 1>::SL;
-  constexpr int NT = QRGeom<NB, 2 * NB + 1, 1>::NT;
   __shared__ Refl<NB, SL, double> refl;
   __shared__ FilterShared<NB> fs;
   const int tid = threadIdx.x, sub = tid & (SL - 1), c = tid / SL;
@@ -1030,43 +1273,28 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1>::NT))
   const int bc = isB ? c - n : 0;
   const double* kw = in.K + f * n;
   const int zprev = first ? 0 : st.z[f];
-  refl_clear<NB, SL, NT, double>(refl, tid);
-  Col<NB, SL, double> col;
-  col.zero_block(0);
-  col.zero_block(1);
+  const int mi = in.m_i ? in.m_i[f] : mr;
+  const int m = mi < 0 ? 0 : (mi > mr ? mr : mi); /* device-resident counts are not checked on the host */
+  const double* const any = st.y + f * n; /* readable, for blocks that are zero */
+  /* Every load of the step is issued here, without branches: the sources are
+   * chosen by address, and the observation block, which the second QR takes,
+   * waits in registers through the first. */
+  Col<NB, SL, double> col, obs;
+  obs.zero_block(0);
+  obs.load_block(1, isB ? (in.pre ? in.wC + f * nn : in.G + f * mr * n) + (int64_t)bc * mr
+                        : (isY ? (in.pre ? in.wo + f * n : in.o + f * mr) : any),
+                 isB || isY ? m : 0, sub);
+  if (!in.pre) obs.scale_block(1, in.C + f * mr, m, sub, 1.0);
   if (!first) {
-    if (isP) {
-      col.load_block(0, st.R + f * nn + (int64_t)c * n, n, sub);
-      if (in.pre) {
-        col.load_block(1, in.wB + f * nn + (int64_t)c * n, n, sub); /* -V F */
-      } else {
-        col.load_block(1, in.F + (in.F_shared ? 0 : f * nn) + (int64_t)c * n, n, sub);
-        col.scale_block(1, kw, n, sub, -1.0);
-      }
-    }
-    if (isB) {
-      if (in.pre) {
-        col.load_block(1, in.wD + f * nn + (int64_t)bc * n, n, sub); /* V H */
-      } else if (in.H) {
-        col.load_block(1, in.H + f * nn + (int64_t)bc * n, n, sub);
-        col.scale_block(1, kw, n, sub, 1.0);
-      } else {
-#pragma unroll
-        for (int l = 0; l < NB / SL; ++l) {
-          const int r = SL * l + sub;
-          col.a[NB / SL + l] = (r == bc) ? kw[r] : 0.0;
-        }
-      }
-    }
-    if (isY) {
-      col.load_block(0, st.y + f * n, n, sub);
-      if (in.pre) {
-        col.load_block(1, in.wc + f * n, n, sub); /* V c */
-      } else if (in.c) {
-        col.load_block(1, in.c + f * n, n, sub);
-        col.scale_block(1, kw, n, sub, 1.0);
-      }
-    }
+    const double* p1 = any;
+    if (isP) p1 = in.pre ? in.wB + f * nn + (int64_t)c * n : in.F + (in.F_shared ? 0 : f * nn) + (int64_t)c * n;
+    if (isB) p1 = in.pre ? in.wD + f * nn + (int64_t)bc * n : (in.H ? in.H + f * nn + (int64_t)bc * n : kw);
+    if (isY) p1 = in.pre ? in.wc + f * n : (in.c ? in.c + f * n : any);
+    const bool diag = isB && !in.pre && !in.H; /* V H = diag(k): entry bc of k itself */
+    col.load_block(0, isP ? st.R + f * nn + (int64_t)c * n : any, isP || isY ? n : 0, sub);
+    col.load_block(1, p1, isP || isB || (isY && (in.pre || in.c)) ? n : 0, sub);
+    col.keep_row(1, diag, bc, sub);
+    if (!in.pre) col.scale_block(1, kw, diag ? 0 : n, sub, isP ? -1.0 : 1.0); /* -V F, V H, V c */
     house_qr<NB, SL, double>(col, refl, c, sub, 0, n, isP || isB || isY);
     if (st.hist) { /* the previous step's final rows: Rdiag, Rsupdiag, y (c/kalman_ultimate.c:140-260) */
       const int64_t hs = st.hslot * st.nf + f;
@@ -1074,26 +1302,12 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1>::NT))
       if (isB) col.store_block(0, st.hRs + hs * nn + (int64_t)bc * n, n, sub);
       if (isY) col.store_block(0, st.hy + hs * n, n, sub);
     }
-    if (isB || isY) col.move_1_to_0();
+    col.move_1_to_0();
+  } else {
+    col.zero_block(0);
   }
-  const int mi = in.m_i ? in.m_i[f] : mr;
-  const int m = mi < 0 ? 0 : (mi > mr ? mr : mi); /* device-resident counts are not checked on the host */
-  if (m > 0) {
-    if (in.pre) {
-      if (isB) col.load_block(1, in.wC + f * nn + (int64_t)bc * mr, m, sub); /* W G, ld mr in an n*n slot */
-      if (isY) col.load_block(1, in.wo + f * n, m, sub);                      /* W o */
-    } else {
-      const double* cw = in.C + f * mr;
-      if (isB) {
-        col.load_block(1, in.G + f * mr * n + (int64_t)bc * mr, m, sub);
-        col.scale_block(1, cw, m, sub, 1.0);
-      }
-      if (isY) {
-        col.load_block(1, in.o + f * mr, m, sub);
-        col.scale_block(1, cw, m, sub, 1.0);
-      }
-    }
-  }
+#pragma unroll
+  for (int l = NB / SL; l < 2 * (NB / SL); ++l) col.a[l] = obs.a[l];
   house_qr<NB, SL, double>(col, refl, c, sub, n, n, isB || isY);
   if (isB) {
     col.store_triu(st.R + f * nn + (int64_t)bc * n, n, bc, sub);
@@ -1113,19 +1327,10 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1>::NT))
   }
   const int z = min(n, zprev + m);
   __syncthreads();
-  if (tid < n) fs.rinv[tid] = 1.0 / fs.R[tid + tid * NB];
-  __syncthreads();
   if (tid < 64) {
     double r = tid < n ? fs.y[tid] : 0.0;
-    if (z == n) {
-      for (int q = n - 1; q >= 0; --q) {
-        const double xq = __shfl(r, q) * fs.rinv[q];
-        if (tid == q) r = xq;
-        else if (tid < q) r -= fs.R[tid + q * NB] * xq;
-      }
-    } else {
-      r = __builtin_nan("");
-    }
+    if (z == n) r = wave_back_solve<NB>(r, fs.R, NB, tid < n ? 1.0 / fs.R[tid + tid * NB] : 0.0, n, tid);
+    else r = __builtin_nan("");
     if (tid < n) st.x[f * n + tid] = r;
   }
   if (tid == 0) st.z[f] = z;
@@ -1381,40 +1586,48 @@ extern "C" int ukhip_qr_launch_set(int fp32, int phase, int n, int columns_per_g
 }
 
 namespace {
-template <int NB, class T>
-void phase_launch(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac, T* fix,
+/* One phase: a wave per step pair up to n = 32, the register kernels of
+ * oddeven_qr.h in the variant the launch table holds above. */
+template <class T>
+bool phase_launch(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac, T* fix,
                   int n, hipStream_t st, int phase) {
-  if constexpr (NB >= 24) {
-    const QrLaunch q = g_qr[sizeof(T) == 8 ? 0 : 1][phase - 1][qr_bucket_index(NB)];
-    const ukqr::Launch v{q.cpl, q.wg};
-    if constexpr (NB == 24) ukqr::phase_launch_b24(lv, in, out, fac, fix, n, st, phase, v);
-    else if constexpr (NB == 32) ukqr::phase_launch_b32(lv, in, out, fac, fix, n, st, phase, v);
-    else if constexpr (NB == 48) ukqr::phase_launch_b48(lv, in, out, fac, fix, n, st, phase, v);
-    else ukqr::phase_launch_b64(lv, in, out, fac, fix, n, st, phase, v);
-  } else {
-    phase_launch_impl<NB, T>(lv, in, out, fac, fix, n, st, phase, ukqr::Launch{1, 0});
+  const int nb = uk_bucket(n);
+  if (nb == 32) {
+    if (in.mr > n) return false;
+    switch ((n + 3) / 4) {
+      case 5: ukqr::mid_phase_5(lv, in, out, fac, fix, n, st, phase); break;
+      case 6: ukqr::mid_phase_6(lv, in, out, fac, fix, n, st, phase); break;
+      case 7: ukqr::mid_phase_7(lv, in, out, fac, fix, n, st, phase); break;
+      default: ukqr::mid_phase_8(lv, in, out, fac, fix, n, st, phase); break;
+    }
+    return true;
   }
+  const int nbq = uk_bucket(n > in.mr ? n : in.mr);
+  if (nbq != 48 && nbq != 64) return false;
+  const QrLaunch q = g_qr[sizeof(T) == 8 ? 0 : 1][phase - 1][qr_bucket_index(nbq)];
+  const ukqr::Launch v{q.cpl, q.wg};
+  if (nbq == 48) ukqr::phase_launch_b48(lv, in, out, fac, fix, n, st, phase, v);
+  else ukqr::phase_launch_b64(lv, in, out, fac, fix, n, st, phase, v);
+  return true;
 }
 
 template <class T>
 hipError_t launch_eliminate(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac,
                             T* fix, int n, hipStream_t st, hipEvent_t* ev) {
-  const int nb = uk_bucket_qr(n > in.mr ? n : in.mr);
   auto mark = [&](int i) {
     if (ev) (void)hipEventRecord(ev[i], st);
   };
-#define L_(NBV)                                                   \
-  mark(0);                                                        \
-  for (int ph = 1; ph <= 3; ++ph) {                               \
-    phase_launch<NBV, T>(lv, in, out, fac, fix, n, st, ph);       \
-    mark(ph);                                                     \
+  mark(0);
+  if (n <= 16) { /* one launch does the three phases: all of the time is counted as phase 1's */
+    if (in.mr > n) return hipErrorInvalidValue;
+    ukqr::level_small(lv, in, out, fac, n, st);
+    for (int ph = 1; ph <= 3; ++ph) mark(ph);
+    return hipGetLastError();
   }
-  switch (nb) {
-    UK_DISPATCH(8, L_) UK_DISPATCH(16, L_) UK_DISPATCH(24, L_) UK_DISPATCH(32, L_) UK_DISPATCH(48, L_)
-    UK_DISPATCH(64, L_)
-    default: return hipErrorInvalidValue;
+  for (int ph = 1; ph <= 3; ++ph) {
+    if (!phase_launch<T>(lv, in, out, fac, fix, n, st, ph)) return hipErrorInvalidValue;
+    mark(ph);
   }
-#undef L_
   return hipGetLastError();
 }
 }  // namespace
@@ -1455,9 +1668,11 @@ extern "C" hipError_t uk_launch_backsub(const uk_level_t* lv, const uk_factors_t
                                         const double* Xup, const double* XTup, double* Xcur, double* XTcur, int n,
                                         int cov, hipStream_t st) {
   const int nb = uk_bucket(n);
-  if (!cov && nb >= 32) {
+  if (!cov) {
 #define E_(NBV) k_estimate<NBV><<<dim3((unsigned)lv->evens), dim3(64), 0, st>>>(*lv, *fac, xout, n)
     switch (nb) {
+      case 8: E_(8); break;
+      case 16: E_(16); break;
       case 32: E_(32); break;
       case 48: E_(48); break;
       case 64: E_(64); break;
@@ -1466,7 +1681,21 @@ extern "C" hipError_t uk_launch_backsub(const uk_level_t* lv, const uk_factors_t
 #undef E_
     return hipGetLastError();
   }
-  if (cov && nb >= 32 && uk_backsub_mfma_enabled()) {
+  if (nb <= 16) { /* X alone is kept between the levels, XT is not touched */
+    const dim3 g((unsigned)((lv->evens + 3) / 4)), b(256);
+#define B_(KSV)                                                                                          \
+  if (cov == 2) k_backsub_small<KSV, true><<<g, b, 0, st>>>(*lv, *fac, xout, Sout, Xup, Xcur, n);         \
+  else k_backsub_small<KSV, false><<<g, b, 0, st>>>(*lv, *fac, xout, Sout, Xup, Xcur, n)
+    switch ((n + 3) / 4) {
+      case 1: B_(1); break;
+      case 2: B_(2); break;
+      case 3: B_(3); break;
+      default: B_(4); break;
+    }
+#undef B_
+    return hipGetLastError();
+  }
+  if (uk_backsub_mfma_enabled()) {
 #define M_(NBV)                                                                                                  \
   if (cov == 2)                                                                                                  \
     k_backsub_mfma<NBV, true><<<dim3((unsigned)lv->evens), dim3(NBV * 8), 0, st>>>(*lv, *fac, xout, Sout, Xup,    \
@@ -1487,7 +1716,7 @@ extern "C" hipError_t uk_launch_backsub(const uk_level_t* lv, const uk_factors_t
   k_backsub<NBV><<<dim3((unsigned)lv->evens), dim3(((2 * NBV + 63) / 64) * 64), 0, st>>>(*lv, *fac, xout, Sout, Xup, \
                                                                                        XTup, Xcur, XTcur, n, cov)
   switch (nb) {
-    UK_DISPATCH(8, L_) UK_DISPATCH(16, L_) UK_DISPATCH(32, L_) UK_DISPATCH(48, L_) UK_DISPATCH(64, L_)
+    UK_DISPATCH(32, L_) UK_DISPATCH(48, L_) UK_DISPATCH(64, L_)
     default: return hipErrorInvalidValue;
   }
 #undef L_

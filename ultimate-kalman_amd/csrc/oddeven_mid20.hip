@@ -1,0 +1,7 @@
+/*
+ * oddeven_mid20.hip -- elimination phases for n = 17 .. 20 (see
+ * oddeven_mid.h; a translation unit of its own so that the kernels compile in parallel).
+ */
+#include "oddeven_mid.h"
+
+UKMID_DEFINE(5)

@@ -48,11 +48,27 @@ struct Launch {
                            const FactorsT<double>& fac, double* fix, int n, hipStream_t st, int phase, Launch v);    \
   void phase_launch_b##NBV(const uk_level_t* lv, const ChainT<float>& in, const ChainT<float>& out,                   \
                            const FactorsT<float>& fac, float* fix, int n, hipStream_t st, int phase, Launch v);
-UKQR_DECLARE(24)
-UKQR_DECLARE(32)
 UKQR_DECLARE(48)
 UKQR_DECLARE(64)
 #undef UKQR_DECLARE
+/* Phase `phase` of one level for n = 4 NK - 3 .. 4 NK, defined in
+ * oddeven_mid<4 NK>.hip; observation blocks of at most n rows. */
+#define UKQR_DECLARE(NKV)                                                                                            \
+  void mid_phase_##NKV(const uk_level_t* lv, const ChainT<double>& in, const ChainT<double>& out,                     \
+                       const FactorsT<double>& fac, double* fix, int n, hipStream_t st, int phase);                   \
+  void mid_phase_##NKV(const uk_level_t* lv, const ChainT<float>& in, const ChainT<float>& out,                       \
+                       const FactorsT<float>& fac, float* fix, int n, hipStream_t st, int phase);
+UKQR_DECLARE(5)
+UKQR_DECLARE(6)
+UKQR_DECLARE(7)
+UKQR_DECLARE(8)
+#undef UKQR_DECLARE
+/* All three phases of one level for n <= 16, one launch (oddeven_small.hip);
+ * observation blocks of at most n rows. */
+void level_small(const uk_level_t* lv, const ChainT<double>& in, const ChainT<double>& out,
+                 const FactorsT<double>& fac, int n, hipStream_t st);
+void level_small(const uk_level_t* lv, const ChainT<float>& in, const ChainT<float>& out, const FactorsT<float>& fac,
+                 int n, hipStream_t st);
 }  // namespace ukqr
 
 namespace {
@@ -129,7 +145,10 @@ struct Col {
 #pragma unroll
     for (int l = 0; l < H; ++l) a[blk * H + l] = T(0);
   }
-  /* block blk <- rows [0, rows) of a column at src (unit stride), zero elsewhere */
+  /* block blk <- rows [0, rows) of a column at src (unit stride), zero
+   * elsewhere. Callers choose src by address and load every role of a column
+   * with one call: a register written again (with zeros, say) waits for the
+   * load it had under way. */
   __device__ __forceinline__ void load_block(int blk, const T* __restrict__ src, int rows, int sub) {
 #pragma unroll
     for (int l = 0; l < H; ++l) {
@@ -144,25 +163,37 @@ struct Col {
       if (r < rows) dst[r] = a[blk * H + l];
     }
   }
-  /* block blk <- column col of B = -diag(k) F (n x n, F column-major), the
-   * whitened evolution block formed as the whitening pass forms it */
-  __device__ __forceinline__ void load_bsynth(int blk, const double* __restrict__ k, const double* __restrict__ F,
-                                              int col, int n, int sub) {
+  /* where mine: block blk <- src[r] scaled by sign * s[r], each product formed
+   * in double and rounded to T (B = -diag(k) F and C = diag(w) G as the
+   * whitening pass forms them), zero at rows >= rows.
+   * ALL: without branches, at clamped rows (src and s readable at their first
+   * entries), so that all loads are issued before the first product; a product
+   * beside its two loads under a branch of its own waits a memory latency per
+   * row. That takes 2 H doubles more at the load, which FP64 phase 1 has (2.17
+   * -> 2.02 ms a smoothing at n = 48, k = 26,664) and the FP32 kernels and
+   * phase 2 have not: they would keep fewer waves or spill (FP32 phase 1 1.45
+   * -> 1.59 ms, FP64 phase 2 at n = 64 3.77 -> 4.26 ms). */
+  template <bool ALL>
+  __device__ __forceinline__ void load_scaled(int blk, bool mine, const double* __restrict__ s,
+                                              const double* __restrict__ src, int rows, int sub, double sign) {
+    const int last = rows > 0 ? rows - 1 : 0;
 #pragma unroll
     for (int l = 0; l < H; ++l) {
       const int r = SL * l + sub;
-      a[blk * H + l] = (r < n) ? T(-k[r] * F[r + (int64_t)col * n]) : T(0);
+      if (ALL) {
+        const int rr = r < last ? r : last;
+        const T x = T(sign * s[rr] * src[rr]);
+        a[blk * H + l] = mine ? ((r < rows) ? x : T(0)) : T(a[blk * H + l]);
+      } else if (mine) {
+        a[blk * H + l] = (r < rows) ? T(sign * s[r] * src[r]) : T(0);
+      }
     }
   }
-  /* block blk <- column col of C = diag(w) G (G mr x n, ld mr; rows >= m zero),
-   * each entry the FP64 product rounded to T, as the whitening pass stores it */
-  __device__ __forceinline__ void load_csynth(int blk, const double* __restrict__ w, const double* __restrict__ G,
-                                              int col, int mr, int m, int sub) {
+  /* block blk reduced to its entry in row col where mine (a diagonal's column
+   * out of the diagonal, loaded as a vector) */
+  __device__ __forceinline__ void keep_row(int blk, bool mine, int col, int sub) {
 #pragma unroll
-    for (int l = 0; l < H; ++l) {
-      const int r = SL * l + sub;
-      a[blk * H + l] = (r < mr && r < m) ? T(w[r] * G[r + (int64_t)col * mr]) : T(0);
-    }
+    for (int l = 0; l < H; ++l) a[blk * H + l] = (!mine || SL * l + sub == col) ? T(a[blk * H + l]) : T(0);
   }
   /* block blk <- column col of a diagonal matrix given by its diagonal d */
   __device__ __forceinline__ void load_diag(int blk, const T* __restrict__ d, int col, int sub) {
@@ -204,12 +235,15 @@ struct Col {
       st[r] = (r <= col) ? a[l] : T(0);
     }
   }
-  /* rows r < rows of block blk scaled by sign * s[r] */
+  /* rows r < rows of block blk scaled by sign * s[r] (no branch; s readable at
+   * its first entry) */
   __device__ __forceinline__ void scale_block(int blk, const T* __restrict__ s, int rows, int sub, T sign) {
+    const int last = rows > 0 ? rows - 1 : 0;
 #pragma unroll
     for (int l = 0; l < H; ++l) {
       const int r = SL * l + sub;
-      if (r < rows) a[blk * H + l] *= sign * s[r];
+      const T f = sign * s[r < last ? r : last];
+      a[blk * H + l] = (r < rows) ? T(a[blk * H + l] * f) : T(a[blk * H + l]);
     }
   }
 };
@@ -251,7 +285,7 @@ __device__ __forceinline__ void block_zero(T* __restrict__ dst, int64_t nn, int 
 }
 
 /* LDS reflector buffers: [buffer][sub][2H + 4] (the +4 skews the sub-lane
- * arrays onto different banks), then [buffer][2] scalars. A stride that
+ * arrays onto different banks), then the tau of each buffer. A stride that
  * lands on bank 0 or 16 of the 32 four-byte banks (2H + 4 = 16 in bucket 24)
  * would put two sub-lanes' reads on the same banks: it is padded by 4 more. */
 template <int NB, int SL, class T = double>
@@ -260,7 +294,7 @@ struct Refl {
   static constexpr int SUBSTRIDE =
       SUBSTRIDE0 + ((SUBSTRIDE0 * (int)sizeof(T) / 4) % 16 == 0 ? 4 : 0);
   T v[2][SL * SUBSTRIDE];
-  T sc[2][2];
+  T sc[2];
 };
 
 /* Reflector prefetch: with one column per lane group the whole reflector is
@@ -334,6 +368,56 @@ __host__ __device__ constexpr bool qr_need(int l, int H, int SEG, int QF) {
 }
 
 /*
+ * The reflector of a column with alpha in its pivot row and square sum s
+ * below it: u_k = alpha - beta, f1 and f2, with which a column a becomes
+ * a - f1 (v . a) v, v = f2 u; f1 = 0: no reflection.
+ * FP64: H = I - tau u u^T with u = x below the pivot, tau = -1 / (beta u_k) =
+ * 1 / (beta^2 + |alpha| |beta|) = f1, f2 = 1. The square root and the
+ * reciprocal are the hardware's estimates (about 2^-23) refined by Newton
+ * steps to an ulp, the reciprocal's estimate started from the unrefined root:
+ * some 12 dependent operations where the correctly rounded sqrt and division,
+ * with their scaling and fix-up sequences, take over 40. A column whose
+ * squared norm below the pivot is below 1e-280 counts as zero, and so does
+ * one whose squares overflow.
+ * FP32: H = I - tau v v^T with v = u / u_k, f1 = tau = (beta - alpha) / beta in
+ * [1, 2], f2 = 1 / u_k: squaring the column's scale, as above, would leave
+ * FP32's range on nearly dependent columns (m << n). The square root and the two reciprocals are the
+ * hardware's 1-ulp instructions: an ulp in tau or in v's scale is the size of
+ * the FP32 rounding the factorization makes anyway (the FP64 refinement
+ * removes both). Sums of squares below 1e-28 are scaled by 2^64 first,
+ * keeping the square root's argument normal.
+ */
+__device__ __forceinline__ void house_scalars(double alpha, double s, double& ukk, double& f1, double& f2) {
+  const double aa = fabs(alpha);
+  const double s2 = fma(alpha, alpha, s);
+  const double y = __builtin_amdgcn_rsq(s2);
+  double g = s2 * y, h = 0.5 * y;
+  const double v0 = fma(aa, g, s2);
+  double w = __builtin_amdgcn_rcp(v0);
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, s2), h, g); /* sqrt(s2) = |beta| */
+  const double v = fma(aa, g, s2);
+  w = fma(fma(-v, w, 1.0), w, w);
+  w = fma(fma(-v, w, 1.0), w, w);
+  ukk = alpha + copysign(g, alpha);
+  f1 = (s > 1e-280 && v0 < __builtin_inf()) ? w : 0.0;
+  f2 = 1.0;
+}
+__device__ __forceinline__ void house_scalars(float alpha, float s, float& ukk, float& f1, float& f2) {
+  const float t2 = fmaf(alpha, alpha, s);
+  const bool tiny = t2 < 1e-28f;
+  float nrm = __builtin_amdgcn_sqrtf(tiny ? t2 * 0x1p64f : t2);
+  nrm = tiny ? nrm * 0x1p-32f : nrm;
+  const float beta = -copysignf(nrm, alpha);
+  ukk = alpha - beta;
+  f2 = __builtin_amdgcn_rcpf(ukk);
+  const float tau = fmaf(-alpha, __builtin_amdgcn_rcpf(beta), 1.0f); /* (beta - alpha) / beta */
+  f1 = s != 0.0f ? tau : 0.0f;
+}
+
+/*
  * One Householder step for pivot k (target row k of block 0), over the CPL
  * columns a lane group holds; k lies in segment SEG.
  *   piv_slot: which of this group's columns is pivot column k (-1: none);
@@ -347,114 +431,51 @@ __host__ __device__ constexpr bool qr_need(int l, int H, int SEG, int QF) {
  */
 /* V (optional, leading dimension ldv): the pivot lanes also store the
  * published vector as column k of V and its tau as tau[k] (a blocked-WY
- * accumulation of the reflectors; a column that counts as zero stores zeros,
- * and granules skipped as exact zeros are left as they are, zero). */
+ * accumulation of the reflectors; a column that counts as zero stores nothing,
+ * and granules skipped as exact zeros are left as they are: V starts zero). */
 template <int NB, int SL, class T, int SEG, int QF>
 __device__ __forceinline__ void house_publish(const Col<NB, SL, T>& col, Refl<NB, SL, T>& R, int buf, int sub, int k,
                                               T* V = nullptr, T* tauv = nullptr, int ldv = 0) {
-  constexpr int H = NB / SL;
+  constexpr int H = NB / SL, GL = qr_gl(H), G0 = SEG * GL; /* the pivot's granule: locals G0 .. G0 + GL - 1 */
   T* vv = &R.v[buf][sub * Refl<NB, SL, T>::SUBSTRIDE];
+  /* only the pivot's granule is masked: the rows of the later granules are all
+   * below the pivot */
   T s0 = T(0), s1 = T(0), alpha = T(0);
 #pragma unroll
-  for (int l = 0; l < H; ++l) {
+  for (int l = 0; l < 2 * H; ++l) {
     if (!qr_need(l, H, SEG, QF)) continue;
-    const int r = SL * l + sub;
-    const T x = col.a[l];
-    alpha = (r == k) ? x : alpha;
-    const T xm = (r > k) ? x : T(0);
-    if (l & 1) s1 = fma(xm, xm, s1);
-    else s0 = fma(xm, xm, s0);
-  }
-#pragma unroll
-  for (int l = H; l < 2 * H; ++l) {
-    if (!qr_need(l, H, SEG, QF)) continue;
-    if (l & 1) s1 = fma(col.a[l], col.a[l], s1);
-    else s0 = fma(col.a[l], col.a[l], s0);
+    T x = col.a[l];
+    if (l >= G0 && l < G0 + GL) {
+      const int r = SL * l + sub;
+      alpha = (r == k) ? T(x) : T(alpha);
+      x = (r > k) ? T(x) : T(0);
+    }
+    if (l & 1) s1 = fma(x, x, s1);
+    else s0 = fma(x, x, s0);
   }
   const T s = group_sum<SL>(s0 + s1);
   alpha = group_sum<SL>(alpha);
-  if constexpr (sizeof(T) == 8) {
-    /* H = I - tau' u u^T with u = x below the pivot and u_k = alpha - beta:
-     * tau' = -1 / (beta u_k), the unit-pivot form's tau / u_k^2, so the
-     * pivot lanes publish their column as it is (one division, no
-     * scaling). |beta u_k| >= beta^2 = ||x||^2, so a column whose squared
-     * norm is below 1e-280 counts as zero (no reflection). */
-    T taup = T(0), ukk = T(0);
-    if (s > T(1e-280)) {
-      const T beta = -copysign(sqrt(fma(alpha, alpha, s)), alpha);
-      ukk = alpha - beta;
-      taup = T(-1) / (beta * ukk);
-    }
+  /* FP64 publishes u and tau, FP32 v = u / u_k (unit pivot) and its tau */
+  T ukk, f1, f2;
+  house_scalars(alpha, s, ukk, f1, f2);
+  const T tau = f1, piv = sizeof(T) == 4 ? T(1) : T(ukk);
 #pragma unroll
-    for (int l = 0; l < H; ++l) {
-      if (!qr_need(l, H, SEG, QF)) continue;
+  for (int l = 0; l < 2 * H; ++l) {
+    if (!qr_need(l, H, SEG, QF)) continue;
+    T x = sizeof(T) == 4 ? T(col.a[l] * f2) : T(col.a[l]);
+    if (l >= G0 && l < G0 + GL) {
       const int r = SL * l + sub;
-      vv[l] = (r > k) ? col.a[l] : (r == k ? ukk : T(0));
+      x = (r > k) ? T(x) : (r == k ? T(piv) : T(0));
     }
+    vv[l] = x;
+  }
+  if (sub == 0) R.sc[buf] = tau;
+  if (V && tau != T(0)) {
+    T* vc = V + (int64_t)k * ldv;
 #pragma unroll
-    for (int l = H; l < 2 * H; ++l)
-      if (qr_need(l, H, SEG, QF)) vv[l] = col.a[l];
-    if (sub == 0) R.sc[buf][0] = taup;
-    if (V) {
-      const T keep = taup != T(0) ? T(1) : T(0);
-      T* vc = V + (int64_t)k * ldv;
-#pragma unroll
-      for (int l = 0; l < H; ++l) {
-        if (!qr_need(l, H, SEG, QF)) continue;
-        const int r = SL * l + sub;
-        vc[r] = keep * ((r > k) ? col.a[l] : (r == k ? ukk : T(0)));
-      }
-#pragma unroll
-      for (int l = H; l < 2 * H; ++l)
-        if (qr_need(l, H, SEG, QF)) vc[NB + SL * (l - H) + sub] = keep * col.a[l];
-      if (sub == 0) tauv[k] = taup;
-    }
-  } else {
-    /* single precision: the unit-pivot form v = x / (alpha - beta), v_k = 1,
-     * tau = (beta - alpha) / beta in [1, 2]; squaring the column's scale, as
-     * the form above does, would leave FP32's range on nearly dependent
-     * columns (m << n) */
-    /* The square root and the two reciprocals are the hardware's 1-ulp
-     * instructions (v_sqrt_f32, v_rcp_f32) instead of the correctly rounded
-     * sequences: they sit on the step's critical path, and an ulp in tau or
-     * in v's scale is the size of the FP32 rounding the factorization makes
-     * anyway (the FP64 refinement removes both). Sums of squares below
-     * 1e-28 are scaled by 2^64 first, keeping the square root's argument
-     * normal. */
-    T tau = T(0), scale = T(0);
-    if (s != T(0)) {
-      const T t2 = fma(alpha, alpha, s);
-      const bool tiny = t2 < T(1e-28);
-      T nrm = __builtin_amdgcn_sqrtf(tiny ? t2 * T(0x1p64) : t2);
-      nrm = tiny ? nrm * T(0x1p-32) : nrm;
-      const T beta = -copysign(nrm, alpha);
-      tau = fma(-alpha, __builtin_amdgcn_rcpf(beta), T(1)); /* (beta - alpha) / beta */
-      scale = __builtin_amdgcn_rcpf(alpha - beta);
-    }
-#pragma unroll
-    for (int l = 0; l < H; ++l) {
-      if (!qr_need(l, H, SEG, QF)) continue;
-      const int r = SL * l + sub;
-      vv[l] = (r > k) ? col.a[l] * scale : (r == k ? T(1) : T(0));
-    }
-#pragma unroll
-    for (int l = H; l < 2 * H; ++l)
-      if (qr_need(l, H, SEG, QF)) vv[l] = col.a[l] * scale;
-    if (sub == 0) R.sc[buf][0] = tau;
-    if (V) {
-      const T keep = tau != T(0) ? T(1) : T(0);
-      T* vc = V + (int64_t)k * ldv;
-#pragma unroll
-      for (int l = 0; l < H; ++l) {
-        if (!qr_need(l, H, SEG, QF)) continue;
-        const int r = SL * l + sub;
-        vc[r] = keep * ((r > k) ? col.a[l] * scale : (r == k ? T(1) : T(0)));
-      }
-#pragma unroll
-      for (int l = H; l < 2 * H; ++l)
-        if (qr_need(l, H, SEG, QF)) vc[NB + SL * (l - H) + sub] = keep * col.a[l] * scale;
-      if (sub == 0) tauv[k] = tau;
-    }
+    for (int l = 0; l < 2 * H; ++l)
+      if (qr_need(l, H, SEG, QF)) vc[(l < H ? 0 : NB) + SL * (l % H) + sub] = vv[l];
+    if (sub == 0) tauv[k] = tau;
   }
 }
 
@@ -466,7 +487,7 @@ __device__ __forceinline__ void house_update(Col<NB, SL, T> (&cols)[CPL], const 
                                              unsigned upd) {
   constexpr int H = NB / SL;
   {
-    const T tau = R.sc[buf][0];
+    const T tau = R.sc[buf];
     if (tau != T(0)) {
       /* v is read from LDS in chunks of CH locals issued back to back. With
        * CPL > 1 every column of the group runs the same branch-free code (a
@@ -671,12 +692,6 @@ __device__ __forceinline__ Col<NB, SL, T> swap_col0(T r00, int sub) {
   return c;
 }
 
-template <int NB, int SL, int NT, class T>
-__device__ __forceinline__ void refl_clear(Refl<NB, SL, T>& R, int tid) {
-  for (int i = tid; i < (int)(sizeof(R) / sizeof(T)); i += NT) reinterpret_cast<T*>(&R)[i] = T(0);
-  __syncthreads();
-}
-
 /*
  * Elimination of one level, three launches (the reference's three phases):
  *
@@ -711,42 +726,46 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1, WG, CPL, true>::NT)
   const int tid = threadIdx.x, sub = tid & (SL - 1), grp = tid / SL;
   const int64_t e = blockIdx.x;
   const int p = (int)find_problem(lv.even_start, lv.nprob, e);
-  const int64_t u = e - lv.even_start[p];
+  const int64_t u0 = lv.even_start[p], L = lv.L[p], s0 = lv.step_start[p], t0 = lv.next_start[p];
+  const int64_t u = e - u0;
   const int64_t j = 2 * u;
-  const int64_t L = lv.L[p];
-  const int64_t s0 = lv.step_start[p];
-  const int64_t t = lv.next_start[p] + u;
+  const int64_t t = t0 + u;
   const int mr = in.mr;
   const int64_t nn = (int64_t)n * n;
   const bool lone = j + 1 == L;
-  refl_clear<NB, SL, NT, T>(refl, tid);
 
   const int64_t sj = s0 + j, sp = s0 + j + 1;
   using St = Stage<NB, CPL, NT, T>;
   __shared__ T sbuf[sizeof(T) == 4 ? St::SIZE : 1]; /* FP32 kernels stage their stores */
   const St stg{sbuf};
-  /* column c of the workgroup's matrix: loads it, returns whether it exists */
+  /* column c of the workgroup's matrix: loads it, returns whether it exists.
+   * Its two sources are chosen by address, so that all columns and roles
+   * share one run of loads; what is formed on load at level 0 follows in
+   * `synth`. */
+  const T* const any = in.o + sj * n; /* readable, for blocks that are zero */
   auto load = [&](Col<NB, SL, T>& col, int c) -> bool {
-    const bool isP = c < n, isQ = !lone && c >= n && c < 2 * n, isR1 = c == 2 * n;
-    const int qc = isP ? c : (isQ ? c - n : 0);
-    if (isP) {
-      if (lone) col.zero_block(0);
-      else if (in.b_synth) col.load_bsynth(0, in.wk + sp * n, in.wF + (in.wFidx ? in.wFidx[sp] * nn : 0), qc, n, sub);
-      else col.load_block(0, in.B + sp * nn + (int64_t)qc * n, n, sub);
-      if (in.c_synth) col.load_csynth(1, in.rC + sj * mr, in.rG + sj * (int64_t)mr * n, qc, mr, in.rm[sj], sub);
-      else col.load_block(1, in.C + sj * nn + (int64_t)qc * mr, mr, sub);
-    }
-    if (isQ) {
-      if (in.d_diag) col.load_diag(0, in.D + sp * nn, qc, sub); /* stored as its diagonal */
-      else col.load_block(0, in.D + sp * nn + (int64_t)qc * n, n, sub);
-      col.zero_block(1);
-    }
-    if (isR1) {
-      if (lone) col.zero_block(0);
-      else col.load_block(0, in.c + sp * n, n, sub);
-      col.load_block(1, in.o + sj * n, mr, sub);
-    }
+    const bool isP = c >= 0 && c < n, isQ = !lone && c >= n && c < 2 * n, isR1 = c == 2 * n;
+    const int64_t qc = isP ? c : (isQ ? c - n : 0);
+    const bool top = !lone && (isQ || isR1 || (isP && !in.b_synth));
+    const bool bot = isR1 || (isP && !in.c_synth);
+    const T* p0 = isP ? in.B + sp * nn + qc * n : (isQ ? in.D + sp * nn + (in.d_diag ? 0 : qc * n) : in.c + sp * n);
+    const T* p1 = isP ? in.C + sj * nn + qc * mr : any;
+    col.load_block(0, top ? p0 : any, top ? n : 0, sub);
+    col.load_block(1, bot ? p1 : any, bot ? mr : 0, sub);
+    if (in.d_diag) col.keep_row(0, isQ, (int)qc, sub); /* stored as its diagonal */
     return isP || isQ || isR1;
+  };
+  /* level 0: B_{j+1} and (FP32) C_j from the raw inputs */
+  const double* const bk = in.b_synth && !lone ? in.wk + sp * n : in.wk;
+  const double* const bF = in.b_synth && !lone ? in.wF + (in.wFidx ? in.wFidx[sp] * nn : 0) : in.wF;
+  const int cm = in.c_synth ? min(mr, in.rm[sj]) : 0;
+  auto synth = [&](Col<NB, SL, T>& col, int c) {
+    const bool isP = c >= 0 && c < n;
+    const int64_t qc = isP ? c : 0;
+    col.template load_scaled<sizeof(T) == 8>(0, isP && in.b_synth && !lone, bk, bF + qc * n, n, sub, -1.0);
+    if (sizeof(T) == 4)
+      col.template load_scaled<false>(1, isP && in.c_synth, in.c_synth ? in.rC + sj * mr : bk,
+                      in.c_synth ? in.rG + sj * (int64_t)mr * n + qc * mr : bF, cm, sub, 1.0);
   };
   auto store = [&](const Col<NB, SL, T>& col, int c) {
     const bool isP = c < n, isQ = !lone && c >= n && c < 2 * n, isR1 = c == 2 * n;
@@ -772,12 +791,17 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1, WG, CPL, true>::NT)
   Col<NB, SL, T> extra;
   unsigned upd = 0;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    const int c = grp * CPL + q;
-    if (!(SW && c == 2 * n) && load(cols[q], c)) upd |= 1u << q;
-    else if (CPL > 1) cols[q].zero_block(0), cols[q].zero_block(1); /* computed on as zeros, never stored */
+  for (int q = 0; q < CPL; ++q) { /* a column that does not exist is zero: computed on, never stored */
+    const int c = (SW && grp * CPL + q == 2 * n) ? -1 : grp * CPL + q;
+    if (load(cols[q], c)) upd |= 1u << q;
   }
-  if (SW && grp == 0) load(extra, 2 * n);
+  if (SW) load(extra, grp == 0 ? 2 * n : -1);
+  if (LV != 2 && (in.b_synth || in.c_synth)) { /* upper-triangular C blocks come with B stored */
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) {
+      synth(cols[q], (SW && grp * CPL + q == 2 * n) ? -1 : grp * CPL + q);
+    }
+  }
   /* LV 1: the stacked rows C_j, o_j fill at most qr_half_rows rows; LV 2: C_j is
    * upper triangular (the pivot columns' block 1) */
   constexpr int QF = QF_DONE | (LV == 1 ? QF_HALF1 : 0) | (LV == 2 ? QF_TRI1 : 0);
@@ -837,54 +861,56 @@ __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1, WG, CPL, true>::NT)
   }
 }
 
-template <int NB, class T, int WG = 0, int CPL = 1, bool DIAG = false>
+/* DV: the level's D and B blocks: 0 both stored in full (the levels above 0, and
+ * level 0 after a dense whitening), 1 D diagonal and B formed on load (level
+ * 0, H = I, every K and C given as 'w'), 2 D in full and B formed on load
+ * (level 0 with H given). The raw loads' registers are only in the instances
+ * that form B. */
+template <int NB, class T, int WG = 0, int CPL = 1, int DV = 0>
 __global__ void __launch_bounds__((QRGeom<NB, 3 * NB + 1, 2, WG, CPL, true>::NT),
                                   (QRGeom<NB, 3 * NB + 1, 2, WG, CPL, true>::MINW))
     k_phase2(uk_level_t lv, ChainT<T> in, ChainT<T> out, FactorsT<T> fac, T* __restrict__ fix, int n) {
   using G = QRGeom<NB, 3 * NB + 1, 2, WG, CPL, true>;
   constexpr int SL = G::SL;
   constexpr int NT = G::NT;
+  constexpr bool DIAG = DV == 1, BS = DV != 0;
   constexpr bool SW = G::SWAP; /* the last column of Bl swapped into column 0's registers */
   __shared__ Refl<NB, SL, T> refl;
   const int tid = threadIdx.x, sub = tid & (SL - 1), grp = tid / SL;
   const int64_t e = blockIdx.x;
   const int p = (int)find_problem(lv.even_start, lv.nprob, e);
-  const int64_t u = e - lv.even_start[p];
+  const int64_t u0 = lv.even_start[p], L = lv.L[p], s0 = lv.step_start[p], t0 = lv.next_start[p];
+  const int64_t u = e - u0;
   const int64_t j = 2 * u;
   if (j == 0) return; /* the chain's first step has no [D; R~] (uniform per block) */
-  const int64_t L = lv.L[p];
-  const int64_t t = lv.next_start[p] + u;
+  const int64_t t = t0 + u;
   const int64_t nn = (int64_t)n * n;
   const bool lone = j + 1 == L;
-  refl_clear<NB, SL, NT, T>(refl, tid);
 
-  const int64_t sj = lv.step_start[p] + j;
+  const int64_t sj = s0 + j;
   T* fz = fix + (int64_t)p * (nn + n);
   using St = Stage<NB, CPL, NT, T>;
   __shared__ T sbuf[sizeof(T) == 4 ? St::SIZE : 1]; /* FP32 kernels stage their stores */
   const St stg{sbuf};
+  const T* const any = in.c + sj * n; /* readable, for blocks that are zero */
   auto load = [&](Col<NB, SL, T>& col, int c) -> bool {
-    const bool isP = c < n, isQ = c >= n && c < 2 * n, isR1 = c == 2 * n, isBl = c > 2 * n && c <= 3 * n;
-    const int qc = isP ? c : (isQ ? c - n : (isBl ? c - 2 * n - 1 : 0));
-    if (isP) {
-      if (DIAG) col.load_diag(0, in.D + sj * nn, qc, sub); /* stored as its diagonal */
-      else col.load_block(0, in.D + sj * nn + (int64_t)qc * n, n, sub);
-      col.load_block(1, fac.R + e * nn + (int64_t)qc * n, n, sub); /* R~_j */
-    }
-    if (isQ) {
-      col.zero_block(0);
-      col.load_block(1, fac.Y + e * nn + (int64_t)qc * n, n, sub); /* X_j (zero for a lone step) */
-    }
-    if (isR1) {
-      col.load_block(0, in.c + sj * n, n, sub);
-      col.load_block(1, fac.cf + e * n, n, sub); /* o_j */
-    }
-    if (isBl) {
-      if (in.b_synth) col.load_bsynth(0, in.wk + sj * n, in.wF + (in.wFidx ? in.wFidx[sj] * nn : 0), qc, n, sub);
-      else col.load_block(0, in.B + sj * nn + (int64_t)qc * n, n, sub);
-      col.zero_block(1);
-    }
+    const bool isP = c >= 0 && c < n, isQ = c >= n && c < 2 * n, isR1 = c == 2 * n, isBl = c > 2 * n && c <= 3 * n;
+    const int64_t qc = isP ? c : (isQ ? c - n : (isBl ? c - 2 * n - 1 : 0));
+    const bool top = isP || isR1 || (isBl && !BS), bot = isP || isQ || isR1;
+    const T* p0 = isP ? in.D + sj * nn + (DIAG ? 0 : qc * n) : (isBl ? in.B + sj * nn + qc * n : any);
+    const T* p1 = isR1 ? fac.cf + e * n : (isQ ? fac.Y : fac.R) + e * nn + qc * n; /* o_j, X_j (zero for a lone step), R~_j */
+    col.load_block(0, top ? p0 : any, top ? n : 0, sub);
+    col.load_block(1, bot ? p1 : any, bot ? n : 0, sub);
+    if (DIAG) col.keep_row(0, isP, (int)qc, sub); /* stored as its diagonal */
     return isP || isQ || isR1 || isBl;
+  };
+  /* level 0: B_j from the raw inputs */
+  const double* const bk = BS ? in.wk + sj * n : nullptr;
+  const double* const bF = BS ? in.wF + (in.wFidx ? in.wFidx[sj] * nn : 0) : nullptr;
+  auto synth = [&](Col<NB, SL, T>& col, int c) {
+    const bool isBl = c > 2 * n && c <= 3 * n;
+    const int64_t qc = isBl ? c - 2 * n - 1 : 0;
+    col.template load_scaled<false>(0, isBl, bk, bF + qc * n, n, sub, -1.0);
   };
   auto store = [&](const Col<NB, SL, T>& col, int c) {
     const bool isP = c < n, isQ = c >= n && c < 2 * n, isR1 = c == 2 * n, isBl = c > 2 * n && c <= 3 * n;
@@ -908,12 +934,18 @@ __global__ void __launch_bounds__((QRGeom<NB, 3 * NB + 1, 2, WG, CPL, true>::NT)
   Col<NB, SL, T> extra;
   unsigned upd = 0;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    const int c = grp * CPL + q;
-    if (!(SW && c == 3 * n) && load(cols[q], c)) upd |= 1u << q;
-    else if (CPL > 1) cols[q].zero_block(0), cols[q].zero_block(1); /* computed on as zeros, never stored */
+  for (int q = 0; q < CPL; ++q) { /* a column that does not exist is zero: computed on, never stored */
+    const int c = (SW && grp * CPL + q == 3 * n) ? -1 : grp * CPL + q;
+    if (load(cols[q], c)) upd |= 1u << q;
   }
-  if (SW && grp == 0) load(extra, 3 * n);
+  if (SW) load(extra, grp == 0 ? 3 * n : -1);
+  if constexpr (BS) {
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) {
+      synth(cols[q], (SW && grp * CPL + q == 3 * n) ? -1 : grp * CPL + q);
+    }
+    if (SW) synth(extra, grp == 0 ? 3 * n : -1);
+  }
   /* block 1 of the pivot columns is R~_j, upper triangular */
   /* DIAG: D_j is diagonal (the chain's d_diag) */
   constexpr int QF = QF_TRI1 | QF_DONE | (DIAG ? QF_DIAG0 : 0);
@@ -1008,45 +1040,52 @@ __global__ void __launch_bounds__((QRGeom<NB, NB + 1, 3, WG, CPL, true>::NT),
   const int tid = threadIdx.x, sub = tid & (SL - 1), grp = tid / SL;
   const int64_t unit = blockIdx.x;
   const int p = (int)find_problem(lv.unit_start, lv.nprob, unit);
-  const int64_t L = lv.L[p];
+  const int64_t u0 = lv.unit_start[p], L = lv.L[p], s0 = lv.step_start[p], t0 = lv.next_start[p];
   if (L == 1) return; /* uniform per block */
-  const int64_t u = unit - lv.unit_start[p];
+  const int64_t u = unit - u0;
   const int64_t j = 2 * u;
-  const int64_t t = lv.next_start[p] + u;
+  const int64_t t = t0 + u;
   const int mr = in.mr;
   const int64_t nn = (int64_t)n * n;
   const bool do_fix = (L & 1) && (u == L / 2 - 1);
-  refl_clear<NB, SL, NT, T>(refl, tid);
 
   /* Q columns numbered from 0 here */
-  const int64_t sp = lv.step_start[p] + j + 1;
+  const int64_t sp = s0 + j + 1;
   using St = Stage<NB, CPL, NT, T>;
   __shared__ T sbuf[sizeof(T) == 4 ? St::SIZE : 1]; /* FP32 kernels stage their stores */
   const St stg{sbuf};
   auto load = [&](Col<NB, SL, T>& col, int c) -> bool {
-    const bool isQ = c < n, isR1 = c == n;
-    const int qc = isQ ? c : 0;
-    if (isQ) {
-      col.load_block(0, out.C + t * nn + (int64_t)qc * mr, mr, sub); /* D~_{j+1} */
-      if (in.c_synth) col.load_csynth(1, in.rC + sp * mr, in.rG + sp * (int64_t)mr * n, qc, mr, in.rm[sp], sub);
-      else col.load_block(1, in.C + sp * nn + (int64_t)qc * mr, mr, sub);
-    }
-    if (isR1) {
-      col.load_block(0, out.o + t * n, mr, sub); /* c~_{j+1} */
-      col.load_block(1, in.o + sp * n, mr, sub);
-    }
+    const bool isQ = c >= 0 && c < n, isR1 = c == n;
+    const int64_t qc = isQ ? c : 0;
+    const bool bot = isR1 || (isQ && !in.c_synth);
+    const T* p0 = isQ ? out.C + t * nn + qc * mr : out.o + t * n; /* D~_{j+1}, c~_{j+1} */
+    const T* p1 = isQ && !in.c_synth ? in.C + sp * nn + qc * mr : in.o + sp * n;
+    col.load_block(0, p0, isQ || isR1 ? mr : 0, sub);
+    col.load_block(1, p1, bot ? mr : 0, sub);
     return isQ || isR1;
+  };
+  /* FP32, level 0: C_{j+1} from the raw inputs */
+  const int cm = in.c_synth ? min(mr, in.rm[sp]) : 0;
+  auto synth = [&](Col<NB, SL, T>& col, int c) {
+    const bool isQ = c >= 0 && c < n;
+    const int64_t qc = isQ ? c : 0;
+    if (sizeof(T) == 4) col.template load_scaled<false>(1, isQ, in.rC + sp * mr, in.rG + sp * (int64_t)mr * n + qc * mr, cm, sub, 1.0);
   };
   Col<NB, SL, T> cols[CPL];
   Col<NB, SL, T> extra;
   unsigned upd = 0;
 #pragma unroll
-  for (int q = 0; q < CPL; ++q) {
-    const int c = grp * CPL + q;
-    if (!(SW && c == n) && load(cols[q], c)) upd |= 1u << q;
-    else if (CPL > 1) cols[q].zero_block(0), cols[q].zero_block(1); /* computed on as zeros, never stored */
+  for (int q = 0; q < CPL; ++q) { /* a column that does not exist is zero: computed on, never stored */
+    const int c = (SW && grp * CPL + q == n) ? -1 : grp * CPL + q;
+    if (load(cols[q], c)) upd |= 1u << q;
   }
-  if (SW && grp == 0) load(extra, n);
+  if (SW) load(extra, grp == 0 ? n : -1);
+  if (sizeof(T) == 4 && LV != 2 && in.c_synth) {
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) {
+      synth(cols[q], (SW && grp * CPL + q == n) ? -1 : grp * CPL + q);
+    }
+  }
   /* LV 1: both blocks (D~_{j+1}, C_{j+1} and the right-hand sides) fill at
    * most qr_half_rows rows; LV 2: C_{j+1} (block 1 of the pivot columns) is upper
    * triangular */
@@ -1215,7 +1254,7 @@ __global__ void __launch_bounds__(WyGeom<NB>::NT, 1)
   T* fz = fix + (int64_t)p * (nn + n);
   for (int i = tid; i < LDV * NB; i += NT) sh.V[i] = T(0);
   for (int i = tid; i < NB; i += NT) sh.tau[i] = T(0);
-  refl_clear<NB, SL, NT, T>(sh.refl, tid);
+  __syncthreads(); /* V and tau zeroed before the panel's groups store into them */
 
   /* ---- 1. panel ---- */
   {
@@ -1377,8 +1416,9 @@ void phases_nb(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, 
     else k_phase1<NB, T, WG, CPL, 0><<<g, b, 0, st>>>(*lv, in, out, fac, n);
   } else if (phase == 2) {
     const dim3 g((unsigned)lv->evens), b(QRGeom<NB, 3 * NB + 1, 2, WG, CPL, true>::NT);
-    if (in.d_diag) k_phase2<NB, T, WG, CPL, true><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
-    else k_phase2<NB, T, WG, CPL, false><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
+    if (in.d_diag && in.b_synth) k_phase2<NB, T, WG, CPL, 1><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
+    else if (in.b_synth) k_phase2<NB, T, WG, CPL, 2><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
+    else k_phase2<NB, T, WG, CPL, 0><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
   } else {
     const dim3 g((unsigned)lv->units), b(QRGeom<NB, NB + 1, 3, WG, CPL, true>::NT);
     if (lvk == 2) k_phase3<NB, T, WG, CPL, 2><<<g, b, 0, st>>>(*lv, in, out, fix, n);

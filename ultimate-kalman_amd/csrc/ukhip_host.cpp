@@ -1040,10 +1040,11 @@ struct SlotTimer {
     for (auto& e : quad) e = make();
     return quad;
   }
-  void phases_done() {
+  /* one: a single launch does the three phases (n <= 16), counted as phase 1 */
+  void phases_done(bool one) {
     if (!first) first = quad[0];
     last = quad[3];
-    for (int p = 0; p < 3; ++p) rec.push_back({UKHIP_OE_PHASE1 + p, quad[p], quad[p + 1], 1});
+    for (int p = 0; p < (one ? 1 : 3); ++p) rec.push_back({UKHIP_OE_PHASE1 + p, quad[p], quad[p + 1], 1});
   }
   /* waits for the stream, adds the slot sums into ms and launches */
   bool collect(double* ms, int32_t* launches) {
@@ -1126,7 +1127,7 @@ static bool run_oddeven_view(uk_oe_view_t* v, int cov, SlotTimer* tm, hipStream_
     if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, v->fix, n, st, tm ? tm->phases() : nullptr),
                 "elimination launch"))
       return false;
-    if (tm) tm->phases_done();
+    if (tm) tm->phases_done(n <= 16);
   }
   for (int l = nl - 1; l >= 0; --l) {
     const uk_factors_t f = fac_at(l);
@@ -1604,7 +1605,7 @@ static bool run_mixed(ukhip_batch* b, int refinements, int fp32_levels, bool cov
       if (!hip_ok(uk_launch_eliminate32(&lv, &in, &out, &f, b->fix32, n, st, tm ? tm->phases() : nullptr),
                   "FP32 elimination launch"))
         return false;
-      if (tm) tm->phases_done();
+      if (tm) tm->phases_done(n <= 16);
       if (l + 1 == lsw && lsw < nl) { /* the next level's chain enters FP64 */
         const size_t ns = (size_t)b->levels[lsw].steps;
         const uk_chain_t& t = top[lsw & 1];
@@ -1627,7 +1628,7 @@ static bool run_mixed(ukhip_batch* b, int refinements, int fp32_levels, bool cov
       if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, b->fix, n, st, tm ? tm->phases() : nullptr),
                   "FP64 elimination launch"))
         return false;
-      if (tm) tm->phases_done();
+      if (tm) tm->phases_done(n <= 16);
     }
   }
   /* x0 from the transformed right-hand sides */
