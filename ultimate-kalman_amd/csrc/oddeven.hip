@@ -1751,14 +1751,19 @@ extern "C" hipError_t uk_launch_filter_smooth(const uk_filter_t* st, int n, int6
   return hipGetLastError();
 }
 
-/* One step of every filter of a batch (k_filter_step). */
+extern "C" hipError_t uk_launch_filter_small(const uk_filter_t* st, const uk_filter_in_t* in, int nf, int n, int first,
+                                             hipStream_t s);
+
+/* One step of every filter of a batch: a wave per filter up to n = 16
+ * (filter_small.hip), else k_filter_step. */
 extern "C" hipError_t uk_launch_filter_step(const uk_filter_t* st, const uk_filter_in_t* in, int nf, int n, int first,
                                             hipStream_t s) {
+  if (n <= 16) return uk_launch_filter_small(st, in, nf, n, first, s);
   const int nb = uk_bucket(n > in->mr ? n : in->mr);
 #define F_(NBV) \
   k_filter_step<NBV><<<dim3((unsigned)nf), dim3(QRGeom<NBV, 2 * NBV + 1, 1>::NT), 0, s>>>(*st, *in, n, first)
   switch (nb) {
-    UK_DISPATCH(8, F_) UK_DISPATCH(16, F_) UK_DISPATCH(32, F_) UK_DISPATCH(48, F_) UK_DISPATCH(64, F_)
+    UK_DISPATCH(32, F_) UK_DISPATCH(48, F_) UK_DISPATCH(64, F_)
     default: return hipErrorInvalidValue;
   }
 #undef F_
