@@ -135,8 +135,8 @@ int ukhip_batch_download_cov(ukhip_batch_t* b, int32_t p, char format, double* o
  * events recorded on the library stream around every launch (group) and
  * summed over the levels; the parts of a multi-dimension batch run one after
  * another. Slots: UKHIP_OE_WEIGH (k_weigh / k_weigh_diag, and k_obs_compress),
- * PHASE1..3 (k_phase1..3; up to n = 16 one launch, k_level_small, does the
- * three phases of a level and is counted as PHASE1), BACKSUB (k_backsub,
+ * PHASE1..3 (k_mid1..3, k_phase1..3; where one launch does the three phases of
+ * a level, k_level_small and k_mid_level, it is counted as PHASE1), BACKSUB (k_backsub,
  * k_backsub_small, k_backsub_mfma, k_estimate),
  * TOTAL (the span from the first launch to the end of the last); for the
  * mixed-precision path also SOLVE (k_solve_est), NORMAL (k_normal, k_gather,

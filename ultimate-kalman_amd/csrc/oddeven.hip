@@ -1587,7 +1587,8 @@ extern "C" int ukhip_qr_launch_set(int fp32, int phase, int n, int columns_per_g
 
 namespace {
 /* One phase: a wave per step pair up to n = 32, the register kernels of
- * oddeven_qr.h in the variant the launch table holds above. */
+ * oddeven_qr.h in the variant the launch table holds above. Phase 0: the whole
+ * level in one launch where there is such a kernel for it (true). */
 template <class T>
 bool phase_launch(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac, T* fix,
                   int n, hipStream_t st, int phase) {
@@ -1595,13 +1596,13 @@ bool phase_launch(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& ou
   if (nb == 32) {
     if (in.mr > n) return false;
     switch ((n + 3) / 4) {
-      case 5: ukqr::mid_phase_5(lv, in, out, fac, fix, n, st, phase); break;
-      case 6: ukqr::mid_phase_6(lv, in, out, fac, fix, n, st, phase); break;
-      case 7: ukqr::mid_phase_7(lv, in, out, fac, fix, n, st, phase); break;
-      default: ukqr::mid_phase_8(lv, in, out, fac, fix, n, st, phase); break;
+      case 5: return ukqr::mid_phase_5(lv, in, out, fac, fix, n, st, phase);
+      case 6: return ukqr::mid_phase_6(lv, in, out, fac, fix, n, st, phase);
+      case 7: return ukqr::mid_phase_7(lv, in, out, fac, fix, n, st, phase);
+      default: return ukqr::mid_phase_8(lv, in, out, fac, fix, n, st, phase);
     }
-    return true;
   }
+  if (phase == 0) return false;
   const int nbq = uk_bucket(n > in.mr ? n : in.mr);
   if (nbq != 48 && nbq != 64) return false;
   const QrLaunch q = g_qr[sizeof(T) == 8 ? 0 : 1][phase - 1][qr_bucket_index(nbq)];
@@ -1613,14 +1614,22 @@ bool phase_launch(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& ou
 
 template <class T>
 hipError_t launch_eliminate(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac,
-                            T* fix, int n, hipStream_t st, hipEvent_t* ev) {
+                            T* fix, int n, hipStream_t st, hipEvent_t* ev, int* one) {
   auto mark = [&](int i) {
     if (ev) (void)hipEventRecord(ev[i], st);
   };
   mark(0);
-  if (n <= 16) { /* one launch does the three phases: all of the time is counted as phase 1's */
+  /* where one launch does the three phases, all of the time is phase 1's */
+  bool whole = false;
+  if (n <= 16) {
     if (in.mr > n) return hipErrorInvalidValue;
     ukqr::level_small(lv, in, out, fac, n, st);
+    whole = true;
+  } else {
+    whole = phase_launch<T>(lv, in, out, fac, fix, n, st, 0);
+  }
+  if (one) *one = whole;
+  if (whole) {
     for (int ph = 1; ph <= 3; ++ph) mark(ph);
     return hipGetLastError();
   }
@@ -1632,28 +1641,30 @@ hipError_t launch_eliminate(const uk_level_t* lv, const ChainT<T>& in, const Cha
 }
 }  // namespace
 
-/* ev (NULL or 4 events) is recorded before phase 1 and after each phase. */
+/* ev (NULL or 4 events) is recorded before phase 1 and after each phase; one
+ * (NULL allowed) receives whether a single launch did the three (ev[1] .. ev[3]
+ * then come after it). */
 extern "C" hipError_t uk_launch_eliminate(const uk_level_t* lv, const uk_chain_t* in, const uk_chain_t* out,
                                           const uk_factors_t* fac, double* fix, int n, hipStream_t st,
-                                          hipEvent_t* ev) {
+                                          hipEvent_t* ev, int* one) {
   const ChainT<double> ci{in->B,      in->D,  in->c,  in->C,     in->o,   in->mr,  in->d_diag, in->c_tri,
                           in->b_synth, in->wk, in->wF, in->wFidx, 0,       nullptr, nullptr,    nullptr};
   const ChainT<double> co{out->B,      out->D,  out->c,  out->C,     out->o,  out->mr, out->d_diag, out->c_tri,
                           out->b_synth, out->wk, out->wF, out->wFidx, 0,       nullptr, nullptr,     nullptr};
   const FactorsT<double> f{fac->R, fac->Bt, fac->Y, fac->cf};
-  return launch_eliminate<double>(lv, ci, co, f, fix, n, st, ev);
+  return launch_eliminate<double>(lv, ci, co, f, fix, n, st, ev, one);
 }
 
 /* The same elimination in single precision (chains, factors and arithmetic). */
 extern "C" hipError_t uk_launch_eliminate32(const uk_level_t* lv, const uk_chain32_t* in, const uk_chain32_t* out,
                                             const uk_factors32_t* fac, float* fix, int n, hipStream_t st,
-                                            hipEvent_t* ev) {
+                                            hipEvent_t* ev, int* one) {
   const ChainT<float> ci{in->B,      in->D,  in->c,  in->C,     in->o,      in->mr,  in->d_diag, in->c_tri,
                          in->b_synth, in->wk, in->wF, in->wFidx, in->c_synth, in->rG, in->rC,     in->rm};
   const ChainT<float> co{out->B,      out->D,  out->c,  out->C,     out->o,      out->mr, out->d_diag, out->c_tri,
                          out->b_synth, out->wk, out->wF, out->wFidx, out->c_synth, out->rG, out->rC,     out->rm};
   const FactorsT<float> f{fac->R, fac->Bt, fac->Y, fac->cf};
-  return launch_eliminate<float>(lv, ci, co, f, fix, n, st, ev);
+  return launch_eliminate<float>(lv, ci, co, f, fix, n, st, ev, one);
 }
 
 /* Back substitution with covariances for n > 16 on the matrix cores (default)

@@ -52,11 +52,12 @@ UKQR_DECLARE(48)
 UKQR_DECLARE(64)
 #undef UKQR_DECLARE
 /* Phase `phase` of one level for n = 4 NK - 3 .. 4 NK, defined in
- * oddeven_mid<4 NK>.hip; observation blocks of at most n rows. */
+ * oddeven_mid<4 NK>.hip; observation blocks of at most n rows. Phase 0: the
+ * whole level in one launch, where that is taken (true), else nothing (false). */
 #define UKQR_DECLARE(NKV)                                                                                            \
-  void mid_phase_##NKV(const uk_level_t* lv, const ChainT<double>& in, const ChainT<double>& out,                     \
+  bool mid_phase_##NKV(const uk_level_t* lv, const ChainT<double>& in, const ChainT<double>& out,                     \
                        const FactorsT<double>& fac, double* fix, int n, hipStream_t st, int phase);                   \
-  void mid_phase_##NKV(const uk_level_t* lv, const ChainT<float>& in, const ChainT<float>& out,                       \
+  bool mid_phase_##NKV(const uk_level_t* lv, const ChainT<float>& in, const ChainT<float>& out,                       \
                        const FactorsT<float>& fac, float* fix, int n, hipStream_t st, int phase);
 UKQR_DECLARE(5)
 UKQR_DECLARE(6)

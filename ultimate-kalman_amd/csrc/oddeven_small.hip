@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(256)
         for (int g = 0; g < NK; ++g) {
           e3[g] = g3[0][g];
           e3[NK + g] = z[NK + g][lane];
-          g3[0][g] = li == 0 ? (g == 0 && lk == 0 ? T(kept3.r00) : T(0)) : T(g3[0][g]);
+          g3[0][g] = li == 0 ? (g == 0 && lk == 0 ? T(kept3.r00) : T(0)) : (4 * g + lk <= li ? T(g3[0][g]) : T(0));
           g3[0][NK + g] = z[g][lane];
         }
         sm_qr<NK, 1, 0, T>(g3, e3, kept3, n, li, lk);
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256)
     if (f2) {
 #pragma unroll
       for (int g = 0; g < NK; ++g) {
-        const T rt = li == 0 ? (g == 0 && lk == 0 ? T(kept.r00) : T(0)) : T(w[0][g]);
+        const T rt = li == 0 ? (g == 0 && lk == 0 ? T(kept.r00) : T(0)) : (4 * g + lk <= li ? T(w[0][g]) : T(0));
         re[NK + g] = w[0][g]; /* o_j, in the lanes li = 0 */
         re[g] = v2[g];
         w[0][NK + g] = rt;

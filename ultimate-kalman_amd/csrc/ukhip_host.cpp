@@ -35,7 +35,7 @@ int uk_bucket_qr(int n);
 hipError_t uk_launch_weigh(const uk_raw_t* raw, const uk_chain_t* out, hipStream_t st);
 hipError_t uk_launch_weigh_obs(const uk_raw_t* raw, const uk_chain_t* out, double* wobs, hipStream_t st);
 hipError_t uk_launch_eliminate(const uk_level_t* lv, const uk_chain_t* in, const uk_chain_t* out,
-                               const uk_factors_t* fac, double* fix, int n, hipStream_t st, hipEvent_t* ev);
+                               const uk_factors_t* fac, double* fix, int n, hipStream_t st, hipEvent_t* ev, int* one);
 hipError_t uk_launch_filter_step(const uk_filter_t* st, const uk_filter_in_t* in, int nf, int n, int first,
                                  hipStream_t s);
 hipError_t uk_launch_filter_smooth(const uk_filter_t* st, int n, int64_t steps, double* xs, double* Ws,
@@ -48,7 +48,7 @@ int uk_assoc_smooth(struct ukhip_batch* b, uint32_t options);
 int uk_assoc_smooth_timed(struct ukhip_batch* b, uint32_t options, double* ms, int32_t* launches);
 void uk_set_error(const char* fmt, ...);
 hipError_t uk_launch_eliminate32(const uk_level_t* lv, const uk_chain32_t* in, const uk_chain32_t* out,
-                                 const uk_factors32_t* fac, float* fix, int n, hipStream_t st, hipEvent_t* ev);
+                                 const uk_factors32_t* fac, float* fix, int n, hipStream_t st, hipEvent_t* ev, int* one);
 hipError_t uk_launch_to32(float* dst, const double* src, int64_t count, hipStream_t st);
 hipError_t uk_launch_weigh_f32(const uk_raw_t* raw, const uk_chain_t* out, const uk_chain32_t* out32, int w64,
                                hipStream_t st);
@@ -1040,7 +1040,7 @@ struct SlotTimer {
     for (auto& e : quad) e = make();
     return quad;
   }
-  /* one: a single launch does the three phases (n <= 16), counted as phase 1 */
+  /* one: a single launch did the three phases, counted as phase 1 */
   void phases_done(bool one) {
     if (!first) first = quad[0];
     last = quad[3];
@@ -1124,10 +1124,11 @@ static bool run_oddeven_view(uk_oe_view_t* v, int cov, SlotTimer* tm, hipStream_
     out.mr = n;
     const uk_factors_t f = fac_at(l);
     uk_level_t lv = v->levels[l]; /* even_start is relative to the level's fac_base */
-    if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, v->fix, n, st, tm ? tm->phases() : nullptr),
+    int one = 0;
+    if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, v->fix, n, st, tm ? tm->phases() : nullptr, &one),
                 "elimination launch"))
       return false;
-    if (tm) tm->phases_done(n <= 16);
+    if (tm) tm->phases_done(one != 0);
   }
   for (int l = nl - 1; l >= 0; --l) {
     const uk_factors_t f = fac_at(l);
@@ -1602,10 +1603,11 @@ static bool run_mixed(ukhip_batch* b, int refinements, int fp32_levels, bool cov
       uk_chain32_t out = b->chain32[(l + 1) & 1]; /* its flags stay 0: a dense chain */
       out.mr = n;
       const uk_factors32_t f = fac32_at(b, l);
-      if (!hip_ok(uk_launch_eliminate32(&lv, &in, &out, &f, b->fix32, n, st, tm ? tm->phases() : nullptr),
+      int one = 0;
+      if (!hip_ok(uk_launch_eliminate32(&lv, &in, &out, &f, b->fix32, n, st, tm ? tm->phases() : nullptr, &one),
                   "FP32 elimination launch"))
         return false;
-      if (tm) tm->phases_done(n <= 16);
+      if (tm) tm->phases_done(one != 0);
       if (l + 1 == lsw && lsw < nl) { /* the next level's chain enters FP64 */
         const size_t ns = (size_t)b->levels[lsw].steps;
         const uk_chain_t& t = top[lsw & 1];
@@ -1625,10 +1627,11 @@ static bool run_mixed(ukhip_batch* b, int refinements, int fp32_levels, bool cov
       uk_chain_t out = top[(l + 1) & 1];
       out.mr = n;
       const uk_factors_t f = fac64(l);
-      if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, b->fix, n, st, tm ? tm->phases() : nullptr),
+      int one = 0;
+      if (!hip_ok(uk_launch_eliminate(&lv, &in, &out, &f, b->fix, n, st, tm ? tm->phases() : nullptr, &one),
                   "FP64 elimination launch"))
         return false;
-      if (tm) tm->phases_done(n <= 16);
+      if (tm) tm->phases_done(one != 0);
     }
   }
   /* x0 from the transformed right-hand sides */
