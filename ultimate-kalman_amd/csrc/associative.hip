@@ -21,15 +21,18 @@
  *                information form
  *   smoothing scan (same scheme, last step first) -> estimates, covariances
  *
- * Every element build and every combine runs in one 256-thread workgroup.
- * Its blocks live in LDS with the odd leading dimension NB + 1, so that the
- * column-per-thread and transposed accesses spread over the LDS banks; the
- * other operand of a combine is staged from HBM into LDS once. (The
- * filtering work blocks of the 64 bucket go to a per-workgroup global slice:
- * six 64 x 65 blocks exceed the 160 KiB of LDS.) Triangular solves keep each
- * right-hand side in one thread's registers. Observations are used whitened
- * (noise covariance I), which is the reference's S = G K G^T + C after the
- * congruence with the whitening W.
+ * Every element build and every combine runs in one workgroup (256 threads, one
+ * wave for n <= 16). Its blocks live in LDS with the odd leading dimension NB +
+ * 1; products run on the FP64 matrix cores straight from there. (The filtering
+ * work blocks of the 64 bucket go to a per-workgroup global slice: seven 64 x
+ * 65 blocks exceed the 160 KiB of LDS.)
+ * Wherever a symmetric positive definite matrix M is inverted in a formula, its
+ * factor takes part instead: with M = G G^T, one forward elimination turns B
+ * into G^{-1} B, and every result is a product of two such blocks
+ * (chol_forward). The filtering combine's (I + Z J)^{-1}, which is not
+ * symmetric, takes two factors: Z = L L^T and N = I + L^T J L (its eigenvalues
+ * are at least 1). Observations are used whitened (noise covariance I), which
+ * is the reference's S = G K G^T + C after the congruence with the whitening W.
  */
 #include <hip/hip_runtime.h>
 
@@ -40,6 +43,7 @@
 
 #include "../../include/kalman.h"
 #include "../../include/ukhip.h"
+#include "oddeven_wave.h"
 #include "ukhip_internal.h"
 
 extern "C" void uk_set_error(const char* fmt, ...);
@@ -48,7 +52,9 @@ extern "C" void* ukhip_stream(void);
 
 namespace {
 
-constexpr int AT = 256;               /* threads of every associative kernel */
+/* threads of the kernels of bucket NB */
+template <int NB>
+constexpr int AT = NB <= 16 ? 64 : 256;
 constexpr int LDS_BYTES = 160 * 1024; /* gfx950 LDS per workgroup */
 
 /* ------------------------------------------------------------------------ */
@@ -60,72 +66,67 @@ __device__ __forceinline__ double at(const double* A, int ld, bool t, int i, int
   return t ? A[k + (int64_t)i * ld] : A[i + (int64_t)k * ld];
 }
 
+typedef double as_d4 __attribute__((ext_vector_type(4)));
+/* D = A B + C on 16 x 16 x 4: lane (li, lk) supplies A[li][lk] and B[lk][li];
+ * element r of the accumulator is D[4 r + lk][li]. So an accumulator is the
+ * next product's B as it stands, and its transpose's A. */
+__device__ __forceinline__ as_d4 as_mfma(double a, double b, as_d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
 /* C (m x q, ld ldc) = alpha op(A) op(B) + beta C with op(A) m x kk and
- * op(B) kk x q. Each thread accumulates a TD x TD register tile. The k loop
- * runs in groups of KU whose loads are all issued before the group's FMAs
- * (one wave per SIMD is typical here, so latency has to be hidden by
- * independent loads); indices are clamped into range and the extra terms
- * zeroed, so there are no branches. Every thread has read its inputs before
- * any output is written, so C may alias A or B. Ends with a barrier. */
+ * op(B) kk x q, on the matrix cores: the waves deal the 16 x 16 tiles of C
+ * between them. Indices are clamped into range (rows and columns beyond C are
+ * not stored) and the terms from kk on zeroed in A and B. Every thread has
+ * read its inputs before any output is written, so C may alias A or B. Ends
+ * with a barrier. */
 template <int NB>
 __device__ void mm(double* C, int ldc, const double* A, int lda, bool tA, const double* B, int ldb, bool tB, int m,
                    int q, int kk, double alpha, double beta) {
-  constexpr int TD = (NB + 15) / 16;
-  constexpr int KU = TD >= 4 ? 4 : 8;
-  const int ti = threadIdx.x % 16, tj = threadIdx.x / 16;
-  int ia[TD], jb[TD];
+  constexpr int TB = (NB + 15) / 16, NW = AT<NB> / 64, PER = (TB * TB + NW - 1) / NW;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4, w = threadIdx.x >> 6;
+  as_d4 acc[PER];
+  int ia[PER], jb[PER];
 #pragma unroll
-  for (int a = 0; a < TD; ++a) {
-    const int i = ti + 16 * a;
-    ia[a] = i < m ? i : m - 1;
+  for (int s = 0; s < PER; ++s) {
+    const int t = w + s * NW, i = (t % TB) * 16 + li, j = (t / TB) * 16 + li;
+    acc[s] = as_d4{0.0, 0.0, 0.0, 0.0};
+    ia[s] = i < m ? i : m - 1;
+    jb[s] = j < q ? j : q - 1;
   }
+#pragma unroll 2
+  for (int k0 = 0; k0 < kk; k0 += 4) {
+    const int k = k0 + lk, kc = k < kk ? k : kk - 1;
+    double av[PER], bv[PER];
 #pragma unroll
-  for (int b = 0; b < TD; ++b) {
-    const int j = tj + 16 * b;
-    jb[b] = j < q ? j : q - 1;
-  }
-  double acc[TD][TD];
-#pragma unroll
-  for (int a = 0; a < TD; ++a)
-#pragma unroll
-    for (int b = 0; b < TD; ++b) acc[a][b] = 0.0;
-  for (int k0 = 0; k0 < kk; k0 += KU) {
-    double av[KU][TD], bv[KU][TD];
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int k = k0 + u < kk ? k0 + u : kk - 1;
-#pragma unroll
-      for (int a = 0; a < TD; ++a) av[u][a] = at(A, lda, tA, ia[a], k);
-#pragma unroll
-      for (int b = 0; b < TD; ++b) bv[u][b] = at(B, ldb, tB, k, jb[b]);
+    for (int s = 0; s < PER; ++s) {
+      av[s] = at(A, lda, tA, ia[s], kc);
+      bv[s] = at(B, ldb, tB, kc, jb[s]);
     }
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      if (k0 + u >= kk) /* uniform: only the last group has a tail */
-#pragma unroll
-        for (int a = 0; a < TD; ++a) av[u][a] = 0.0;
-#pragma unroll
-      for (int a = 0; a < TD; ++a)
-#pragma unroll
-        for (int b = 0; b < TD; ++b) acc[a][b] = fma(av[u][a], bv[u][b], acc[a][b]);
-    }
+    for (int s = 0; s < PER; ++s) acc[s] = as_mfma(k < kk ? av[s] : 0.0, k < kk ? bv[s] : 0.0, acc[s]);
   }
   __syncthreads();
 #pragma unroll
-  for (int a = 0; a < TD; ++a)
+  for (int s = 0; s < PER; ++s) {
+    const int t = w + s * NW;
+    if (t < TB * TB) {
 #pragma unroll
-    for (int b = 0; b < TD; ++b) {
-      const int i = ti + 16 * a, j = tj + 16 * b;
-      if (i < m && j < q) {
-        double* c = &C[i + (int64_t)j * ldc];
-        *c = beta == 0.0 ? alpha * acc[a][b] : fma(beta, *c, alpha * acc[a][b]);
+      for (int r = 0; r < 4; ++r) {
+        const int i = (t % TB) * 16 + 4 * r + lk, j = (t / TB) * 16 + li;
+        if (i < m && j < q) {
+          double* c = &C[i + (int64_t)j * ldc];
+          *c = beta == 0.0 ? alpha * acc[s][r] : fma(beta, *c, alpha * acc[s][r]);
+        }
       }
     }
+  }
   __syncthreads();
 }
 
 /* y (m) = alpha op(A) x + beta y, one thread per row, the k loop in groups
  * of 8 loads with two partial sums; y may alias x. */
+template <int NB>
 __device__ void mv(double* y, const double* A, int lda, bool tA, const double* x, int m, int kk, double alpha,
                    double beta) {
   double r0 = 0.0, r1 = 0.0;
@@ -157,11 +158,11 @@ __device__ void mv(double* y, const double* A, int lda, bool tA, const double* x
  * thread's loads are issued before its stores. */
 template <int NB>
 __device__ void copy_mat(double* D, int ldd, const double* S, int lds, bool t, int m, int q) {
-  constexpr int PER = (NB * NB + AT - 1) / AT;
+  constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
   double v[PER];
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int idx = (int)threadIdx.x + u * AT;
+    const int idx = (int)threadIdx.x + u * AT<NB>;
     const int r = idx % NB, c = idx / NB;
     int i = t ? c : r, j = t ? r : c;
     i = i < m ? i : m - 1;
@@ -170,7 +171,7 @@ __device__ void copy_mat(double* D, int ldd, const double* S, int lds, bool t, i
   }
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int idx = (int)threadIdx.x + u * AT;
+    const int idx = (int)threadIdx.x + u * AT<NB>;
     const int r = idx % NB, c = idx / NB;
     const int i = t ? c : r, j = t ? r : c;
     if (idx < NB * NB && i < m && j < q) D[i + (int64_t)j * ldd] = v[u];
@@ -182,10 +183,10 @@ __device__ void copy_mat(double* D, int ldd, const double* S, int lds, bool t, i
  * [n, NB) of the NB x NB block become the identity. */
 template <int NB>
 __device__ void set_identity(double* D, int ld, int n, double d) {
-  constexpr int PER = (NB * NB + AT - 1) / AT;
+  constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int idx = (int)threadIdx.x + u * AT;
+    const int idx = (int)threadIdx.x + u * AT<NB>;
     const int i = idx % NB, j = idx / NB;
     if (idx < NB * NB) D[i + (int64_t)j * ld] = (i == j) ? (i < n ? d : 1.0) : 0.0;
   }
@@ -193,14 +194,16 @@ __device__ void set_identity(double* D, int ld, int n, double d) {
 }
 
 /* y (m) = a x + y */
+template <int NB>
 __device__ void axpy(double* y, const double* x, int m, double a) {
-  for (int i = threadIdx.x; i < m; i += AT) y[i] = fma(a, x[i], y[i]);
+  for (int i = threadIdx.x; i < m; i += AT<NB>) y[i] = fma(a, x[i], y[i]);
   __syncthreads();
 }
 
 /* y (m) = x */
+template <int NB>
 __device__ void copy_vec(double* y, const double* x, int m) {
-  for (int i = threadIdx.x; i < m; i += AT) y[i] = x[i];
+  for (int i = threadIdx.x; i < m; i += AT<NB>) y[i] = x[i];
   __syncthreads();
 }
 
@@ -235,13 +238,13 @@ struct GJScratch {
  */
 template <int NB>
 __device__ double* gj_inverse(double* A, double* W, int ld, int n, GJScratch<NB>& g) {
-  for (int i = threadIdx.x; i <= NB; i += AT) g.key[i] = 0ull;
+  for (int i = threadIdx.x; i <= NB; i += AT<NB>) g.key[i] = 0ull;
   __syncthreads();
-  for (int r = threadIdx.x; r < n; r += AT) atomicMax(&g.key[0], pivot_key(A[r], r));
+  for (int r = threadIdx.x; r < n; r += AT<NB>) atomicMax(&g.key[0], pivot_key(A[r], r));
   __syncthreads();
   double* cur = A;
   double* nxt = W;
-  constexpr int PER = (NB * NB + AT - 1) / AT;
+  constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
   for (int k = 0; k < n; ++k) {
     const int p = pivot_row(g.key[k]);
     if (threadIdx.x == 0) g.piv[k] = p;
@@ -249,7 +252,7 @@ __device__ double* gj_inverse(double* A, double* W, int ld, int n, GJScratch<NB>
     double pj[PER], fk[PER], aj[PER];
 #pragma unroll
     for (int u = 0; u < PER; ++u) { /* all loads first, indices clamped into the block */
-      const int idx = (int)threadIdx.x + u * AT;
+      const int idx = (int)threadIdx.x + u * AT<NB>;
       const int r = idx < NB * NB ? idx % NB : 0, j = idx < NB * NB ? idx / NB : 0;
       const int sr = (r == p) ? k : (r == k ? p : r);
       pj[u] = cur[p + j * ld];
@@ -258,7 +261,7 @@ __device__ double* gj_inverse(double* A, double* W, int ld, int n, GJScratch<NB>
     }
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int idx = (int)threadIdx.x + u * AT;
+      const int idx = (int)threadIdx.x + u * AT<NB>;
       const int r = idx % NB, j = idx / NB;
       if (idx < NB * NB && r < n && j < n) {
         const double rowk = (j == k ? 1.0 : pj[u]) * rp;
@@ -282,7 +285,7 @@ __device__ double* gj_inverse(double* A, double* W, int ld, int n, GJScratch<NB>
     }
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < NB * NB; idx += AT) {
+  for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
     const int r = idx % NB, j = idx / NB;
     if (r < n && j < n) nxt[r + j * ld] = cur[r + g.col[j] * ld];
   }
@@ -299,94 +302,213 @@ __device__ double* inverse(const double* A, double* W1, double* W2, int ld, int 
   return gj_inverse<NB>(W1, W2, ld, n, g);
 }
 
-/* LU with partial pivoting (LAPACK dgetrf order, whole rows swapped) of the
- * leading n x n block of M (ld) in place; row k was interchanged with row
- * piv[k] at step k. Used where the matrices can be ill-conditioned
- * (information-form steps, smoothing gains): solving with the factors keeps
- * the error at the level of a backward-stable solve, where multiplying by an
- * explicit inverse can lose a further factor. */
-template <int NB>
-__device__ void lu(double* M, int ld, int n, int* piv, GJScratch<NB>& g) {
-  for (int i = threadIdx.x; i <= NB; i += AT) g.key[i] = 0ull;
-  __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    for (int r = k + (int)threadIdx.x; r < n; r += AT) atomicMax(&g.key[k], pivot_key(M[r + k * ld], r));
+/*
+ * One step of the Cholesky factorization of a symmetric positive definite 16 x
+ * 16 tile on one wave (accumulator layout): a is reduced to D L^T (row K final
+ * at step K), wt becomes the transposed inverse of the unit lower factor. The
+ * pivots are kept by row (pr) and by column (pc). FLOOR: a pivot below fl (lane
+ * li: of row li), the rounding error of its original diagonal entry, counts as
+ * that error, so that a semidefinite matrix has a factor too (a perturbation
+ * of the size of the matrix's own rounding); NaN stays NaN.
+ */
+template <int K, bool FLOOR>
+__device__ __forceinline__ void chol_step(double (&a)[4], double (&wt)[4], double (&pr)[4], double& pc, double fl,
+                                          int li, int lk) {
+  constexpr int G = K / 4, KR = K % 4;
+  double x[4];
+#pragma unroll
+  for (int g = G; g < 4; ++g) x[g] = row_lane<K>(a[g]);
+  double p = one_lane(x[G], 16 * KR);
+  if (FLOOR) {
+    const double f = one_lane(fl, K);
+    p = p < f ? f : p;
+  }
+  double rp = __builtin_amdgcn_rcp(p);
+  rp = fma(fma(-p, rp, 1.0), rp, rp);
+  rp = fma(fma(-p, rp, 1.0), rp, rp);
+  const double row = rows_sum(lk == KR ? a[G] : 0.0) * rp; /* row K over the pivot, on every lane row */
+  x[G] = lk > KR ? x[G] : 0.0;
+#pragma unroll
+  for (int g = G; g < 4; ++g) a[g] = fma(-x[g], row, a[g]);
+  const double m = li > K ? row : 0.0;
+#pragma unroll
+  for (int g = 0; g <= G; ++g) wt[g] = fma(-row_lane<K>(wt[g]), m, wt[g]);
+  pr[G] = lk == KR ? p : pr[G];
+  pc = li == K ? p : pc;
+}
+template <bool FLOOR, int... K>
+__device__ __forceinline__ void chol_steps(double (&a)[4], double (&wt)[4], double (&pr)[4], double& pc,
+                                           double fl, int lim, int li, int lk,
+                                           std::integer_sequence<int, K...>) {
+  auto one = [&](auto k) {
+    if (k.value < lim) chol_step<k.value, FLOOR>(a, wt, pr, pc, fl, li, lk);
+  };
+  (one(std::integral_constant<int, K>{}), ...);
+}
+__device__ __forceinline__ double rsqrt_ulp(double p) {
+  const double y = __builtin_amdgcn_rsq(p);
+  const double y1 = fma(0.5 * y, fma(-p * y, y, 1.0), y);
+  return fma(0.5 * y1, fma(-p * y1, y1, 1.0), y1);
+}
+
+/*
+ * Forward elimination with a symmetric positive definite M = G G^T (n x n, ld,
+ * both triangles given): every block B[i] (n x q, ldb) and every vector (nv of
+ * them at v, NB apart) becomes G^{-1} times itself. KEEP: M becomes G (lower
+ * triangular, zeros above), else it is left half reduced.
+ * Panels of 16: each wave factors the panel's diagonal tile in its registers
+ * (the same work on every wave, instead of a barrier), takes T_r = G_pp^{-1}
+ * M_pr for the block rows r below, and then 16 columns at a time of what is
+ * dealt to it: T = G_pp^{-1} X_p, X_r -= T_r^T T. One barrier per panel.
+ * A pivoted Gauss-Jordan inverse in LDS, one barrier per column, took this
+ * place: 138 us a filtering combine at n = 48 with it.
+ */
+template <int NB, bool KEEP, bool FLOOR, int NBLK>
+__device__ void chol_forward(double* M, int ld, int n, double* const (&B)[NBLK], int q, int ldb, double* v, int nv) {
+  constexpr int TB = (NB + 15) / 16, NW = AT<NB> / 64;
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int tn = (n + 15) >> 4, tq = (q + 15) >> 4;
+  double diag[TB];
+  if (FLOOR) {
+#pragma unroll
+    for (int p = 0; p < TB; ++p) diag[p] = 16 * p + li < n ? fmax(2.2e-16 * M[(16 * p + li) * (ld + 1)], 1e-290) : 0.0;
     __syncthreads();
-    const int pr = pivot_row(g.key[k]);
-    if (pr != k)
-      for (int j = threadIdx.x; j < n; j += AT) {
-        const double t = M[k + j * ld];
-        M[k + j * ld] = M[pr + j * ld];
-        M[pr + j * ld] = t;
+  }
+#pragma unroll 1
+  for (int p = 0; p < tn; ++p) {
+    const int p0 = 16 * p;
+    double a[4], wt[4], pr[4], pc = 1.0, fl = 0.0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int r = 4 * g + lk;
+      const bool in = p0 + r < n && p0 + li < n;
+      const double x = M[in ? p0 + r + (p0 + li) * ld : 0];
+      a[g] = in ? x : (r == li ? 1.0 : 0.0);
+      wt[g] = r == li ? 1.0 : 0.0;
+      pr[g] = 1.0;
+    }
+    if (FLOOR) {
+#pragma unroll
+      for (int i = 0; i < TB; ++i) fl = p == i ? diag[i] : fl;
+    }
+    chol_steps<FLOOR>(a, wt, pr, pc, fl, n - p0, li, lk, std::make_integer_sequence<int, 16>{});
+    const double sc = rsqrt_ulp(pc);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) wt[g] *= sc; /* G_pp^{-T}: A operand of G_pp^{-1} */
+    auto row_tile = [&](const double* X, int ldx, int cols, double (&t)[4]) { /* t = G_pp^{-1} X_p, 16 columns at X */
+      double b[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int r = p0 + 4 * g + lk;
+        const bool in = r < n && li < cols;
+        const double x = X[in ? r + (int64_t)li * ldx : 0];
+        b[g] = in ? x : 0.0;
       }
-    if (threadIdx.x == 0) piv[k] = pr;
+      as_d4 acc = as_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int g = 0; g < 4; ++g) acc = as_mfma(wt[g], b[g], acc);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) t[g] = acc[g];
+    };
+    double tr[TB > 1 ? TB - 1 : 1][4];
+#pragma unroll
+    for (int i = 0; i < TB - 1; ++i)
+      if (p + 1 + i < tn) row_tile(M + (p0 + 16 * (1 + i)) * ld, ld, n - (p0 + 16 * (1 + i)), tr[i]);
+    const int trail = tn - 1 - p, tot = trail + NBLK * tq + (nv > 0 ? 1 : 0);
+    for (int t = w; t < tot; t += NW) {
+      double* X;
+      int ldx, cols;
+      if (t < trail) {
+        X = M + (p0 + 16 * (1 + t)) * ld;
+        ldx = ld;
+        cols = n - (p0 + 16 * (1 + t));
+      } else if (t < trail + NBLK * tq) {
+        const int u = t - trail, blk = u / tq, c0 = 16 * (u - blk * tq);
+        double* Bb = B[0];
+#pragma unroll
+        for (int i = 1; i < NBLK; ++i) Bb = blk == i ? B[i] : Bb;
+        X = Bb + (int64_t)c0 * ldb;
+        ldx = ldb;
+        cols = q - c0;
+      } else {
+        X = v;
+        ldx = NB;
+        cols = nv;
+      }
+      double tc[4];
+      row_tile(X, ldx, cols, tc);
+      if (t >= trail && li < cols) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          if (p0 + 4 * g + lk < n) X[p0 + 4 * g + lk + (int64_t)li * ldx] = tc[g];
+      }
+#pragma unroll
+      for (int i = 0; i < TB - 1; ++i) {
+        const int r0 = p0 + 16 * (1 + i);
+        if (r0 < n) {
+          as_d4 acc;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const bool in = r0 + 4 * g + lk < n && li < cols;
+            const double x = X[in ? r0 + 4 * g + lk + (int64_t)li * ldx : 0];
+            acc[g] = in ? x : 0.0;
+          }
+#pragma unroll
+          for (int g = 0; g < 4; ++g) acc = as_mfma(-tr[i][g], tc[g], acc);
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (r0 + 4 * g + lk < n && li < cols) X[r0 + 4 * g + lk + (int64_t)li * ldx] = acc[g];
+        }
+      }
+    }
+    if (KEEP) { /* G_rp = T_r^T, below the diagonal, where this panel reads nothing */
+#pragma unroll
+      for (int i = 0; i < TB - 1; ++i) {
+        const int r = p0 + 16 * (1 + i) + li;
+        if (i % NW == w && r < n) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (p0 + 4 * g + lk < n) M[r + (p0 + 4 * g + lk) * ld] = tr[i][g];
+        }
+      }
+    }
     __syncthreads();
-    const double d = M[k + k * ld];
-    for (int i = k + 1 + (int)threadIdx.x; i < n; i += AT) M[i + k * ld] /= d;
-    __syncthreads();
-    const int rem = n - k - 1;
-    for (int idx = threadIdx.x; idx < rem * rem; idx += AT) {
-      const int i = k + 1 + idx % rem, j = k + 1 + idx / rem;
-      M[i + j * ld] = fma(-M[i + k * ld], M[k + j * ld], M[i + j * ld]);
+    if (KEEP && w == 0) { /* G_pp = (D^{-1/2} a)^T; no later panel reads this block */
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int k = 4 * g + lk;
+        if (p0 + k < n && p0 + li < n) M[p0 + li + (p0 + k) * ld] = li >= k ? a[g] * rsqrt_ulp(pr[g]) : 0.0;
+      }
+    }
+  }
+  if (KEEP) {
+    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
+      const int i = idx % NB, j = idx / NB;
+      if (i < n && j < n && (i >> 4) < (j >> 4)) M[i + j * ld] = 0.0;
     }
     __syncthreads();
   }
 }
 
-/* X (n x q, ld ldx) <- A^{-1} X, or A^{-T} X when trans, with the factors of
- * lu(A): one thread per right-hand side, in place. */
-__device__ void lu_solve(const double* M, int ld, const int* piv, int n, double* X, int ldx, int q, bool trans) {
-  for (int j = threadIdx.x; j < q; j += AT) {
-    double* x = X + (int64_t)j * ldx;
-    if (!trans) {
-      for (int k = 0; k < n; ++k)
-        if (piv[k] != k) {
-          const double t = x[k];
-          x[k] = x[piv[k]];
-          x[piv[k]] = t;
-        }
-      for (int i = 0; i < n; ++i) {
-        double s = x[i];
-        for (int k = 0; k < i; ++k) s = fma(-M[i + k * ld], x[k], s);
-        x[i] = s;
-      }
-      for (int i = n - 1; i >= 0; --i) {
-        double s = x[i];
-        for (int k = i + 1; k < n; ++k) s = fma(-M[i + k * ld], x[k], s);
-        x[i] = s / M[i + i * ld];
-      }
-    } else {
-      for (int i = 0; i < n; ++i) {
-        double s = x[i];
-        for (int k = 0; k < i; ++k) s = fma(-M[k + i * ld], x[k], s);
-        x[i] = s / M[i + i * ld];
-      }
-      for (int i = n - 1; i >= 0; --i) {
-        double s = x[i];
-        for (int k = i + 1; k < n; ++k) s = fma(-M[k + i * ld], x[k], s);
-        x[i] = s;
-      }
-      for (int k = n - 1; k >= 0; --k)
-        if (piv[k] != k) {
-          const double t = x[k];
-          x[k] = x[piv[k]];
-          x[piv[k]] = t;
-        }
-    }
-  }
-  __syncthreads();
+/* W (ld) <- G^{-1} of M = G G^T (M is consumed); M^{-1} = W^T W */
+template <int NB>
+__device__ void chol_inverse_factor(double* M, double* W, int ld, int n) {
+  set_identity<NB>(W, ld, n, 1.0);
+  double* const B[1] = {W};
+  chol_forward<NB, false, false>(M, ld, n, B, n, ld, nullptr, 0);
 }
 
 /* Per-thread registers holding an n x n global block (ld n) distributed over
- * the NB x NB grid: entry idx = threadIdx.x + u * AT. */
+ * the NB x NB grid: entry idx = threadIdx.x + u * AT<NB>. */
 template <int NB>
 struct RegBlk {
-  static constexpr int PER = (NB * NB + AT - 1) / AT;
+  static constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
   double v[PER];
   __device__ void load(const double* G, int n) {
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int idx = (int)threadIdx.x + u * AT;
+      const int idx = (int)threadIdx.x + u * AT<NB>;
       const int i = idx % NB, j = idx / NB;
       v[u] = (idx < NB * NB && i < n && j < n) ? G[i + (int64_t)j * n] : 0.0;
     }
@@ -395,7 +517,7 @@ struct RegBlk {
   __device__ void store(double* D, int ld, int n, bool t) const {
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const int idx = (int)threadIdx.x + u * AT;
+      const int idx = (int)threadIdx.x + u * AT<NB>;
       const int i = idx % NB, j = idx / NB;
       if (idx < NB * NB && i < n && j < n) D[t ? j + i * ld : i + j * ld] = v[u];
     }
@@ -444,7 +566,7 @@ struct Ld {
 /* ------------------------------------------------------------------------ */
 
 template <int NB>
-__global__ void __launch_bounds__(AT) ka_model(uk_chain_t wch, const int8_t* first, AsModel md, int n) {
+__global__ void __launch_bounds__(AT<NB>) ka_model(uk_chain_t wch, const int8_t* first, AsModel md, int n) {
   constexpr int L = Ld<NB>::L;
   __shared__ double B0[Ld<NB>::SZ], B1[Ld<NB>::SZ], B2[Ld<NB>::SZ];
   __shared__ GJScratch<NB> g;
@@ -456,8 +578,24 @@ __global__ void __launch_bounds__(AT) ka_model(uk_chain_t wch, const int8_t* fir
   double* Bw = B0;
   copy_mat<NB>(Bw, L, wch.B + s * nn, n, false, n, n);
   mm<NB>(md.F + s * nn, n, Di, L, false, Bw, L, false, n, n, n, -1.0, 0.0);   /* F = -D^{-1} B */
-  mv(md.c + s * n, Di, L, false, wch.c + s * n, n, n, 1.0, 0.0);             /* c = D^{-1} c_w */
+  mv<NB>(md.c + s * n, Di, L, false, wch.c + s * n, n, n, 1.0, 0.0);             /* c = D^{-1} c_w */
   mm<NB>(md.Q + s * nn, n, Di, L, false, Di, L, true, n, n, n, 1.0, 0.0);     /* Q = D^{-1} D^{-T} */
+}
+
+/* The same where every H is the identity and every K given as 'w': the model is
+ * the input's, Q = diag(1 / k^2). Consecutive threads, consecutive elements. */
+__global__ void __launch_bounds__(256) ka_model_diag(uk_raw_t raw, AsModel md, int n) {
+  const int64_t s = blockIdx.x;
+  if (raw.first[s]) return;
+  const int nn = n * n;
+  const double* F = raw.F + raw.Fidx[s] * nn;
+  for (int i = threadIdx.x; i < nn; i += 256) {
+    const int c = i / n, r = i - c * n;
+    const double k = raw.K[s * n + c];
+    md.F[s * nn + i] = F[i];
+    md.Q[s * nn + i] = r == c ? 1.0 / (k * k) : 0.0;
+  }
+  for (int i = threadIdx.x; i < n; i += 256) md.c[s * n + i] = raw.c[s * n + i];
 }
 
 /* ------------------------------------------------------------------------ */
@@ -465,63 +603,59 @@ __global__ void __launch_bounds__(AT) ka_model(uk_chain_t wch, const int8_t* fir
 /* ------------------------------------------------------------------------ */
 
 template <int NB>
-__global__ void __launch_bounds__(AT) ka_prior(const AsProb* probs, uk_chain_t wch, const int32_t* m_obs, AsModel md,
-                                               int n, int mr) {
+__global__ void __launch_bounds__(AT<NB>) ka_prior(const AsProb* probs, uk_chain_t wch, const int32_t* m_obs, AsModel md,
+                                                   int n, int mr) {
   constexpr int L = Ld<NB>::L;
   __shared__ double Lm[Ld<NB>::SZ], Mx[Ld<NB>::SZ], Qi[Ld<NB>::SZ], T2[Ld<NB>::SZ];
   __shared__ double et[NB], v1[NB], v2[NB];
-  __shared__ int piv[NB];
-  __shared__ GJScratch<NB> g;
   const AsProb pr = probs[blockIdx.x];
   const int64_t nn = (int64_t)n * n;
   set_identity<NB>(Lm, L, n, 0.0);
-  for (int i = threadIdx.x; i < n; i += AT) et[i] = 0.0;
+  for (int i = threadIdx.x; i < n; i += AT<NB>) et[i] = 0.0;
   __syncthreads();
   for (int64_t t = 0; t <= pr.p; ++t) {
     const int64_t s = pr.s0 + t;
     if (t > 0) {
-      /* predict: with Mx = Lam + F^T Q^{-1} F and r = eta - F^T Q^{-1} c,
-       * Lam <- Q^{-1} - Q^{-1} F Mx^{-1} F^T Q^{-1}, eta <- Q^{-1} c + Q^{-1} F Mx^{-1} r */
+      /* predict: with Mx = Lam + F^T Q^{-1} F = G G^T and r = eta - F^T Q^{-1} c,
+       * Lam <- Q^{-1} - Y^T Y, eta <- Q^{-1} c + Y^T y,
+       * Y = G^{-1} F^T Q^{-1}, y = G^{-1} r */
       const double* F = md.F + s * nn;
       copy_mat<NB>(Mx, L, md.Q + s * nn, n, false, n, n);
-      lu<NB>(Mx, L, n, piv, g);
-      set_identity<NB>(Qi, L, n, 1.0);
-      lu_solve(Mx, L, piv, n, Qi, L, n, false);                              /* Qi = Q^{-1} */
+      chol_inverse_factor<NB>(Mx, Qi, L, n);
+      mm<NB>(Qi, L, Qi, L, true, Qi, L, false, n, n, n, 1.0, 0.0);            /* Qi = Q^{-1} */
       mm<NB>(T2, L, Qi, L, false, F, n, false, n, n, n, 1.0, 0.0);            /* T2 = Q^{-1} F */
       copy_mat<NB>(Mx, L, Lm, L, false, n, n);
       mm<NB>(Mx, L, F, n, true, T2, L, false, n, n, n, 1.0, 1.0);             /* Mx = Lam + F^T T2 */
-      mv(v1, Qi, L, false, md.c + s * n, n, n, 1.0, 0.0);                    /* v1 = Q^{-1} c */
-      mv(v2, F, n, true, v1, n, n, -1.0, 0.0);
-      axpy(v2, et, n, 1.0);                                                  /* v2 = r */
-      lu<NB>(Mx, L, n, piv, g);
-      lu_solve(Mx, L, piv, n, v2, NB, 1, false);                             /* v2 = Mx^{-1} r */
+      mv<NB>(v1, Qi, L, false, md.c + s * n, n, n, 1.0, 0.0);                /* v1 = Q^{-1} c */
+      mv<NB>(v2, F, n, true, v1, n, n, -1.0, 0.0);
+      axpy<NB>(v2, et, n, 1.0);                                              /* v2 = r */
       copy_mat<NB>(Lm, L, T2, L, true, n, n);                                /* Lm = T2^T */
-      lu_solve(Mx, L, piv, n, Lm, L, n, false);                              /* Lm = Mx^{-1} T2^T */
-      mm<NB>(Qi, L, T2, L, false, Lm, L, false, n, n, n, -1.0, 1.0);
-      copy_mat<NB>(Lm, L, Qi, L, false, n, n);                               /* Lam- */
-      mv(et, T2, L, false, v2, n, n, 1.0, 0.0);
-      axpy(et, v1, n, 1.0);                                                  /* eta- */
+      double* const B[1] = {Lm};
+      chol_forward<NB, false, false>(Mx, L, n, B, n, L, v2, 1);              /* Lm = Y, v2 = y */
+      mm<NB>(Qi, L, Lm, L, true, Lm, L, false, n, n, n, -1.0, 1.0);           /* Lam- */
+      mv<NB>(et, Lm, L, true, v2, n, n, 1.0, 0.0);
+      axpy<NB>(et, v1, n, 1.0);                                              /* eta- */
+      copy_mat<NB>(Lm, L, Qi, L, false, n, n);
     }
     const int m = m_obs[s];
     if (m > 0) { /* update: Lam += C^T C, eta += C^T o (whitened) */
       const double* Cw = wch.C + s * nn;
       mm<NB>(Lm, L, Cw, mr, true, Cw, mr, false, n, n, m, 1.0, 1.0);
-      mv(et, Cw, mr, true, wch.o + s * n, n, m, 1.0, 1.0);
+      mv<NB>(et, Cw, mr, true, wch.o + s * n, n, m, 1.0, 1.0);
     }
     if (t < pr.p) {
       copy_mat<NB>(md.Lam + s * nn, n, Lm, L, false, n, n);
-      for (int i = threadIdx.x; i < n; i += AT) md.eta[s * n + i] = et[i];
+      for (int i = threadIdx.x; i < n; i += AT<NB>) md.eta[s * n + i] = et[i];
       __syncthreads();
     }
   }
   /* P_p = Lam^{-1}, x_p = P_p eta */
   const int64_t sp = pr.s0 + pr.p;
   copy_mat<NB>(Mx, L, Lm, L, false, n, n);
-  lu<NB>(Mx, L, n, piv, g);
-  set_identity<NB>(Qi, L, n, 1.0);
-  lu_solve(Mx, L, piv, n, Qi, L, n, false);
+  chol_inverse_factor<NB>(Mx, Qi, L, n);
+  mm<NB>(Qi, L, Qi, L, true, Qi, L, false, n, n, n, 1.0, 0.0);
   copy_mat<NB>(md.Pf + sp * nn, n, Qi, L, false, n, n);
-  mv(md.xf + sp * n, Qi, L, false, et, n, n, 1.0, 0.0);
+  mv<NB>(md.xf + sp * n, Qi, L, false, et, n, n, 1.0, 0.0);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -529,23 +663,22 @@ __global__ void __launch_bounds__(AT) ka_prior(const AsProb* probs, uk_chain_t w
 /* ------------------------------------------------------------------------ */
 
 /*
- * Step s with model (F, c, Q) and whitened observation (C, o), noise I:
- *   S = C Q C^T + I, gain K = Q C^T S^{-1} = T^T with T = S^{-1} C Q,
- *   A = F - K C F,  b = c + K (o - C c),  Z = Q - K C Q,
- *   e = (C F)^T S^{-1} (o - C c),  J = (C F)^T S^{-1} C F.
+ * Step s with model (F, c, Q) and whitened observation (C, o), noise I: with
+ * S = C Q C^T + I = G G^T, Y_1 = G^{-1} C Q, Y_2 = G^{-1} C F,
+ *   A = F - Y_1^T Y_2,  b = c + Y_1^T G^{-1} (o - C c),  Z = Q - Y_1^T Y_1,
+ *   e = Y_2^T G^{-1} (o - C c),  J = Y_2^T Y_2.
  * The first element after the prior (x_p, P_p) uses Q1 = Q + F P_p F^T in
- * place of Q, A = 0, and b = m1 + K (o - C m1) with m1 = F x_p + c
- * (Z = Q1 - K S K^T = Q1 - K C Q1). Unobserved: A = F (0 if first), b = c
+ * place of Q, A = 0, and b = m1 + Y_1^T G^{-1} (o - C m1) with m1 = F x_p + c.
+ * Unobserved: A = F (0 if first), b = c
  * (m1 if first), Z = Q (Q1), e = 0, J = 0.
  */
 template <int NB>
-__global__ void __launch_bounds__(AT) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
+__global__ void __launch_bounds__(AT<NB>) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
                                                const int32_t* m_obs, AsModel md, AsElems el, int n, int mr) {
   constexpr int L = Ld<NB>::L;
   __shared__ double Qs[Ld<NB>::SZ], CQ[Ld<NB>::SZ], S[Ld<NB>::SZ], T[Ld<NB>::SZ];
-  __shared__ double w1[NB], r[NB], rc[NB];
-  __shared__ int piv[NB];
-  __shared__ GJScratch<NB> g;
+  __shared__ double w1[NB], rr[2 * NB];
+  double *const r = rr, *const rc = rr + NB;
   const int64_t ge = blockIdx.x;
   const AsProb pr = probs[elem_prob[ge]];
   const int64_t t = ge - pr.e0 + pr.p + 1;
@@ -562,15 +695,15 @@ __global__ void __launch_bounds__(AT) ka_felem(const AsProb* probs, const int32_
   const int64_t spv = pr.s0 + pr.p;
 
   copy_mat<NB>(Qs, L, md.Q + s * nn, n, false, n, n);                       /* Qs = Q */
-  copy_vec(w1, c, n);
+  copy_vec<NB>(w1, c, n);
   if (firstel) { /* Q1 = Q + F P F^T, m1 = F x + c */
     mm<NB>(T, L, F, n, false, md.Pf + spv * nn, n, false, n, n, n, 1.0, 0.0);
     mm<NB>(Qs, L, T, L, false, F, n, true, n, n, n, 1.0, 1.0);
-    mv(w1, F, n, false, md.xf + spv * n, n, n, 1.0, 1.0);
+    mv<NB>(w1, F, n, false, md.xf + spv * n, n, n, 1.0, 1.0);
   }
   const int m = m_obs[s];
   if (m == 0) {
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT) {
+    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
       const int i = idx % NB, j = idx / NB;
       if (i < n && j < n) {
         A[i + j * n] = firstel ? 0.0 : F[i + j * n];
@@ -578,7 +711,7 @@ __global__ void __launch_bounds__(AT) ka_felem(const AsProb* probs, const int32_
         J[i + j * n] = 0.0;
       }
     }
-    for (int i = threadIdx.x; i < n; i += AT) {
+    for (int i = threadIdx.x; i < n; i += AT<NB>) {
       b[i] = w1[i];
       e[i] = 0.0;
     }
@@ -589,36 +722,29 @@ __global__ void __launch_bounds__(AT) ka_felem(const AsProb* probs, const int32_
   mm<NB>(CQ, L, T, L, false, Qs, L, false, m, n, n, 1.0, 0.0);               /* CQ = C Q */
   set_identity<NB>(S, L, m, 1.0);
   mm<NB>(S, L, CQ, L, false, T, L, true, m, m, n, 1.0, 1.0);                 /* S = C Q C^T + I */
-  mv(r, T, L, false, w1, m, n, -1.0, 0.0);
-  axpy(r, ow, m, 1.0);                                                       /* r = o - C w1 */
-  mv(rc, T, L, false, c, m, n, -1.0, 0.0);
-  axpy(rc, ow, m, 1.0);                                                      /* rc = o - C c */
-  mm<NB>(J, n, T, L, false, F, n, false, m, n, n, 1.0, 0.0);                 /* C F, parked in J's slot */
+  mv<NB>(r, T, L, false, w1, m, n, -1.0, 0.0);
+  axpy<NB>(r, ow, m, 1.0);                                                       /* r = o - C w1 */
+  mv<NB>(rc, T, L, false, c, m, n, -1.0, 0.0);
+  axpy<NB>(rc, ow, m, 1.0);                                                      /* rc = o - C c */
   copy_mat<NB>(Z, n, Qs, L, false, n, n);                                    /* Z = Q (Qs is free now) */
-  /* S can be ill-conditioned on the first element (Q1 holds the prior
-   * covariance): LU solves rather than an explicit inverse */
-  lu<NB>(S, L, m, piv, g);
-  copy_mat<NB>(T, L, CQ, L, false, m, n);
-  lu_solve(S, L, piv, m, T, L, n, false);                                    /* T = S^{-1} C Q (the gain^T) */
-  mv(b, T, L, true, r, n, m, 1.0, 0.0);
-  axpy(b, w1, n, 1.0);                                                       /* b = w1 + gain r */
-  mm<NB>(Z, n, T, L, true, CQ, L, false, n, n, m, -1.0, 1.0);                /* Z = Q - gain C Q */
-  copy_mat<NB>(CQ, L, J, n, false, m, n);                                    /* CQ <- C F */
+  mm<NB>(Qs, L, T, L, false, F, n, false, m, n, n, 1.0, 0.0);                /* Qs = C F */
+  double* const B[2] = {CQ, Qs};
+  chol_forward<NB, false, false>(S, L, m, B, n, L, rr, 2);                   /* CQ = Y_1, Qs = Y_2, r, rc = G^{-1} of them */
+  mv<NB>(b, CQ, L, true, r, n, m, 1.0, 0.0);
+  axpy<NB>(b, w1, n, 1.0);                                                   /* b = w1 + Y_1^T r */
+  mm<NB>(Z, n, CQ, L, true, CQ, L, false, n, n, m, -1.0, 1.0);               /* Z = Q - Y_1^T Y_1 */
   if (firstel) {
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT) {
+    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
       const int i = idx % NB, j = idx / NB;
       if (i < n && j < n) A[i + j * n] = 0.0;
     }
     __syncthreads();
   } else {
     copy_mat<NB>(A, n, F, n, false, n, n);
-    mm<NB>(A, n, T, L, true, CQ, L, false, n, n, m, -1.0, 1.0);              /* A = F - gain C F */
+    mm<NB>(A, n, CQ, L, true, Qs, L, false, n, n, m, -1.0, 1.0);             /* A = F - Y_1^T Y_2 */
   }
-  lu_solve(S, L, piv, m, rc, NB, 1, false);                                  /* rc = S^{-1} (o - C c) */
-  mv(e, CQ, L, true, rc, n, m, 1.0, 0.0);                                    /* e = (C F)^T S^{-1} rc */
-  copy_mat<NB>(T, L, CQ, L, false, m, n);
-  lu_solve(S, L, piv, m, T, L, n, false);                                    /* T = S^{-1} C F */
-  mm<NB>(J, n, CQ, L, true, T, L, false, n, n, m, 1.0, 0.0);                 /* J = (C F)^T S^{-1} C F */
+  mv<NB>(e, Qs, L, true, rc, n, m, 1.0, 0.0);                                /* e = Y_2^T rc */
+  mm<NB>(J, n, Qs, L, true, Qs, L, false, n, n, m, 1.0, 0.0);                /* J = Y_2^T Y_2 */
 }
 
 /* ------------------------------------------------------------------------ */
@@ -632,14 +758,21 @@ struct Blk {
 };
 template <int NB>
 struct Work {
-  double *M, *W1, *W2, *R, *T, *v1, *v2;
-  GJScratch<NB>* g;
+  double *W1, *T, *T2, *Aj; /* W1: J_j, or E_j of the smoothing combine */
+  double *v, *t0;           /* two vectors, NB apart; one */
 };
 
-/* a <- a (x) element g, filtering:
- *   M = I + Z_i J_j,  Y^T = M^{-1} A_i,  X = A_j M^{-1},
- *   e = Y (e_j - J_j b_i) + e_i,  J = Y J_j A_i + J_i,
- *   b = X (b_i + Z_i e_j) + b_j,  Z = X Z_i A_j^T + Z_j,  A = X A_i.
+/* a <- a (x) element g, filtering (A, b, Z, e, J of the reference's combine):
+ *   A = A_j (I + Z_i J_j)^{-1} A_i,       b = A_j (I + Z_i J_j)^{-1} (b_i + Z_i e_j) + b_j,
+ *   Z = A_j (I + Z_i J_j)^{-1} Z_i A_j^T + Z_j,
+ *   e = A_i^T (I + J_j Z_i)^{-1} (e_j - J_j b_i) + e_i,
+ *   J = A_i^T (I + J_j Z_i)^{-1} J_j A_i + J_i.
+ * With Z_i = L L^T and N = I + L^T J_j L = G G^T: (I + Z_i J_j)^{-1} = L N^{-1}
+ * L^{-1}, so that with Y_1 = G^{-1} L^{-1} A_i, Y_2 = G^{-1} L^T J_j A_i, Y_b =
+ * G^{-1} L^T A_j^T, y_0 = G^{-1} (L^{-1} b_i + L^T e_j), y_1 = G^{-1} L^T (e_j -
+ * J_j b_i):
+ *   A = Y_b^T Y_1, b = Y_b^T y_0 + b_j, Z = Y_b^T Y_b + Z_j, e = Y_1^T y_1 + e_i,
+ *   J = Y_1^T Y_2 + J_i.
  * Element g's blocks are read from HBM into registers first (all loads in
  * flight together) and written into LDS where they are needed. */
 template <int NB>
@@ -647,40 +780,46 @@ __device__ void filt_combine(const Blk& a, const Work<NB>& w, const AsElems& el,
   constexpr int L = Ld<NB>::L;
   const int64_t nn = (int64_t)n * n;
   const double *bj = el.b + g * n, *ej = el.e + g * n;
-  /* Up to NB = 48 all three blocks are requested at once; the 64 bucket
-   * fetches A_j and Z_j where they are used, to stay within its registers. */
+  /* Up to NB = 48 Z_j is requested with the others; the 64 bucket fetches it
+   * where it is used, to stay within its registers. */
   constexpr bool EARLY = NB <= 48;
   RegBlk<NB> rA, rZ, rJ;
   rJ.load(el.J + g * nn, n);
-  if (EARLY) {
-    rA.load(el.A + g * nn, n);
-    rZ.load(el.Z + g * nn, n);
+  rA.load(el.A + g * nn, n);
+  if (EARLY) rZ.load(el.Z + g * nn, n);
+  rJ.store(w.W1, L, n, false);
+  rA.store(w.Aj, L, n, false);
+  for (int i = threadIdx.x; i < n; i += AT<NB>) {
+    w.v[i] = a.b[i];
+    w.t0[i] = ej[i];
   }
-  rJ.store(w.T, L, n, false);                                                /* T = J_j */
-  set_identity<NB>(w.M, L, n, 1.0);
-  mm<NB>(w.M, L, a.Z, L, false, w.T, L, false, n, n, n, 1.0, 1.0);           /* M = I + Z_i J_j */
-  mv(w.v2, w.T, L, false, a.b, n, n, -1.0, 0.0);
-  axpy(w.v2, ej, n, 1.0);                                                    /* v2 = e_j - J_j b_i */
-  mm<NB>(w.T, L, w.T, L, false, a.A, L, false, n, n, n, 1.0, 0.0);           /* T = J_j A_i */
-  double* Mi = inverse<NB>(w.M, w.W1, w.W2, L, n, *w.g);                     /* M^{-1} */
-  double* F = w.M;
-  mm<NB>(F, L, Mi, L, false, a.A, L, false, n, n, n, 1.0, 0.0);              /* F = Y^T */
-  mv(a.e, F, L, true, w.v2, n, n, 1.0, 1.0);                                 /* e */
-  mm<NB>(a.J, L, F, L, true, w.T, L, false, n, n, n, 1.0, 1.0);              /* J */
-  if (!EARLY) rA.load(el.A + g * nn, n);
-  rA.store(w.R, L, n, false);                                                /* R = A_j */
   __syncthreads();
-  mm<NB>(w.T, L, w.R, L, false, Mi, L, false, n, n, n, 1.0, 0.0);            /* T = X */
-  mv(w.v1, a.Z, L, false, ej, n, n, 1.0, 0.0);
-  axpy(w.v1, a.b, n, 1.0);
-  mv(a.b, w.T, L, false, w.v1, n, n, 1.0, 0.0);
-  axpy(a.b, bj, n, 1.0);                                                     /* b */
-  mm<NB>(F, L, w.T, L, false, a.Z, L, false, n, n, n, 1.0, 0.0);             /* F = X Z_i */
+  mm<NB>(w.T2, L, w.W1, L, false, a.A, L, false, n, n, n, 1.0, 0.0);         /* T2 = J_j A_i */
+  {
+    double* const B[1] = {a.A};
+    chol_forward<NB, true, true>(a.Z, L, n, B, n, L, w.v, 1);                /* Z = L, A = L^{-1} A_i, v = L^{-1} b_i */
+  }
+  mv<NB>(w.v, a.Z, L, true, w.t0, n, n, 1.0, 1.0);                           /* v = L^{-1} b_i + L^T e_j */
+  mv<NB>(w.t0, w.W1, L, false, a.b, n, n, -1.0, 1.0);                        /* t0 = e_j - J_j b_i */
+  mv<NB>(w.v + NB, a.Z, L, true, w.t0, n, n, 1.0, 0.0);
+  mm<NB>(w.T, L, w.W1, L, false, a.Z, L, false, n, n, n, 1.0, 0.0);          /* T = J_j L */
+  mm<NB>(w.T, L, a.Z, L, true, w.T, L, false, n, n, n, 1.0, 0.0);
+  for (int i = threadIdx.x; i < n; i += AT<NB>) w.T[i * (L + 1)] += 1.0;     /* T = N (read after the next barrier) */
+  mm<NB>(w.T2, L, a.Z, L, true, w.T2, L, false, n, n, n, 1.0, 0.0);
+  mm<NB>(w.Aj, L, a.Z, L, true, w.Aj, L, true, n, n, n, 1.0, 0.0);           /* L^T A_j^T */
+  {
+    double* const B[3] = {a.A, w.T2, w.Aj};
+    chol_forward<NB, false, false>(w.T, L, n, B, n, L, w.v, 2);              /* Y_1, Y_2, Y_b, y_0, y_1 */
+  }
+  mv<NB>(a.b, w.Aj, L, true, w.v, n, n, 1.0, 0.0);
+  axpy<NB>(a.b, bj, n, 1.0);                                                 /* b */
+  mv<NB>(a.e, a.A, L, true, w.v + NB, n, n, 1.0, 1.0);                       /* e */
+  mm<NB>(a.J, L, a.A, L, true, w.T2, L, false, n, n, n, 1.0, 1.0);           /* J */
   if (!EARLY) rZ.load(el.Z + g * nn, n);
   rZ.store(a.Z, L, n, false);                                                /* Z = Z_j */
   __syncthreads();
-  mm<NB>(a.Z, L, F, L, false, w.R, L, true, n, n, n, 1.0, 1.0);              /* Z */
-  mm<NB>(a.A, L, w.T, L, false, a.A, L, false, n, n, n, 1.0, 0.0);           /* A */
+  mm<NB>(a.Z, L, w.Aj, L, true, w.Aj, L, false, n, n, n, 1.0, 1.0);          /* Z */
+  mm<NB>(a.A, L, w.Aj, L, true, a.A, L, false, n, n, n, 1.0, 0.0);           /* A */
 }
 
 /* a <- a (x) element g, smoothing; a is the running suffix and g the next
@@ -696,8 +835,8 @@ __device__ void smooth_combine(const Blk& a, const Work<NB>& w, const AsElems& e
   rE.store(w.W1, L, n, false);                                               /* W1 = E_j */
   __syncthreads();
   mm<NB>(a.A, L, w.W1, L, false, a.A, L, false, n, n, n, 1.0, 0.0);
-  mv(a.b, w.W1, L, false, a.b, n, n, 1.0, 0.0);
-  axpy(a.b, gj, n, 1.0);
+  mv<NB>(a.b, w.W1, L, false, a.b, n, n, 1.0, 0.0);
+  axpy<NB>(a.b, gj, n, 1.0);
   mm<NB>(w.T, L, w.W1, L, false, a.Z, L, false, n, n, n, 1.0, 0.0);
   rL.store(a.Z, L, n, false);
   __syncthreads();
@@ -716,7 +855,7 @@ __device__ void blk_load(const Blk& a, int ld, const AsElems& el, int64_t g, int
     r.load(el.J + g * nn, n);
     r.store(a.J, ld, n, false);
   }
-  for (int i = threadIdx.x; i < n; i += AT) {
+  for (int i = threadIdx.x; i < n; i += AT<NB>) {
     a.b[i] = el.b[g * n + i];
     if (filt) a.e[i] = el.e[g * n + i];
   }
@@ -726,7 +865,7 @@ __device__ void blk_load(const Blk& a, int ld, const AsElems& el, int64_t g, int
 template <int NB>
 __device__ void blk_store(const Blk& a, int ld, const AsElems& el, int64_t g, int n, bool filt) {
   const int64_t nn = (int64_t)n * n;
-  for (int idx = threadIdx.x; idx < NB * NB; idx += AT) {
+  for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
     const int i = idx % NB, j = idx / NB;
     if (i < n && j < n) {
       el.A[g * nn + i + j * n] = a.A[i + j * ld];
@@ -734,7 +873,7 @@ __device__ void blk_store(const Blk& a, int ld, const AsElems& el, int64_t g, in
       if (filt) el.J[g * nn + i + j * n] = a.J[i + j * ld];
     }
   }
-  for (int i = threadIdx.x; i < n; i += AT) {
+  for (int i = threadIdx.x; i < n; i += AT<NB>) {
     el.b[g * n + i] = a.b[i];
     if (filt) el.e[g * n + i] = a.e[i];
   }
@@ -746,8 +885,8 @@ template <int NB, bool FILT>
 struct ScanPlan {
   static constexpr int SZ = Ld<NB>::SZ;
   static constexpr int ACC = FILT ? 3 * SZ + 2 * NB : 2 * SZ + NB;
-  static constexpr int WORK = FILT ? 5 * SZ + 2 * NB : 2 * SZ;             /* M, W1, W2, R, T, v1, v2 | W1, T */
-  static constexpr bool WORK_GLOBAL = (ACC + WORK) * 8 + NB * 4 + 256 > LDS_BYTES;
+  static constexpr int WORK = FILT ? 4 * SZ + 3 * NB : 2 * SZ;             /* W1, T, T2, Aj, v, t0 | W1, T */
+  static constexpr bool WORK_GLOBAL = (ACC + WORK) * 8 > LDS_BYTES;
   static constexpr int LDS = ACC + (WORK_GLOBAL ? 0 : WORK);
 };
 
@@ -766,13 +905,12 @@ __device__ void scan_setup(double* lds, double* gwork, Blk& a, Work<NB>& w) {
   double* p = SP::WORK_GLOBAL ? gwork + (int64_t)blockIdx.x * SP::WORK : q;
   w.W1 = p; p += SZ;
   w.T = p; p += SZ;
-  w.M = w.W2 = w.R = w.v1 = w.v2 = nullptr;
+  w.T2 = w.Aj = w.v = w.t0 = nullptr;
   if (FILT) {
-    w.M = p; p += SZ;
-    w.W2 = p; p += SZ;
-    w.R = p; p += SZ;
-    w.v1 = p; p += NB;
-    w.v2 = p; p += NB;
+    w.T2 = p; p += SZ;
+    w.Aj = p; p += SZ;
+    w.v = p; p += 2 * NB;
+    w.t0 = p;
   }
 }
 
@@ -800,14 +938,12 @@ struct Chunk {
 
 /* pass 1: the total of every chunk */
 template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT) ka_scan_reduce(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
+__global__ void __launch_bounds__(AT<NB>) ka_scan_reduce(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
   using SP = ScanPlan<NB, FILT>;
   __shared__ double lds[SP::LDS];
-  __shared__ GJScratch<NB> gjs;
   Blk a;
   Work<NB> w;
   scan_setup<NB, FILT>(lds, gwork, a, w);
-  w.g = &gjs;
   const Chunk c = ch[blockIdx.x];
   blk_load<NB>(a, Ld<NB>::L, el, c.first, n, FILT);
   for (int i = 1; i < c.len; ++i) combine<NB, FILT>(a, w, el, c.first + (int64_t)i * c.dir, n);
@@ -817,15 +953,13 @@ __global__ void __launch_bounds__(AT) ka_scan_reduce(const Chunk* ch, AsElems el
 /* pass 2, one Hillis-Steele round over the chunk totals of every problem:
  * out[t] = in[t - d] (x) in[t] when rank >= d, else in[t]. */
 template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT) ka_scan_round(const Chunk* ch, AsElems in, AsElems out, int d, int n,
+__global__ void __launch_bounds__(AT<NB>) ka_scan_round(const Chunk* ch, AsElems in, AsElems out, int d, int n,
                                                     double* gwork) {
   using SP = ScanPlan<NB, FILT>;
   __shared__ double lds[SP::LDS];
-  __shared__ GJScratch<NB> gjs;
   Blk a;
   Work<NB> w;
   scan_setup<NB, FILT>(lds, gwork, a, w);
-  w.g = &gjs;
   const Chunk c = ch[blockIdx.x];
   if (c.rank >= d) {
     blk_load<NB>(a, Ld<NB>::L, in, c.tot - d, n, FILT);
@@ -839,14 +973,12 @@ __global__ void __launch_bounds__(AT) ka_scan_round(const Chunk* ch, AsElems in,
 /* pass 3: every prefix within a chunk, seeded with the inclusive total of
  * the chunk before it; results overwrite the elements in place. */
 template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT) ka_scan_down(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
+__global__ void __launch_bounds__(AT<NB>) ka_scan_down(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
   using SP = ScanPlan<NB, FILT>;
   __shared__ double lds[SP::LDS];
-  __shared__ GJScratch<NB> gjs;
   Blk a;
   Work<NB> w;
   scan_setup<NB, FILT>(lds, gwork, a, w);
-  w.g = &gjs;
   const Chunk c = ch[blockIdx.x];
   int i0 = 0;
   if (c.rank == 0) {
@@ -867,14 +999,15 @@ __global__ void __launch_bounds__(AT) ka_scan_down(const Chunk* ch, AsElems el, 
 /* ------------------------------------------------------------------------ */
 
 /* filtered (x, P) of steps p+1 .. k-1: (b, Z) of the filtering prefixes */
-__global__ void __launch_bounds__(AT) ka_filtered(const AsProb* probs, const int32_t* elem_prob, AsElems el,
+template <int NB>
+__global__ void __launch_bounds__(AT<NB>) ka_filtered(const AsProb* probs, const int32_t* elem_prob, AsElems el,
                                                   AsModel md, int n) {
   const int64_t g = blockIdx.x;
   const AsProb pr = probs[elem_prob[g]];
   const int64_t s = pr.s0 + (g - pr.e0) + pr.p + 1;
   const int64_t nn = (int64_t)n * n;
-  for (int idx = threadIdx.x; idx < n * n; idx += AT) md.Pf[s * nn + idx] = el.Z[g * nn + idx];
-  for (int i = threadIdx.x; i < n; i += AT) md.xf[s * n + i] = el.b[g * n + i];
+  for (int idx = threadIdx.x; idx < n * n; idx += AT<NB>) md.Pf[s * nn + idx] = el.Z[g * nn + idx];
+  for (int i = threadIdx.x; i < n; i += AT<NB>) md.xf[s * n + i] = el.b[g * n + i];
 }
 
 /*
@@ -886,13 +1019,11 @@ __global__ void __launch_bounds__(AT) ka_filtered(const AsProb* probs, const int
  *           L = (Lam + F^T Q^{-1} F)^{-1}, E = L F^T Q^{-1}, g = L (eta - F^T Q^{-1} c).
  */
 template <int NB>
-__global__ void __launch_bounds__(AT) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md, AsElems el,
+__global__ void __launch_bounds__(AT<NB>) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md, AsElems el,
                                                int n) {
   constexpr int L = Ld<NB>::L;
   __shared__ double M[Ld<NB>::SZ], T[Ld<NB>::SZ], U[Ld<NB>::SZ];
   __shared__ double v1[NB], v2[NB];
-  __shared__ int piv[NB];
-  __shared__ GJScratch<NB> g;
   const int64_t s = blockIdx.x;
   const AsProb pr = probs[step_prob[s]];
   const int64_t t = s - pr.s0;
@@ -901,11 +1032,11 @@ __global__ void __launch_bounds__(AT) ka_selem(const AsProb* probs, const int32_
   double* gv = el.b + s * n;
   double* Lo = el.Z + s * nn;
   if (t == pr.k - 1) {
-    for (int idx = threadIdx.x; idx < n * n; idx += AT) {
+    for (int idx = threadIdx.x; idx < n * n; idx += AT<NB>) {
       E[idx] = 0.0;
       Lo[idx] = md.Pf[s * nn + idx];
     }
-    for (int i = threadIdx.x; i < n; i += AT) gv[i] = md.xf[s * n + i];
+    for (int i = threadIdx.x; i < n; i += AT<NB>) gv[i] = md.xf[s * n + i];
     return;
   }
   const double* F = md.F + (s + 1) * nn;
@@ -916,52 +1047,48 @@ __global__ void __launch_bounds__(AT) ka_selem(const AsProb* probs, const int32_
     const double* x = md.xf + s * n;
     copy_mat<NB>(U, L, P, n, false, n, n);                                   /* U = P */
     copy_mat<NB>(M, L, F, n, false, n, n);                                   /* M = F */
-    mm<NB>(T, L, U, L, false, M, L, true, n, n, n, 1.0, 0.0);                /* T = P F^T */
-    mv(v1, M, L, false, x, n, n, 1.0, 0.0);
-    axpy(v1, c, n, 1.0);                                                     /* v1 = F x + c */
-    mm<NB>(U, L, M, L, false, T, L, false, n, n, n, 1.0, 0.0);               /* U = F P F^T */
-    copy_mat<NB>(M, L, Q, n, false, n, n);
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT) {
-      const int i = idx % NB, j = idx / NB;
-      if (i < n && j < n) M[i + j * L] += U[i + j * L];                      /* M = F P F^T + Q */
-    }
-    __syncthreads();
-    lu<NB>(M, L, n, piv, g);
-    copy_mat<NB>(U, L, T, L, true, n, n);                                    /* U = F P */
-    lu_solve(M, L, piv, n, U, L, n, true);                                   /* U = E^T */
-    copy_mat<NB>(E, n, U, L, true, n, n);
-    mv(gv, U, L, true, v1, n, n, -1.0, 0.0);
-    axpy(gv, x, n, 1.0);                                                     /* g = x - E (F x + c) */
-    copy_mat<NB>(M, L, T, L, true, n, n);                                    /* M = F P */
-    copy_mat<NB>(Lo, n, P, n, false, n, n);
-    mm<NB>(Lo, n, U, L, true, M, L, false, n, n, n, -1.0, 1.0);              /* L = P - E F P */
-  } else {
-    copy_mat<NB>(M, L, Q, n, false, n, n);
-    lu<NB>(M, L, n, piv, g);
-    copy_mat<NB>(T, L, F, n, false, n, n);
-    lu_solve(M, L, piv, n, T, L, n, false);                                  /* T = Q^{-1} F */
-    copy_vec(v1, c, n);
-    lu_solve(M, L, piv, n, v1, NB, 1, false);                                /* v1 = Q^{-1} c */
-    copy_mat<NB>(U, L, md.Lam + s * nn, n, false, n, n);
-    mm<NB>(U, L, F, n, true, T, L, false, n, n, n, 1.0, 1.0);                /* U = Lam + F^T Q^{-1} F */
-    lu<NB>(U, L, n, piv, g);
+    mm<NB>(T, L, M, L, false, U, L, false, n, n, n, 1.0, 0.0);               /* T = F P */
+    mv<NB>(v1, M, L, false, x, n, n, 1.0, 0.0);
+    axpy<NB>(v1, c, n, 1.0);                                                 /* v1 = F x + c */
+    copy_mat<NB>(U, L, Q, n, false, n, n);
+    mm<NB>(U, L, T, L, false, M, L, true, n, n, n, 1.0, 1.0);                /* U = F P F^T + Q = G G^T */
     set_identity<NB>(M, L, n, 1.0);
-    lu_solve(U, L, piv, n, M, L, n, false);                                  /* M = L */
-    copy_mat<NB>(Lo, n, M, L, false, n, n);
-    mm<NB>(E, n, M, L, false, T, L, true, n, n, n, 1.0, 0.0);                /* E = L (Q^{-1} F)^T */
-    mv(v2, F, n, true, v1, n, n, -1.0, 0.0);
-    axpy(v2, md.eta + s * n, n, 1.0);
-    mv(gv, M, L, false, v2, n, n, 1.0, 0.0);                                 /* g = L (eta - F^T Q^{-1} c) */
+    double* const B[2] = {T, M};
+    chol_forward<NB, false, false>(U, L, n, B, n, L, nullptr, 0);            /* T = Y = G^{-1} F P, M = G^{-1} */
+    mm<NB>(E, n, T, L, true, M, L, false, n, n, n, 1.0, 0.0);                /* E = Y^T G^{-1} */
+    mv<NB>(v2, M, L, false, v1, n, n, 1.0, 0.0);
+    mv<NB>(gv, T, L, true, v2, n, n, -1.0, 0.0);
+    axpy<NB>(gv, x, n, 1.0);                                                 /* g = x - E (F x + c) */
+    copy_mat<NB>(Lo, n, P, n, false, n, n);
+    mm<NB>(Lo, n, T, L, true, T, L, false, n, n, n, -1.0, 1.0);              /* L = P - Y^T Y */
+  } else {
+    copy_mat<NB>(U, L, Q, n, false, n, n);
+    copy_mat<NB>(T, L, F, n, false, n, n);
+    copy_vec<NB>(v1, c, n);
+    set_identity<NB>(M, L, n, 1.0);
+    double* const B[2] = {T, M};
+    chol_forward<NB, false, false>(U, L, n, B, n, L, v1, 1);                 /* Q = G G^T: T = Y = G^{-1} F, M = G^{-1}, v1 = G^{-1} c */
+    mm<NB>(M, L, M, L, true, T, L, false, n, n, n, 1.0, 0.0);                /* M = Q^{-1} F */
+    copy_mat<NB>(U, L, md.Lam + s * nn, n, false, n, n);
+    mm<NB>(U, L, T, L, true, T, L, false, n, n, n, 1.0, 1.0);                /* U = Lam + F^T Q^{-1} F */
+    mv<NB>(v2, T, L, true, v1, n, n, -1.0, 0.0);
+    axpy<NB>(v2, md.eta + s * n, n, 1.0);                                    /* v2 = eta - F^T Q^{-1} c */
+    chol_inverse_factor<NB>(U, T, L, n);
+    mm<NB>(T, L, T, L, true, T, L, false, n, n, n, 1.0, 0.0);                /* T = L */
+    copy_mat<NB>(Lo, n, T, L, false, n, n);
+    mm<NB>(E, n, T, L, false, M, L, true, n, n, n, 1.0, 0.0);                /* E = L (Q^{-1} F)^T */
+    mv<NB>(gv, T, L, false, v2, n, n, 1.0, 0.0);                             /* g = L (eta - F^T Q^{-1} c) */
   }
 }
 
 /* the smoothing prefix of step s (taken from the last step) is (E, g, L):
  * estimate g, covariance L */
-__global__ void __launch_bounds__(AT) ka_results(AsElems el, double* xout, double* Sout, int n) {
+template <int NB>
+__global__ void __launch_bounds__(AT<NB>) ka_results(AsElems el, double* xout, double* Sout, int n) {
   const int64_t s = blockIdx.x;
   const int64_t nn = (int64_t)n * n;
-  for (int idx = threadIdx.x; idx < n * n; idx += AT) Sout[s * nn + idx] = el.Z[s * nn + idx];
-  for (int i = threadIdx.x; i < n; i += AT) xout[s * n + i] = el.b[s * n + i];
+  for (int idx = threadIdx.x; idx < n * n; idx += AT<NB>) Sout[s * nn + idx] = el.Z[s * nn + idx];
+  for (int i = threadIdx.x; i < n; i += AT<NB>) xout[s * n + i] = el.b[s * n + i];
 }
 
 } /* namespace */
@@ -975,6 +1102,7 @@ extern "C" void uk_batch_view(ukhip_batch* b, const uk_raw_t** raw, double** xou
 extern "C" void uk_batch_set_assoc_ws(ukhip_batch* b, void* p, size_t bytes);
 extern "C" void uk_batch_chain0(ukhip_batch* b, uk_chain_t* ch, const int32_t** m0);
 extern "C" hipError_t uk_batch_weigh_dense0(ukhip_batch* b, hipStream_t st);
+extern "C" hipError_t uk_batch_weigh_level0(ukhip_batch* b, hipStream_t st);
 
 namespace {
 
@@ -1012,9 +1140,12 @@ int64_t make_chunks(std::vector<Chunk>& out, int64_t base, int64_t len, int dir,
   return nch;
 }
 
-/* chunk length: about CHUNKS_TARGET chunks over the batch (two workgroups per
- * compute unit at one workgroup per unit), at least 4 */
-constexpr int64_t CHUNKS_TARGET = 512;
+/* Chunks aimed at over a batch: as many as the filtering scan's workgroups
+ * that are resident at once (by its LDS: one per CU in buckets 48 and 64, two
+ * in 32, ten single waves in 16). More would only add to the rounds over the
+ * chunk totals. Chunks have at least 4 elements. */
+template <int NB>
+constexpr int64_t CHUNKS_TARGET = NB <= 16 ? 2560 : (NB <= 32 ? 512 : 256);
 
 template <int NB>
 int run_assoc(ukhip_batch* b) {
@@ -1061,8 +1192,8 @@ int run_assoc(ukhip_batch* b) {
     probs[p] = pr;
     s0 += pr.k;
   }
-  const int64_t fchunk = std::max<int64_t>(4, (ne + CHUNKS_TARGET - 1) / CHUNKS_TARGET);
-  const int64_t schunk = std::max<int64_t>(4, (S + CHUNKS_TARGET - 1) / CHUNKS_TARGET);
+  const int64_t fchunk = std::max<int64_t>(4, (ne + CHUNKS_TARGET<NB> - 1) / CHUNKS_TARGET<NB>);
+  const int64_t schunk = std::max<int64_t>(4, (S + CHUNKS_TARGET<NB> - 1) / CHUNKS_TARGET<NB>);
   std::vector<Chunk> fch, sch;
   int64_t ftot = 0, stot = 0, maxr_f = 0, maxr_s = 0;
   for (int p = 0; p < nprob; ++p) {
@@ -1142,7 +1273,7 @@ int run_assoc(ukhip_batch* b) {
   const Chunk* d_sch = (const Chunk*)put(sch.data(), sch.size() * sizeof(Chunk));
   if (!ok(hipMemcpyAsync(W + o_tab, tab.data(), to, hipMemcpyHostToDevice, st), "upload scan tables")) return -1;
 
-  const dim3 blk(AT);
+  const dim3 blk(AT<NB>);
   AsTimer* tm = t_timer;
   auto mark = [&](int slot, int launches) { /* slot's launches are done: its closing event */
     if (!tm) return;
@@ -1150,9 +1281,13 @@ int run_assoc(ukhip_batch* b) {
     (void)hipEventRecord(tm->ev[slot + 1], st);
   };
   if (tm) (void)hipEventRecord(tm->ev[0], st);
-  if (!ok(uk_batch_weigh_dense0(b, st), "k_weigh")) return -1;
+  /* with every K and C given as 'w' and H = I only the observations need
+   * whitening, and the model is the input's */
+  const bool diag = raw->H_ident && !raw->K_full && !raw->C_full && mr == raw->mr;
+  if (!ok(diag ? uk_batch_weigh_level0(b, st) : uk_batch_weigh_dense0(b, st), "k_weigh")) return -1;
   mark(UKHIP_AS_WEIGH, 1);
-  ka_model<NB><<<dim3((unsigned)S), blk, 0, st>>>(wch, raw->first, md, n);
+  if (diag) ka_model_diag<<<dim3((unsigned)S), dim3(256), 0, st>>>(*raw, md, n);
+  else ka_model<NB><<<dim3((unsigned)S), blk, 0, st>>>(wch, raw->first, md, n);
   mark(UKHIP_AS_MODEL, 1);
   ka_prior<NB><<<dim3((unsigned)nprob), blk, 0, st>>>(d_probs, wch, m_obs, md, n, mr);
   mark(UKHIP_AS_PRIOR, 1);
@@ -1169,7 +1304,7 @@ int run_assoc(ukhip_batch* b) {
     }
     ka_scan_down<NB, true><<<dim3(nc), blk, 0, st>>>(d_fch, fe, ft[cur], n, gw);
     mark(UKHIP_AS_FSCAN, 2 + rounds);
-    ka_filtered<<<dim3((unsigned)ne), blk, 0, st>>>(d_probs, d_elem_prob, fe, md, n);
+    ka_filtered<NB><<<dim3((unsigned)ne), blk, 0, st>>>(d_probs, d_elem_prob, fe, md, n);
     mark(UKHIP_AS_FILTERED, 1);
   } else {
     mark(UKHIP_AS_FELEM, 0);
@@ -1189,7 +1324,7 @@ int run_assoc(ukhip_batch* b) {
     }
     ka_scan_down<NB, false><<<dim3(nc), blk, 0, st>>>(d_sch, se, stt[cur], n, gw);
     mark(UKHIP_AS_SSCAN, 2 + rounds);
-    ka_results<<<dim3((unsigned)S), blk, 0, st>>>(se, xout, Sout, n);
+    ka_results<NB><<<dim3((unsigned)S), blk, 0, st>>>(se, xout, Sout, n);
     mark(UKHIP_AS_RESULTS, 1);
   }
   if (!ok(hipGetLastError(), "associative launches")) return -1;
@@ -1228,7 +1363,7 @@ extern "C" int uk_assoc_smooth(struct ukhip_batch* b, uint32_t options) {
   const int32_t* m0;
   uk_batch_chain0(b, &ch0, &m0);
   switch (uk_bucket(raw->n > ch0.mr ? raw->n : ch0.mr)) {
-    case 8: return run_assoc<8>(b);
+    case 8:
     case 16: return run_assoc<16>(b);
     case 32: return run_assoc<32>(b);
     case 48: return run_assoc<48>(b);

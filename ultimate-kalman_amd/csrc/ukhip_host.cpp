@@ -1886,6 +1886,14 @@ extern "C" hipError_t uk_batch_weigh_dense0(ukhip_batch* b, hipStream_t st) {
   return uk_launch_weigh(&b->raw, &b->chain[0], st);
 }
 
+/* whitens it as the odd-even path does: with every K and C given as 'w' and H =
+ * I, only C, o, c and D's diagonal are stored */
+extern "C" hipError_t uk_batch_weigh_level0(ukhip_batch* b, hipStream_t st) {
+  if (b->compress) return hipErrorInvalidValue;
+  const uk_chain_t w0 = level0_chain(b, b->chain[0]);
+  return uk_launch_weigh(&b->raw, &w0, st);
+}
+
 /* ------------------------------------------------------------------------ */
 /* the reference's smoother entry points (c/kalman.h:148-149)                */
 /* ------------------------------------------------------------------------ */
