@@ -21,11 +21,9 @@
  *                information form
  *   smoothing scan (same scheme, last step first) -> estimates, covariances
  *
- * Every element build and every combine runs in one workgroup (256 threads, one
- * wave for n <= 16). Its blocks live in LDS with the odd leading dimension NB +
- * 1; products run on the FP64 matrix cores straight from there. (The filtering
- * work blocks of the 64 bucket go to a per-workgroup global slice: seven 64 x
- * 65 blocks exceed the 160 KiB of LDS.)
+ * Every element build and every combine runs in one workgroup, on the FP64
+ * matrix cores, with the matrices in registers (see Geo): one wave for n <= 16,
+ * three to four waves above.
  * Wherever a symmetric positive definite matrix M is inverted in a formula, its
  * factor takes part instead: with M = G G^T, one forward elimination turns B
  * into G^{-1} B, and every result is a product of two such blocks
@@ -55,7 +53,6 @@ namespace {
 /* threads of the kernels of bucket NB */
 template <int NB>
 constexpr int AT = NB <= 16 ? 64 : 256;
-constexpr int LDS_BYTES = 160 * 1024; /* gfx950 LDS per workgroup */
 
 /* ------------------------------------------------------------------------ */
 /* workgroup-level dense algebra on blocks of order <= NB                    */
@@ -351,178 +348,303 @@ __device__ __forceinline__ double rsqrt_ulp(double p) {
   return fma(0.5 * y1, fma(-p * y1, y1, 1.0), y1);
 }
 
+/* ------------------------------------------------------------------------ */
+/* tile columns                                                              */
+/* ------------------------------------------------------------------------ */
+
 /*
- * Forward elimination with a symmetric positive definite M = G G^T (n x n, ld,
- * both triangles given): every block B[i] (n x q, ldb) and every vector (nv of
- * them at v, NB apart) becomes G^{-1} times itself. KEEP: M becomes G (lower
- * triangular, zeros above), else it is left half reduced.
- * Panels of 16: each wave factors the panel's diagonal tile in its registers
- * (the same work on every wave, instead of a barrier), takes T_r = G_pp^{-1}
- * M_pr for the block rows r below, and then 16 columns at a time of what is
- * dealt to it: T = G_pp^{-1} X_p, X_r -= T_r^T T. One barrier per panel.
+ * The layout of the element builds, the prior and the scans: a matrix of order
+ * n <= 16 NT is NT x NT tiles in the accumulator layout, wave w holds tile
+ * column w in NT registers quads, and vectors are a tile column too (on a wave
+ * of their own for NT = 2 and 3; on wave 0 next to its matrix columns for NT =
+ * 1 and for NT = 4, where a fifth wave would halve the registers of all).
+ * All products have the form Y = P^T X (tmul): X and Y stay in the registers
+ * of their waves and only P goes through LDS, where a tile is stored as it
+ * lies in the lanes (for NT = 1 it does not leave the registers, and the kernel
+ * uses no LDS and no barrier). Rows and columns from n on are zeros.
+ * Against blocks of whole workgroups in LDS (products and eliminations on the
+ * matrix cores as here) a filtering combine takes 41 us instead of 72 at n = 48,
+ * with two workgroups on a CU instead of one, and 12 us instead of 25 for n <=
+ * 16, launch included.
+ */
+template <int NT>
+struct Geo {
+  static constexpr bool SEP = NT == 2 || NT == 3; /* the vectors have a wave of their own */
+  static constexpr int WAVES = NT + (SEP ? 1 : 0);
+  static constexpr int THREADS = 64 * WAVES;
+};
+template <int NT>
+struct Who { /* of this lane */
+  int li, lk, lane, w;
+  bool mat, vec;
+  __device__ Who() {
+    lane = threadIdx.x & 63;
+    li = lane & 15;
+    lk = lane >> 4;
+    w = NT == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    mat = !Geo<NT>::SEP || w < NT;
+    vec = w == (Geo<NT>::SEP ? NT : 0);
+  }
+};
+template <int NT>
+__device__ __forceinline__ void sync() {
+  if (NT > 1) __syncthreads();
+}
+
+/* a matrix shared by the waves: tile (r, c) as it lies in the lanes */
+template <int NT>
+struct Sh {
+  double* p;
+  __device__ __forceinline__ void put(const as_d4 (&X)[NT], const Who<NT>& me) {
+    if (!me.mat) return;
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) p[((me.w * NT + r) * 4 + g) * 64 + me.lane] = X[r][g];
+  }
+  /* the transpose of an upper triangular matrix */
+  __device__ __forceinline__ void put_upper_t(const as_d4 (&X)[NT], const Who<NT>& me) {
+    if (!me.mat) return;
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+      if (r <= me.w) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) p[(r * NT + me.w) * 256 + me.li * 16 + 4 * g + me.lk] = X[r][g];
+      }
+  }
+  __device__ __forceinline__ as_d4 tile(int r, int c, const Who<NT>& me) const {
+    as_d4 t;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) t[g] = p[((c * NT + r) * 4 + g) * 64 + me.lane];
+    return t;
+  }
+};
+template <>
+struct Sh<1> {
+  as_d4 v;
+  __device__ __forceinline__ void put(const as_d4 (&X)[1], const Who<1>&) { v = X[0]; }
+  __device__ __forceinline__ void put_upper_t(const as_d4 (&X)[1], const Who<1>& me) { /* the product with I is exact */
+    as_d4 y = as_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int g = 0; g < 4; ++g) y = as_mfma(X[0][g], 4 * g + me.lk == me.li ? 1.0 : 0.0, y);
+    v = y;
+  }
+  __device__ __forceinline__ as_d4 tile(int, int, const Who<1>&) const { return v; }
+};
+template <int NT>
+struct Lds {
+  double b0[NT * NT * 256], b1[NT * NT * 256], wt[256], tr[NT * 256];
+};
+template <>
+struct Lds<1> {
+  double b0[1], b1[1], wt[1], tr[1];
+};
+template <int NT>
+__device__ __forceinline__ Sh<NT> sh(double* p) {
+  Sh<NT> s;
+  if constexpr (NT > 1) s.p = p;
+  return s;
+}
+
+/* Lets the matrix products before it finish. The compiler places the wait
+ * states between a product and the first read of its result, but it counts
+ * them along one of the paths that lead there: where products are under a
+ * condition, another path can be too short, and the read gets the sum without
+ * its last term. So code with conditions on products ends with this. */
+__device__ __forceinline__ void mfma_drain() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 15\n\ts_nop 3");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+/* Y += SGN P^T X over the first kk rows of P and X; LOWER: P is lower
+ * triangular; rlo: X starts at tile row rlo; ihi: the last row of Y wanted */
+template <int NT, int SGN = 1, bool LOWER = false>
+__device__ __forceinline__ void tmul(const Sh<NT>& P, const as_d4 (&X)[NT], as_d4 (&Y)[NT], int kk, const Who<NT>& me,
+                                     int rlo = 0, int ihi = NT - 1) {
+#pragma unroll
+  for (int r = 0; r < NT; ++r) {
+    if (16 * r < kk && r >= rlo) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if ((!LOWER || r >= i) && i <= ihi) {
+          const as_d4 p = P.tile(r, i, me);
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (NT > 1 || 4 * g < kk) Y[i] = as_mfma(SGN < 0 ? -p[g] : p[g], X[r][g], Y[i]);
+        }
+      }
+    }
+  }
+  mfma_drain();
+}
+template <int NT>
+__device__ __forceinline__ void zero(as_d4 (&X)[NT]) {
+#pragma unroll
+  for (int r = 0; r < NT; ++r) X[r] = as_d4{0.0, 0.0, 0.0, 0.0};
+}
+/* X += 1 on the diagonal from row `lo` to below row `hi` */
+template <int NT>
+__device__ __forceinline__ void add_diag(as_d4 (&X)[NT], int lo, int hi, const Who<NT>& me) {
+  const int col = 16 * me.w + me.li;
+#pragma unroll
+  for (int r = 0; r < NT; ++r) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) X[r][g] += 16 * r + 4 * g + me.lk == col && col >= lo && col < hi ? 1.0 : 0.0;
+  }
+}
+/* this wave's column of G (rows x cols, ld); T: of its transpose, whose loads
+ * are the contiguous ones (taken for symmetric matrices too) */
+template <int NT, bool T>
+__device__ __forceinline__ void load(as_d4 (&X)[NT], const double* G, int rows, int cols, int ld, const Who<NT>& me) {
+  const int col = 16 * me.w + me.li, lr = T ? cols : rows, lc = T ? rows : cols;
+  double v[NT][4];
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 16 * r + 4 * g + me.lk;
+      v[r][g] = G[row < lr && col < lc ? (T ? col + row * ld : row + col * ld) : 0];
+    }
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 16 * r + 4 * g + me.lk;
+      X[r][g] = row < lr && col < lc ? v[r][g] : 0.0;
+    }
+}
+template <int NT, bool T>
+__device__ __forceinline__ void store(const as_d4 (&X)[NT], double* G, int n, const Who<NT>& me) {
+  const int col = 16 * me.w + me.li;
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 16 * r + 4 * g + me.lk;
+      if (row < n && col < n) G[T ? col + row * n : row + col * n] = X[r][g];
+    }
+}
+/* a vector, the same in every column of its tiles */
+template <int NT>
+__device__ __forceinline__ void load_vec(as_d4 (&X)[NT], const double* v, int n, const Who<NT>& me) {
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 16 * r + 4 * g + me.lk;
+      const double x = v[row < n ? row : 0];
+      X[r][g] = row < n ? x : 0.0;
+    }
+}
+template <int NT>
+__device__ __forceinline__ void store_vec(const as_d4 (&X)[NT], double* v, int n, const Who<NT>& me) {
+  if (me.li != 0) return;
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int row = 16 * r + 4 * g + me.lk;
+      if (row < n) v[row] = X[r][g];
+    }
+}
+/* column K of the tiles in all columns */
+template <int K, int NT>
+__device__ __forceinline__ void spread(as_d4 (&X)[NT]) {
+#pragma unroll
+  for (int r = 0; r < NT; ++r)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) X[r][g] = row_lane<K>(X[r][g]);
+}
+
+/* row tile p of X through G_pp^{-1}, whose transpose is wt */
+template <int NT>
+__device__ __forceinline__ void panel_solve(as_d4& x, const as_d4& wt) {
+  as_d4 y = as_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int g = 0; g < 4; ++g) y = as_mfma(wt[g], x[g], y);
+  x = y;
+}
+
+/*
+ * Forward elimination with a symmetric positive definite M = G G^T (tile rows
+ * <= w of column w are used): M becomes G^T (rows <= w) and every R becomes
+ * G^{-1} R; R1 of all waves, the others of those that hold matrix columns.
+ * Rows of M from lim on are the identity's. Wave p factors diagonal tile p in its
+ * registers and hands out the inverse of its factor, the waves solve row tile
+ * p, hand out M's, and update the rows below: two barriers a panel.
  * A pivoted Gauss-Jordan inverse in LDS, one barrier per column, took this
  * place: 138 us a filtering combine at n = 48 with it.
  */
-template <int NB, bool KEEP, bool FLOOR, int NBLK>
-__device__ void chol_forward(double* M, int ld, int n, double* const (&B)[NBLK], int q, int ldb, double* v, int nv) {
-  constexpr int TB = (NB + 15) / 16, NW = AT<NB> / 64;
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int tn = (n + 15) >> 4, tq = (q + 15) >> 4;
-  double diag[TB];
+template <int NT, bool FLOOR, class... R>
+__device__ __forceinline__ void chol_forward(Lds<NT>& s, as_d4 (&M)[NT], int lim, const Who<NT>& me, as_d4 (&R1)[NT],
+                                             R&... Rs) {
+  double fl = 0.0;
   if (FLOOR) {
 #pragma unroll
-    for (int p = 0; p < TB; ++p) diag[p] = 16 * p + li < n ? fmax(2.2e-16 * M[(16 * p + li) * (ld + 1)], 1e-290) : 0.0;
-    __syncthreads();
+    for (int i = 0; i < NT; ++i)
+      if (me.w == i) {
+        double d = 0.0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) d = 4 * g + me.lk == me.li ? M[i][g] : d;
+        fl = fmax(2.2e-16 * rows_sum(d), 1e-290);
+      }
   }
-#pragma unroll 1
-  for (int p = 0; p < tn; ++p) {
-    const int p0 = 16 * p;
-    double a[4], wt[4], pr[4], pc = 1.0, fl = 0.0;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int r = 4 * g + lk;
-      const bool in = p0 + r < n && p0 + li < n;
-      const double x = M[in ? p0 + r + (p0 + li) * ld : 0];
-      a[g] = in ? x : (r == li ? 1.0 : 0.0);
-      wt[g] = r == li ? 1.0 : 0.0;
-      pr[g] = 1.0;
-    }
-    if (FLOOR) {
-#pragma unroll
-      for (int i = 0; i < TB; ++i) fl = p == i ? diag[i] : fl;
-    }
-    chol_steps<FLOOR>(a, wt, pr, pc, fl, n - p0, li, lk, std::make_integer_sequence<int, 16>{});
-    const double sc = rsqrt_ulp(pc);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) wt[g] *= sc; /* G_pp^{-T}: A operand of G_pp^{-1} */
-    auto row_tile = [&](const double* X, int ldx, int cols, double (&t)[4]) { /* t = G_pp^{-1} X_p, 16 columns at X */
-      double b[4];
+  for (int p = 0; p < NT; ++p) {
+    as_d4 wt;
+    if (me.w == p) {
+      double a[4], t[4], pr[4], pc = 1.0;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int r = p0 + 4 * g + lk;
-        const bool in = r < n && li < cols;
-        const double x = X[in ? r + (int64_t)li * ldx : 0];
-        b[g] = in ? x : 0.0;
+        a[g] = M[p][g];
+        t[g] = 4 * g + me.lk == me.li ? 1.0 : 0.0;
+        pr[g] = 1.0;
       }
-      as_d4 acc = as_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int g = 0; g < 4; ++g) acc = as_mfma(wt[g], b[g], acc);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) t[g] = acc[g];
-    };
-    double tr[TB > 1 ? TB - 1 : 1][4];
-#pragma unroll
-    for (int i = 0; i < TB - 1; ++i)
-      if (p + 1 + i < tn) row_tile(M + (p0 + 16 * (1 + i)) * ld, ld, n - (p0 + 16 * (1 + i)), tr[i]);
-    const int trail = tn - 1 - p, tot = trail + NBLK * tq + (nv > 0 ? 1 : 0);
-    for (int t = w; t < tot; t += NW) {
-      double* X;
-      int ldx, cols;
-      if (t < trail) {
-        X = M + (p0 + 16 * (1 + t)) * ld;
-        ldx = ld;
-        cols = n - (p0 + 16 * (1 + t));
-      } else if (t < trail + NBLK * tq) {
-        const int u = t - trail, blk = u / tq, c0 = 16 * (u - blk * tq);
-        double* Bb = B[0];
-#pragma unroll
-        for (int i = 1; i < NBLK; ++i) Bb = blk == i ? B[i] : Bb;
-        X = Bb + (int64_t)c0 * ldb;
-        ldx = ldb;
-        cols = q - c0;
-      } else {
-        X = v;
-        ldx = NB;
-        cols = nv;
-      }
-      double tc[4];
-      row_tile(X, ldx, cols, tc);
-      if (t >= trail && li < cols) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          if (p0 + 4 * g + lk < n) X[p0 + 4 * g + lk + (int64_t)li * ldx] = tc[g];
-      }
-#pragma unroll
-      for (int i = 0; i < TB - 1; ++i) {
-        const int r0 = p0 + 16 * (1 + i);
-        if (r0 < n) {
-          as_d4 acc;
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const bool in = r0 + 4 * g + lk < n && li < cols;
-            const double x = X[in ? r0 + 4 * g + lk + (int64_t)li * ldx : 0];
-            acc[g] = in ? x : 0.0;
-          }
-#pragma unroll
-          for (int g = 0; g < 4; ++g) acc = as_mfma(-tr[i][g], tc[g], acc);
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            if (r0 + 4 * g + lk < n && li < cols) X[r0 + 4 * g + lk + (int64_t)li * ldx] = acc[g];
-        }
-      }
-    }
-    if (KEEP) { /* G_rp = T_r^T, below the diagonal, where this panel reads nothing */
-#pragma unroll
-      for (int i = 0; i < TB - 1; ++i) {
-        const int r = p0 + 16 * (1 + i) + li;
-        if (i % NW == w && r < n) {
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            if (p0 + 4 * g + lk < n) M[r + (p0 + 4 * g + lk) * ld] = tr[i][g];
-        }
-      }
-    }
-    __syncthreads();
-    if (KEEP && w == 0) { /* G_pp = (D^{-1/2} a)^T; no later panel reads this block */
+      chol_steps<FLOOR>(a, t, pr, pc, fl, lim - 16 * p, me.li, me.lk, std::make_integer_sequence<int, 16>{});
+      const double sc = rsqrt_ulp(pc);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int k = 4 * g + lk;
-        if (p0 + k < n && p0 + li < n) M[p0 + li + (p0 + k) * ld] = li >= k ? a[g] * rsqrt_ulp(pr[g]) : 0.0;
+        wt[g] = t[g] * sc;
+        M[p][g] = me.li >= 4 * g + me.lk ? a[g] * rsqrt_ulp(pr[g]) : 0.0;
+        if (NT > 1) s.wt[g * 64 + me.lane] = wt[g];
+      }
+    }
+    if (NT > 1) {
+      sync<NT>();
+#pragma unroll
+      for (int g = 0; g < 4; ++g) wt[g] = s.wt[g * 64 + me.lane];
+    }
+    panel_solve<NT>(R1[p], wt);
+    if (me.mat) (panel_solve<NT>(Rs[p], wt), ...);
+    mfma_drain();
+    if (p + 1 < NT) {
+      if (me.mat && me.w > p) {
+        panel_solve<NT>(M[p], wt);
+        mfma_drain();
+#pragma unroll
+        for (int g = 0; g < 4; ++g) s.tr[(me.w * 4 + g) * 64 + me.lane] = M[p][g];
+      }
+      sync<NT>();
+#pragma unroll
+      for (int r = p + 1; r < NT; ++r) {
+        as_d4 t;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) t[g] = -s.tr[(r * 4 + g) * 64 + me.lane];
+        auto update = [&](as_d4(&X)[NT]) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) X[r] = as_mfma(t[g], X[p][g], X[r]);
+        };
+        update(R1);
+        if (me.mat) {
+          (update(Rs), ...);
+          if (me.w >= r) update(M);
+        }
+        mfma_drain();
       }
     }
   }
-  if (KEEP) {
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
-      const int i = idx % NB, j = idx / NB;
-      if (i < n && j < n && (i >> 4) < (j >> 4)) M[i + j * ld] = 0.0;
-    }
-    __syncthreads();
-  }
 }
-
-/* W (ld) <- G^{-1} of M = G G^T (M is consumed); M^{-1} = W^T W */
-template <int NB>
-__device__ void chol_inverse_factor(double* M, double* W, int ld, int n) {
-  set_identity<NB>(W, ld, n, 1.0);
-  double* const B[1] = {W};
-  chol_forward<NB, false, false>(M, ld, n, B, n, ld, nullptr, 0);
-}
-
-/* Per-thread registers holding an n x n global block (ld n) distributed over
- * the NB x NB grid: entry idx = threadIdx.x + u * AT<NB>. */
-template <int NB>
-struct RegBlk {
-  static constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
-  double v[PER];
-  __device__ void load(const double* G, int n) {
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int idx = (int)threadIdx.x + u * AT<NB>;
-      const int i = idx % NB, j = idx / NB;
-      v[u] = (idx < NB * NB && i < n && j < n) ? G[i + (int64_t)j * n] : 0.0;
-    }
-  }
-  /* D (ld) <- the block, or its transpose; no barrier */
-  __device__ void store(double* D, int ld, int n, bool t) const {
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int idx = (int)threadIdx.x + u * AT<NB>;
-      const int i = idx % NB, j = idx / NB;
-      if (idx < NB * NB && i < n && j < n) D[t ? j + i * ld : i + j * ld] = v[u];
-    }
-  }
-};
 
 /* ------------------------------------------------------------------------ */
 /* batch data                                                                */
@@ -602,60 +724,98 @@ __global__ void __launch_bounds__(256) ka_model_diag(uk_raw_t raw, AsModel md, i
 /* prior: information filter over steps 0..p, one workgroup per problem      */
 /* ------------------------------------------------------------------------ */
 
-template <int NB>
-__global__ void __launch_bounds__(AT<NB>) ka_prior(const AsProb* probs, uk_chain_t wch, const int32_t* m_obs, AsModel md,
-                                                   int n, int mr) {
-  constexpr int L = Ld<NB>::L;
-  __shared__ double Lm[Ld<NB>::SZ], Mx[Ld<NB>::SZ], Qi[Ld<NB>::SZ], T2[Ld<NB>::SZ];
-  __shared__ double et[NB], v1[NB], v2[NB];
+template <int NT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS) ka_prior(const AsProb* probs, uk_chain_t wch, const int32_t* m_obs,
+                                                             AsModel md, int n, int mr) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Sh<NT> b0 = sh<NT>(s.b0), b1 = sh<NT>(s.b1);
   const AsProb pr = probs[blockIdx.x];
   const int64_t nn = (int64_t)n * n;
-  set_identity<NB>(Lm, L, n, 0.0);
-  for (int i = threadIdx.x; i < n; i += AT<NB>) et[i] = 0.0;
-  __syncthreads();
+  as_d4 Lm[NT], et[NT]; /* information matrix; vector (vector waves) */
+  zero<NT>(Lm);
+  zero<NT>(et);
   for (int64_t t = 0; t <= pr.p; ++t) {
-    const int64_t s = pr.s0 + t;
+    const int64_t st = pr.s0 + t;
     if (t > 0) {
-      /* predict: with Mx = Lam + F^T Q^{-1} F = G G^T and r = eta - F^T Q^{-1} c,
-       * Lam <- Q^{-1} - Y^T Y, eta <- Q^{-1} c + Y^T y,
-       * Y = G^{-1} F^T Q^{-1}, y = G^{-1} r */
-      const double* F = md.F + s * nn;
-      copy_mat<NB>(Mx, L, md.Q + s * nn, n, false, n, n);
-      chol_inverse_factor<NB>(Mx, Qi, L, n);
-      mm<NB>(Qi, L, Qi, L, true, Qi, L, false, n, n, n, 1.0, 0.0);            /* Qi = Q^{-1} */
-      mm<NB>(T2, L, Qi, L, false, F, n, false, n, n, n, 1.0, 0.0);            /* T2 = Q^{-1} F */
-      copy_mat<NB>(Mx, L, Lm, L, false, n, n);
-      mm<NB>(Mx, L, F, n, true, T2, L, false, n, n, n, 1.0, 1.0);             /* Mx = Lam + F^T T2 */
-      mv<NB>(v1, Qi, L, false, md.c + s * n, n, n, 1.0, 0.0);                /* v1 = Q^{-1} c */
-      mv<NB>(v2, F, n, true, v1, n, n, -1.0, 0.0);
-      axpy<NB>(v2, et, n, 1.0);                                              /* v2 = r */
-      copy_mat<NB>(Lm, L, T2, L, true, n, n);                                /* Lm = T2^T */
-      double* const B[1] = {Lm};
-      chol_forward<NB, false, false>(Mx, L, n, B, n, L, v2, 1);              /* Lm = Y, v2 = y */
-      mm<NB>(Qi, L, Lm, L, true, Lm, L, false, n, n, n, -1.0, 1.0);           /* Lam- */
-      mv<NB>(et, Lm, L, true, v2, n, n, 1.0, 0.0);
-      axpy<NB>(et, v1, n, 1.0);                                              /* eta- */
-      copy_mat<NB>(Lm, L, Qi, L, false, n, n);
+      /* predict: with Q = G G^T, W = G^{-1}, Y = W F, y = W c and Lam + Y^T Y =
+       * H H^T, V = H^{-1} Y^T W, v = H^{-1} (eta - Y^T y):
+       * Lam <- W^T W - V^T V, eta <- W^T y + V^T v */
+      as_d4 M[NT], Y[NT], W[NT], y[NT], D[NT];
+      load<NT, true>(M, md.Q + st * nn, n, n, n, me);
+      add_diag<NT>(M, n, 16 * NT, me);
+      load<NT, false>(Y, md.F + st * nn, n, n, n, me);
+      zero<NT>(W);
+      add_diag<NT>(W, 0, n, me);
+      load_vec<NT>(y, md.c + st * n, n, me);
+      chol_forward<NT, false>(s, M, n, me, y, Y, W);
+      b0.put(Y, me);
+      b1.put(W, me);
+      sync<NT>();
+      zero<NT>(D);
+      if (me.mat) {
+        tmul<NT>(b0, W, D, n, me); /* Y^T W */
+        tmul<NT>(b0, Y, Lm, n, me);
+        zero<NT>(M);
+        tmul<NT>(b1, W, M, n, me); /* Q^{-1} */
+      }
+      as_d4 ey[NT];
+      zero<NT>(ey);
+      if (me.vec) {
+        tmul<NT, -1>(b0, y, et, n, me);
+        tmul<NT>(b1, y, ey, n, me);
+      }
+      add_diag<NT>(Lm, n, 16 * NT, me);
+      chol_forward<NT, false>(s, Lm, n, me, et, D);
+      b0.put(D, me);
+      sync<NT>();
+      if (me.mat) {
+        tmul<NT, -1>(b0, D, M, n, me);
+#pragma unroll
+        for (int r = 0; r < NT; ++r) Lm[r] = M[r];
+      }
+      if (me.vec) {
+        tmul<NT>(b0, et, ey, n, me);
+#pragma unroll
+        for (int r = 0; r < NT; ++r) et[r] = ey[r];
+      }
+      sync<NT>();
     }
-    const int m = m_obs[s];
+    const int m = m_obs[st];
     if (m > 0) { /* update: Lam += C^T C, eta += C^T o (whitened) */
-      const double* Cw = wch.C + s * nn;
-      mm<NB>(Lm, L, Cw, mr, true, Cw, mr, false, n, n, m, 1.0, 1.0);
-      mv<NB>(et, Cw, mr, true, wch.o + s * n, n, m, 1.0, 1.0);
+      as_d4 C[NT], o[NT];
+      load<NT, false>(C, wch.C + st * nn, m, n, mr, me);
+      load_vec<NT>(o, wch.o + st * n, m, me);
+      b0.put(C, me);
+      sync<NT>();
+      if (me.mat) tmul<NT>(b0, C, Lm, m, me);
+      if (me.vec) tmul<NT>(b0, o, et, m, me);
+      sync<NT>();
     }
     if (t < pr.p) {
-      copy_mat<NB>(md.Lam + s * nn, n, Lm, L, false, n, n);
-      for (int i = threadIdx.x; i < n; i += AT<NB>) md.eta[s * n + i] = et[i];
-      __syncthreads();
+      if (me.mat) store<NT, true>(Lm, md.Lam + st * nn, n, me);
+      if (me.vec) store_vec<NT>(et, md.eta + st * n, n, me);
     }
   }
-  /* P_p = Lam^{-1}, x_p = P_p eta */
+  /* P_p = Lam^{-1} = W^T W, x_p = P_p eta = W^T (W eta) */
   const int64_t sp = pr.s0 + pr.p;
-  copy_mat<NB>(Mx, L, Lm, L, false, n, n);
-  chol_inverse_factor<NB>(Mx, Qi, L, n);
-  mm<NB>(Qi, L, Qi, L, true, Qi, L, false, n, n, n, 1.0, 0.0);
-  copy_mat<NB>(md.Pf + sp * nn, n, Qi, L, false, n, n);
-  mv<NB>(md.xf + sp * n, Qi, L, false, et, n, n, 1.0, 0.0);
+  as_d4 W[NT], P[NT], x[NT];
+  zero<NT>(W);
+  add_diag<NT>(W, 0, n, me);
+  add_diag<NT>(Lm, n, 16 * NT, me);
+  chol_forward<NT, false>(s, Lm, n, me, et, W);
+  b0.put(W, me);
+  sync<NT>();
+  if (me.mat) {
+    zero<NT>(P);
+    tmul<NT>(b0, W, P, n, me);
+    store<NT, true>(P, md.Pf + sp * nn, n, me);
+  }
+  if (me.vec) {
+    zero<NT>(x);
+    tmul<NT>(b0, et, x, n, me);
+    store_vec<NT>(x, md.xf + sp * n, n, me);
+  }
 }
 
 /* ------------------------------------------------------------------------ */
@@ -672,94 +832,117 @@ __global__ void __launch_bounds__(AT<NB>) ka_prior(const AsProb* probs, uk_chain
  * Unobserved: A = F (0 if first), b = c
  * (m1 if first), Z = Q (Q1), e = 0, J = 0.
  */
-template <int NB>
-__global__ void __launch_bounds__(AT<NB>) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
-                                               const int32_t* m_obs, AsModel md, AsElems el, int n, int mr) {
-  constexpr int L = Ld<NB>::L;
-  __shared__ double Qs[Ld<NB>::SZ], CQ[Ld<NB>::SZ], S[Ld<NB>::SZ], T[Ld<NB>::SZ];
-  __shared__ double w1[NB], rr[2 * NB];
-  double *const r = rr, *const rc = rr + NB;
+template <int NT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
+                                                             const int32_t* m_obs, AsModel md, AsElems el, int n, int mr) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Sh<NT> b0 = sh<NT>(s.b0), b1 = sh<NT>(s.b1);
   const int64_t ge = blockIdx.x;
   const AsProb pr = probs[elem_prob[ge]];
   const int64_t t = ge - pr.e0 + pr.p + 1;
-  const int64_t s = pr.s0 + t;
+  const int64_t st = pr.s0 + t;
   const bool firstel = t == pr.p + 1;
   const int64_t nn = (int64_t)n * n;
-  const double* F = md.F + s * nn;
-  const double* c = md.c + s * n;
-  double* A = el.A + ge * nn;
-  double* b = el.b + ge * n;
-  double* Z = el.Z + ge * nn;
-  double* e = el.e + ge * n;
-  double* J = el.J + ge * nn;
   const int64_t spv = pr.s0 + pr.p;
+  const int m = m_obs[st];
 
-  copy_mat<NB>(Qs, L, md.Q + s * nn, n, false, n, n);                       /* Qs = Q */
-  copy_vec<NB>(w1, c, n);
+  as_d4 Q[NT], F[NT], c[NT], w1[NT];
+  load<NT, true>(Q, md.Q + st * nn, n, n, n, me);
+  load<NT, false>(F, md.F + st * nn, n, n, n, me);
+  load_vec<NT>(c, md.c + st * n, n, me);
+#pragma unroll
+  for (int r = 0; r < NT; ++r) w1[r] = c[r];
   if (firstel) { /* Q1 = Q + F P F^T, m1 = F x + c */
-    mm<NB>(T, L, F, n, false, md.Pf + spv * nn, n, false, n, n, n, 1.0, 0.0);
-    mm<NB>(Qs, L, T, L, false, F, n, true, n, n, n, 1.0, 1.0);
-    mv<NB>(w1, F, n, false, md.xf + spv * n, n, n, 1.0, 1.0);
-  }
-  const int m = m_obs[s];
-  if (m == 0) {
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
-      const int i = idx % NB, j = idx / NB;
-      if (i < n && j < n) {
-        A[i + j * n] = firstel ? 0.0 : F[i + j * n];
-        Z[i + j * n] = Qs[i + j * L];
-        J[i + j * n] = 0.0;
-      }
+    as_d4 Ft[NT], P[NT], x[NT], U[NT];
+    load<NT, true>(Ft, md.F + st * nn, n, n, n, me);
+    load<NT, true>(P, md.Pf + spv * nn, n, n, n, me);
+    load_vec<NT>(x, md.xf + spv * n, n, me);
+    b0.put(Ft, me);
+    b1.put(P, me);
+    sync<NT>();
+    if (me.mat) {
+      zero<NT>(U);
+      tmul<NT>(b1, Ft, U, n, me);
+      tmul<NT>(b0, U, Q, n, me);
     }
-    for (int i = threadIdx.x; i < n; i += AT<NB>) {
-      b[i] = w1[i];
-      e[i] = 0.0;
-    }
-    return;
+    if (me.vec) tmul<NT>(b0, x, w1, n, me);
+    sync<NT>();
   }
-  const double* ow = wch.o + s * n;
-  copy_mat<NB>(T, L, wch.C + s * nn, mr, false, m, n);                       /* T = C (m x n) */
-  mm<NB>(CQ, L, T, L, false, Qs, L, false, m, n, n, 1.0, 0.0);               /* CQ = C Q */
-  set_identity<NB>(S, L, m, 1.0);
-  mm<NB>(S, L, CQ, L, false, T, L, true, m, m, n, 1.0, 1.0);                 /* S = C Q C^T + I */
-  mv<NB>(r, T, L, false, w1, m, n, -1.0, 0.0);
-  axpy<NB>(r, ow, m, 1.0);                                                       /* r = o - C w1 */
-  mv<NB>(rc, T, L, false, c, m, n, -1.0, 0.0);
-  axpy<NB>(rc, ow, m, 1.0);                                                      /* rc = o - C c */
-  copy_mat<NB>(Z, n, Qs, L, false, n, n);                                    /* Z = Q (Qs is free now) */
-  mm<NB>(Qs, L, T, L, false, F, n, false, m, n, n, 1.0, 0.0);                /* Qs = C F */
-  double* const B[2] = {CQ, Qs};
-  chol_forward<NB, false, false>(S, L, m, B, n, L, rr, 2);                   /* CQ = Y_1, Qs = Y_2, r, rc = G^{-1} of them */
-  mv<NB>(b, CQ, L, true, r, n, m, 1.0, 0.0);
-  axpy<NB>(b, w1, n, 1.0);                                                   /* b = w1 + Y_1^T r */
-  mm<NB>(Z, n, CQ, L, true, CQ, L, false, n, n, m, -1.0, 1.0);               /* Z = Q - Y_1^T Y_1 */
-  if (firstel) {
-    for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
-      const int i = idx % NB, j = idx / NB;
-      if (i < n && j < n) A[i + j * n] = 0.0;
+  as_d4 J[NT], e[NT];
+  zero<NT>(J);
+  zero<NT>(e);
+  if (m > 0) {
+    as_d4 Ct[NT], S[NT], CQ[NT], CF[NT], y[NT];
+    load<NT, true>(Ct, wch.C + st * nn, m, n, mr, me);
+    load_vec<NT>(y, wch.o + st * n, m, me);
+    b0.put(Ct, me);
+    b1.put(Q, me);
+    sync<NT>();
+    zero<NT>(CQ);
+    zero<NT>(CF);
+    zero<NT>(S);
+    if (me.mat) {
+      tmul<NT>(b0, Q, CQ, n, me);
+      tmul<NT>(b0, F, CF, n, me);
+      as_d4 U[NT];
+      zero<NT>(U);
+      tmul<NT>(b1, Ct, U, n, me);               /* Q C^T */
+      tmul<NT>(b0, U, S, n, me, 0, me.w);       /* S = C Q C^T + I */
+      add_diag<NT>(S, 0, 16 * NT, me);
     }
-    __syncthreads();
-  } else {
-    copy_mat<NB>(A, n, F, n, false, n, n);
-    mm<NB>(A, n, CQ, L, true, Qs, L, false, n, n, m, -1.0, 1.0);             /* A = F - Y_1^T Y_2 */
+    if (me.vec) { /* column 0: o - C w1, the others: o - C c */
+      as_d4 x[NT];
+#pragma unroll
+      for (int r = 0; r < NT; ++r)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) x[r][g] = me.li == 0 ? double(w1[r][g]) : double(c[r][g]);
+      tmul<NT, -1>(b0, x, y, n, me);
+    }
+    chol_forward<NT, false>(s, S, m, me, y, CQ, CF); /* CQ = Y_1, CF = Y_2 */
+    b0.put(CQ, me);
+    b1.put(CF, me);
+    sync<NT>();
+    if (me.mat) {
+      tmul<NT, -1>(b0, CQ, Q, m, me);           /* Z = Q - Y_1^T Y_1 */
+      if (!firstel) tmul<NT, -1>(b0, CF, F, m, me); /* A = F - Y_1^T Y_2 */
+      tmul<NT>(b1, CF, J, m, me);               /* J = Y_2^T Y_2 */
+    }
+    if (me.vec) {
+      tmul<NT>(b0, y, w1, m, me);               /* b = w1 + Y_1^T r (column 0) */
+      tmul<NT>(b1, y, e, m, me);                /* e = Y_2^T rc (column 1) */
+      spread<1>(e);
+    }
   }
-  mv<NB>(e, Qs, L, true, rc, n, m, 1.0, 0.0);                                /* e = Y_2^T rc */
-  mm<NB>(J, n, Qs, L, true, Qs, L, false, n, n, m, 1.0, 0.0);                /* J = Y_2^T Y_2 */
+  if (me.mat) {
+    if (firstel) zero<NT>(F);
+    store<NT, false>(F, el.A + ge * nn, n, me);
+    store<NT, true>(Q, el.Z + ge * nn, n, me);
+    store<NT, true>(J, el.J + ge * nn, n, me);
+  }
+  if (me.vec) {
+    store_vec<NT>(w1, el.b + ge * n, n, me);
+    store_vec<NT>(e, el.e + ge * n, n, me);
+  }
 }
 
 /* ------------------------------------------------------------------------ */
 /* combines (c :889-1016, matlab :240-262)                                   */
 /* ------------------------------------------------------------------------ */
 
-/* blocks of an accumulator or of the work area (LDS, or global for the
- * filtering work of the 64 bucket), leading dimension Ld<NB>::L */
-struct Blk {
-  double *A, *b, *Z, *e, *J;
+/* The accumulator of a scan: its blocks' columns, and on the vector wave b and
+ * e, which lie in A's and Z's registers where that wave holds no matrix. */
+template <int NT, bool SEP = Geo<NT>::SEP>
+struct Acc {
+  as_d4 A[NT], Z[NT], J[NT], vb[NT], ve[NT];
+  __device__ __forceinline__ as_d4 (&b())[NT] { return vb; }
+  __device__ __forceinline__ as_d4 (&e())[NT] { return ve; }
 };
-template <int NB>
-struct Work {
-  double *W1, *T, *T2, *Aj; /* W1: J_j, or E_j of the smoothing combine */
-  double *v, *t0;           /* two vectors, NB apart; one */
+template <int NT>
+struct Acc<NT, true> {
+  as_d4 A[NT], Z[NT], J[NT];
+  __device__ __forceinline__ as_d4 (&b())[NT] { return A; }
+  __device__ __forceinline__ as_d4 (&e())[NT] { return Z; }
 };
 
 /* a <- a (x) element g, filtering (A, b, Z, e, J of the reference's combine):
@@ -772,152 +955,182 @@ struct Work {
  * G^{-1} L^T A_j^T, y_0 = G^{-1} (L^{-1} b_i + L^T e_j), y_1 = G^{-1} L^T (e_j -
  * J_j b_i):
  *   A = Y_b^T Y_1, b = Y_b^T y_0 + b_j, Z = Y_b^T Y_b + Z_j, e = Y_1^T y_1 + e_i,
- *   J = Y_1^T Y_2 + J_i.
- * Element g's blocks are read from HBM into registers first (all loads in
- * flight together) and written into LDS where they are needed. */
-template <int NB>
-__device__ void filt_combine(const Blk& a, const Work<NB>& w, const AsElems& el, int64_t g, int n) {
-  constexpr int L = Ld<NB>::L;
+ *   J = Y_1^T Y_2 + J_i. */
+template <int NT>
+__device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsElems& el, int64_t g, int n,
+                                             const Who<NT>& me) {
+  constexpr bool SEP = Geo<NT>::SEP;
   const int64_t nn = (int64_t)n * n;
-  const double *bj = el.b + g * n, *ej = el.e + g * n;
-  /* Up to NB = 48 Z_j is requested with the others; the 64 bucket fetches it
-   * where it is used, to stay within its registers. */
-  constexpr bool EARLY = NB <= 48;
-  RegBlk<NB> rA, rZ, rJ;
-  rJ.load(el.J + g * nn, n);
-  rA.load(el.A + g * nn, n);
-  if (EARLY) rZ.load(el.Z + g * nn, n);
-  rJ.store(w.W1, L, n, false);
-  rA.store(w.Aj, L, n, false);
-  for (int i = threadIdx.x; i < n; i += AT<NB>) {
-    w.v[i] = a.b[i];
-    w.t0[i] = ej[i];
-  }
-  __syncthreads();
-  mm<NB>(w.T2, L, w.W1, L, false, a.A, L, false, n, n, n, 1.0, 0.0);         /* T2 = J_j A_i */
+  Sh<NT> b0 = sh<NT>(s.b0), b1 = sh<NT>(s.b1);
+  as_d4 B1[NT], T2[NT], x[NT]; /* x: vector wave */
   {
-    double* const B[1] = {a.A};
-    chol_forward<NB, true, true>(a.Z, L, n, B, n, L, w.v, 1);                /* Z = L, A = L^{-1} A_i, v = L^{-1} b_i */
+    as_d4 Jj[NT];
+    if (me.mat) {
+      load<NT, true>(Jj, el.J + g * nn, n, n, n, me);
+      load<NT, true>(B1, el.A + g * nn, n, n, n, me); /* A_j^T */
+    }
+    if (me.vec) load_vec<NT>(x, el.e + g * n, n, me);
+    b0.put(Jj, me);
   }
-  mv<NB>(w.v, a.Z, L, true, w.t0, n, n, 1.0, 1.0);                           /* v = L^{-1} b_i + L^T e_j */
-  mv<NB>(w.t0, w.W1, L, false, a.b, n, n, -1.0, 1.0);                        /* t0 = e_j - J_j b_i */
-  mv<NB>(w.v + NB, a.Z, L, true, w.t0, n, n, 1.0, 0.0);
-  mm<NB>(w.T, L, w.W1, L, false, a.Z, L, false, n, n, n, 1.0, 0.0);          /* T = J_j L */
-  mm<NB>(w.T, L, a.Z, L, true, w.T, L, false, n, n, n, 1.0, 0.0);
-  for (int i = threadIdx.x; i < n; i += AT<NB>) w.T[i * (L + 1)] += 1.0;     /* T = N (read after the next barrier) */
-  mm<NB>(w.T2, L, a.Z, L, true, w.T2, L, false, n, n, n, 1.0, 0.0);
-  mm<NB>(w.Aj, L, a.Z, L, true, w.Aj, L, true, n, n, n, 1.0, 0.0);           /* L^T A_j^T */
-  {
-    double* const B[3] = {a.A, w.T2, w.Aj};
-    chol_forward<NB, false, false>(w.T, L, n, B, n, L, w.v, 2);              /* Y_1, Y_2, Y_b, y_0, y_1 */
+  sync<NT>();
+  if (me.mat) {
+    zero<NT>(T2);
+    tmul<NT>(b0, a.A, T2, n, me); /* J_j A_i */
   }
-  mv<NB>(a.b, w.Aj, L, true, w.v, n, n, 1.0, 0.0);
-  axpy<NB>(a.b, bj, n, 1.0);                                                 /* b */
-  mv<NB>(a.e, a.A, L, true, w.v + NB, n, n, 1.0, 1.0);                       /* e */
-  mm<NB>(a.J, L, a.A, L, true, w.T2, L, false, n, n, n, 1.0, 1.0);           /* J */
-  if (!EARLY) rZ.load(el.Z + g * nn, n);
-  rZ.store(a.Z, L, n, false);                                                /* Z = Z_j */
-  __syncthreads();
-  mm<NB>(a.Z, L, w.Aj, L, true, w.Aj, L, false, n, n, n, 1.0, 1.0);          /* Z */
-  mm<NB>(a.A, L, w.Aj, L, true, a.A, L, false, n, n, n, 1.0, 0.0);           /* A */
+  if (me.vec) { /* column 0: e_j; the others: e_j - J_j b_i */
+    as_d4 u[NT];
+#pragma unroll
+    for (int r = 0; r < NT; ++r) u[r] = x[r];
+    tmul<NT, -1>(b0, a.b(), u, n, me);
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) x[r][h] = me.li == 0 ? double(x[r][h]) : double(u[r][h]);
+  }
+  if (me.mat) add_diag<NT>(a.Z, n, 16 * NT, me);
+  as_d4 M[NT]; /* Z = L L^T, then N = G G^T (e is the vector wave's Z) */
+#pragma unroll
+  for (int r = 0; r < NT; ++r) M[r] = a.Z[r];
+  if constexpr (SEP) chol_forward<NT, true>(s, M, n, me, a.A);
+  else chol_forward<NT, true>(s, M, n, me, a.b(), a.A); /* L^{-1} A_i, L^{-1} b_i */
+  b1.put_upper_t(M, me);
+  sync<NT>();
+  if (me.mat) {
+    as_d4 Lc[NT], T[NT], C2[NT];
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      Lc[r] = as_d4{0.0, 0.0, 0.0, 0.0};
+      if (r >= me.w) Lc[r] = b1.tile(r, me.w, me);
+    }
+    zero<NT>(T);
+    tmul<NT>(b0, Lc, T, n, me, me.w); /* J_j L */
+    zero<NT>(M);
+    tmul<NT, 1, true>(b1, T, M, n, me, 0, me.w);
+    add_diag<NT>(M, 0, 16 * NT, me);  /* N */
+    zero<NT>(C2);
+    tmul<NT, 1, true>(b1, T2, C2, n, me);
+    zero<NT>(T);
+    tmul<NT, 1, true>(b1, B1, T, n, me);
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      T2[r] = C2[r]; /* L^T J_j A_i */
+      B1[r] = T[r];  /* L^T A_j^T */
+    }
+  }
+  if (me.vec) { /* column 0: L^{-1} b_i + L^T e_j; the others: L^T (e_j - J_j b_i) */
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) a.b()[r][h] = me.li == 0 ? double(a.b()[r][h]) : 0.0;
+    tmul<NT, 1, true>(b1, x, a.b(), n, me);
+  }
+  if constexpr (SEP) chol_forward<NT, false>(s, M, n, me, a.A, T2, B1); /* y_0 | y_1 and Y_1, Y_2, Y_b */
+  else chol_forward<NT, false>(s, M, n, me, a.b(), a.A, T2, B1);
+  if (me.mat) load<NT, true>(a.Z, el.Z + g * nn, n, n, n, me);
+  as_d4 bn[NT];
+  if (me.vec) load_vec<NT>(bn, el.b + g * n, n, me);
+  b0.put(B1, me);
+  b1.put(a.A, me);
+  sync<NT>();
+  if (me.mat) {
+    tmul<NT>(b1, T2, a.J, n, me);
+    tmul<NT>(b0, B1, a.Z, n, me);
+#pragma unroll
+    for (int r = 0; r < NT; ++r) T2[r] = a.A[r];
+  }
+  if (me.vec) {
+    tmul<NT>(b0, a.b(), bn, n, me);
+    spread<0>(bn);
+    as_d4 y1[NT];
+    zero<NT>(y1);
+    tmul<NT>(b1, a.b(), y1, n, me);
+    spread<1>(y1);
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      a.e()[r] += y1[r];
+      a.b()[r] = bn[r];
+    }
+  }
+  if (me.mat) {
+    zero<NT>(a.A);
+    tmul<NT>(b0, T2, a.A, n, me);
+  }
+  sync<NT>();
 }
 
 /* a <- a (x) element g, smoothing; a is the running suffix and g the next
  * earlier step: E = E_j E_i, g = E_j g_i + g_j, L = E_j L_i E_j^T + L_j. */
-template <int NB>
-__device__ void smooth_combine(const Blk& a, const Work<NB>& w, const AsElems& el, int64_t g, int n) {
-  constexpr int L = Ld<NB>::L;
+template <int NT>
+__device__ __forceinline__ void smooth_combine(Acc<NT>& a, Lds<NT>& s, const AsElems& el, int64_t g, int n,
+                                               const Who<NT>& me) {
   const int64_t nn = (int64_t)n * n;
-  const double* gj = el.b + g * n;
-  RegBlk<NB> rE, rL;
-  rE.load(el.A + g * nn, n);
-  rL.load(el.Z + g * nn, n);
-  rE.store(w.W1, L, n, false);                                               /* W1 = E_j */
-  __syncthreads();
-  mm<NB>(a.A, L, w.W1, L, false, a.A, L, false, n, n, n, 1.0, 0.0);
-  mv<NB>(a.b, w.W1, L, false, a.b, n, n, 1.0, 0.0);
-  axpy<NB>(a.b, gj, n, 1.0);
-  mm<NB>(w.T, L, w.W1, L, false, a.Z, L, false, n, n, n, 1.0, 0.0);
-  rL.store(a.Z, L, n, false);
-  __syncthreads();
-  mm<NB>(a.Z, L, w.T, L, false, w.W1, L, true, n, n, n, 1.0, 1.0);
-}
-
-template <int NB>
-__device__ void blk_load(const Blk& a, int ld, const AsElems& el, int64_t g, int n, bool filt) {
-  const int64_t nn = (int64_t)n * n;
-  RegBlk<NB> r;
-  r.load(el.A + g * nn, n);
-  r.store(a.A, ld, n, false);
-  r.load(el.Z + g * nn, n);
-  r.store(a.Z, ld, n, false);
-  if (filt) {
-    r.load(el.J + g * nn, n);
-    r.store(a.J, ld, n, false);
+  Sh<NT> b0 = sh<NT>(s.b0), b1 = sh<NT>(s.b1);
+  as_d4 Et[NT], Lj[NT], gj[NT];
+  if (me.mat) {
+    load<NT, true>(Et, el.A + g * nn, n, n, n, me); /* E_j^T */
+    load<NT, true>(Lj, el.Z + g * nn, n, n, n, me);
   }
-  for (int i = threadIdx.x; i < n; i += AT<NB>) {
-    a.b[i] = el.b[g * n + i];
-    if (filt) a.e[i] = el.e[g * n + i];
-  }
-  __syncthreads();
-}
-
-template <int NB>
-__device__ void blk_store(const Blk& a, int ld, const AsElems& el, int64_t g, int n, bool filt) {
-  const int64_t nn = (int64_t)n * n;
-  for (int idx = threadIdx.x; idx < NB * NB; idx += AT<NB>) {
-    const int i = idx % NB, j = idx / NB;
-    if (i < n && j < n) {
-      el.A[g * nn + i + j * n] = a.A[i + j * ld];
-      el.Z[g * nn + i + j * n] = a.Z[i + j * ld];
-      if (filt) el.J[g * nn + i + j * n] = a.J[i + j * ld];
+  if (me.vec) load_vec<NT>(gj, el.b + g * n, n, me);
+  b0.put(Et, me);
+  b1.put(a.Z, me);
+  sync<NT>();
+  if (me.mat) {
+    as_d4 U[NT];
+    zero<NT>(U);
+    tmul<NT>(b1, Et, U, n, me); /* L_i E_j^T */
+    tmul<NT>(b0, U, Lj, n, me);
+    zero<NT>(U);
+    tmul<NT>(b0, a.A, U, n, me);
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      a.Z[r] = Lj[r];
+      a.A[r] = U[r];
     }
   }
-  for (int i = threadIdx.x; i < n; i += AT<NB>) {
-    el.b[g * n + i] = a.b[i];
-    if (filt) el.e[g * n + i] = a.e[i];
+  if (me.vec) {
+    tmul<NT>(b0, a.b(), gj, n, me);
+#pragma unroll
+    for (int r = 0; r < NT; ++r) a.b()[r] = gj[r];
   }
-  __syncthreads();
+  sync<NT>();
 }
 
-/* LDS plan of a scan kernel: accumulator, then the work area when it fits */
-template <int NB, bool FILT>
-struct ScanPlan {
-  static constexpr int SZ = Ld<NB>::SZ;
-  static constexpr int ACC = FILT ? 3 * SZ + 2 * NB : 2 * SZ + NB;
-  static constexpr int WORK = FILT ? 4 * SZ + 3 * NB : 2 * SZ;             /* W1, T, T2, Aj, v, t0 | W1, T */
-  static constexpr bool WORK_GLOBAL = (ACC + WORK) * 8 > LDS_BYTES;
-  static constexpr int LDS = ACC + (WORK_GLOBAL ? 0 : WORK);
-};
-
-template <int NB, bool FILT>
-__device__ void scan_setup(double* lds, double* gwork, Blk& a, Work<NB>& w) {
-  using SP = ScanPlan<NB, FILT>;
-  constexpr int SZ = SP::SZ;
-  double* q = lds;
-  a.A = q; q += SZ;
-  a.Z = q; q += SZ;
-  a.J = nullptr;
-  a.e = nullptr;
-  if (FILT) { a.J = q; q += SZ; }
-  a.b = q; q += NB;
-  if (FILT) { a.e = q; q += NB; }
-  double* p = SP::WORK_GLOBAL ? gwork + (int64_t)blockIdx.x * SP::WORK : q;
-  w.W1 = p; p += SZ;
-  w.T = p; p += SZ;
-  w.T2 = w.Aj = w.v = w.t0 = nullptr;
-  if (FILT) {
-    w.T2 = p; p += SZ;
-    w.Aj = p; p += SZ;
-    w.v = p; p += 2 * NB;
-    w.t0 = p;
+template <int NT, bool FILT>
+__device__ __forceinline__ void acc_load(Acc<NT>& a, const AsElems& el, int64_t g, int n, const Who<NT>& me) {
+  const int64_t nn = (int64_t)n * n;
+  if (me.mat) {
+    load<NT, false>(a.A, el.A + g * nn, n, n, n, me);
+    load<NT, true>(a.Z, el.Z + g * nn, n, n, n, me);
+    if (FILT) load<NT, true>(a.J, el.J + g * nn, n, n, n, me);
+  }
+  if (me.vec) {
+    load_vec<NT>(a.b(), el.b + g * n, n, me);
+    if (FILT) load_vec<NT>(a.e(), el.e + g * n, n, me);
   }
 }
-
-template <int NB, bool FILT>
-__device__ __forceinline__ void combine(const Blk& a, const Work<NB>& w, const AsElems& el, int64_t g, int n) {
-  if (FILT) filt_combine<NB>(a, w, el, g, n);
-  else smooth_combine<NB>(a, w, el, g, n);
+template <int NT, bool FILT>
+__device__ __forceinline__ void acc_store(const Acc<NT>& ac, const AsElems& el, int64_t g, int n, Who<NT> me) {
+  Acc<NT>& a = const_cast<Acc<NT>&>(ac);
+  asm volatile("" : "+s"(n), "+v"(me.li), "+v"(me.lk));
+  const int64_t nn = (int64_t)n * n;
+  if (me.mat) {
+    store<NT, false>(a.A, el.A + g * nn, n, me);
+    store<NT, true>(a.Z, el.Z + g * nn, n, me);
+    if (FILT) store<NT, true>(a.J, el.J + g * nn, n, me);
+  }
+  if (me.vec) {
+    store_vec<NT>(a.b(), el.b + g * n, n, me);
+    if (FILT) store_vec<NT>(a.e(), el.e + g * n, n, me);
+  }
+}
+/* n and the lane are opaque, so that the addresses and masks made from them are
+ * made in each combine: kept over a chunk's loop they took a fifth of the
+ * registers */
+template <int NT, bool FILT>
+__device__ __forceinline__ void combine(Acc<NT>& a, Lds<NT>& s, const AsElems& el, int64_t g, int n, Who<NT> me) {
+  asm volatile("" : "+s"(n), "+v"(me.li), "+v"(me.lk), "+v"(me.lane));
+  if constexpr (FILT) filt_combine<NT>(a, s, el, g, n, me);
+  else smooth_combine<NT>(a, s, el, g, n, me);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -936,61 +1149,57 @@ struct Chunk {
   int32_t pad;
 };
 
+/* waves per SIMD the scans are compiled for: two workgroups of four waves on a
+ * CU at NT = 3; all registers for one wave at NT = 4 */
+template <int NT>
+constexpr int SCAN_OCC = NT == 4 ? 1 : 2;
+
 /* pass 1: the total of every chunk */
-template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT<NB>) ka_scan_reduce(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
-  using SP = ScanPlan<NB, FILT>;
-  __shared__ double lds[SP::LDS];
-  Blk a;
-  Work<NB> w;
-  scan_setup<NB, FILT>(lds, gwork, a, w);
+template <int NT, bool FILT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_scan_reduce(const Chunk* ch, AsElems el, AsElems tot,
+                                                                               int n) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Acc<NT> a;
   const Chunk c = ch[blockIdx.x];
-  blk_load<NB>(a, Ld<NB>::L, el, c.first, n, FILT);
-  for (int i = 1; i < c.len; ++i) combine<NB, FILT>(a, w, el, c.first + (int64_t)i * c.dir, n);
-  blk_store<NB>(a, Ld<NB>::L, tot, c.tot, n, FILT);
+  acc_load<NT, FILT>(a, el, c.first, n, me);
+#pragma unroll 1
+  for (int i = 1; i < c.len; ++i) combine<NT, FILT>(a, s, el, c.first + (int64_t)i * c.dir, n, me);
+  acc_store<NT, FILT>(a, tot, c.tot, n, me);
 }
 
 /* pass 2, one Hillis-Steele round over the chunk totals of every problem:
  * out[t] = in[t - d] (x) in[t] when rank >= d, else in[t]. */
-template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT<NB>) ka_scan_round(const Chunk* ch, AsElems in, AsElems out, int d, int n,
-                                                    double* gwork) {
-  using SP = ScanPlan<NB, FILT>;
-  __shared__ double lds[SP::LDS];
-  Blk a;
-  Work<NB> w;
-  scan_setup<NB, FILT>(lds, gwork, a, w);
+template <int NT, bool FILT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_scan_round(const Chunk* ch, AsElems in, AsElems out,
+                                                                              int d, int n) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Acc<NT> a;
   const Chunk c = ch[blockIdx.x];
-  if (c.rank >= d) {
-    blk_load<NB>(a, Ld<NB>::L, in, c.tot - d, n, FILT);
-    combine<NB, FILT>(a, w, in, c.tot, n);
-  } else {
-    blk_load<NB>(a, Ld<NB>::L, in, c.tot, n, FILT);
-  }
-  blk_store<NB>(a, Ld<NB>::L, out, c.tot, n, FILT);
+  const bool join = c.rank >= d;
+  acc_load<NT, FILT>(a, in, join ? c.tot - d : c.tot, n, me);
+  if (join) combine<NT, FILT>(a, s, in, c.tot, n, me);
+  acc_store<NT, FILT>(a, out, c.tot, n, me);
 }
 
 /* pass 3: every prefix within a chunk, seeded with the inclusive total of
  * the chunk before it; results overwrite the elements in place. */
-template <int NB, bool FILT>
-__global__ void __launch_bounds__(AT<NB>) ka_scan_down(const Chunk* ch, AsElems el, AsElems tot, int n, double* gwork) {
-  using SP = ScanPlan<NB, FILT>;
-  __shared__ double lds[SP::LDS];
-  Blk a;
-  Work<NB> w;
-  scan_setup<NB, FILT>(lds, gwork, a, w);
+template <int NT, bool FILT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_scan_down(const Chunk* ch, AsElems el, AsElems tot,
+                                                                             int n) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Acc<NT> a;
   const Chunk c = ch[blockIdx.x];
-  int i0 = 0;
-  if (c.rank == 0) {
-    blk_load<NB>(a, Ld<NB>::L, el, c.first, n, FILT);
-    i0 = 1;
-  } else {
-    blk_load<NB>(a, Ld<NB>::L, tot, c.tot - 1, n, FILT);
-  }
+  const int i0 = c.rank == 0 ? 1 : 0;
+  if (i0) acc_load<NT, FILT>(a, el, c.first, n, me);
+  else acc_load<NT, FILT>(a, tot, c.tot - 1, n, me);
+#pragma unroll 1
   for (int i = i0; i < c.len; ++i) {
     const int64_t g = c.first + (int64_t)i * c.dir;
-    combine<NB, FILT>(a, w, el, g, n);
-    blk_store<NB>(a, Ld<NB>::L, el, g, n, FILT);
+    combine<NT, FILT>(a, s, el, g, n, me);
+    acc_store<NT, FILT>(a, el, g, n, me);
   }
 }
 
@@ -1018,66 +1227,97 @@ __global__ void __launch_bounds__(AT<NB>) ka_filtered(const AsProb* probs, const
  *   t < p:  from the information form (Lam, eta),
  *           L = (Lam + F^T Q^{-1} F)^{-1}, E = L F^T Q^{-1}, g = L (eta - F^T Q^{-1} c).
  */
-template <int NB>
-__global__ void __launch_bounds__(AT<NB>) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md, AsElems el,
-                                               int n) {
-  constexpr int L = Ld<NB>::L;
-  __shared__ double M[Ld<NB>::SZ], T[Ld<NB>::SZ], U[Ld<NB>::SZ];
-  __shared__ double v1[NB], v2[NB];
-  const int64_t s = blockIdx.x;
-  const AsProb pr = probs[step_prob[s]];
-  const int64_t t = s - pr.s0;
+template <int NT>
+__global__ void __launch_bounds__(Geo<NT>::THREADS) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md,
+                                                             AsElems el, int n) {
+  __shared__ Lds<NT> s;
+  const Who<NT> me;
+  Sh<NT> b0 = sh<NT>(s.b0), b1 = sh<NT>(s.b1);
+  const int64_t st = blockIdx.x;
+  const AsProb pr = probs[step_prob[st]];
+  const int64_t t = st - pr.s0;
   const int64_t nn = (int64_t)n * n;
-  double* E = el.A + s * nn;
-  double* gv = el.b + s * n;
-  double* Lo = el.Z + s * nn;
+  double* E = el.A + st * nn;
+  double* gv = el.b + st * n;
+  double* Lo = el.Z + st * nn;
   if (t == pr.k - 1) {
-    for (int idx = threadIdx.x; idx < n * n; idx += AT<NB>) {
+    for (int idx = threadIdx.x; idx < n * n; idx += Geo<NT>::THREADS) {
       E[idx] = 0.0;
-      Lo[idx] = md.Pf[s * nn + idx];
+      Lo[idx] = md.Pf[st * nn + idx];
     }
-    for (int i = threadIdx.x; i < n; i += AT<NB>) gv[i] = md.xf[s * n + i];
+    for (int i = threadIdx.x; i < n; i += Geo<NT>::THREADS) gv[i] = md.xf[st * n + i];
     return;
   }
-  const double* F = md.F + (s + 1) * nn;
-  const double* c = md.c + (s + 1) * n;
-  const double* Q = md.Q + (s + 1) * nn;
+  const double* F = md.F + (st + 1) * nn;
+  as_d4 M[NT], Y[NT], W[NT], y[NT], D[NT], P[NT], x[NT];
+  load<NT, true>(M, md.Q + (st + 1) * nn, n, n, n, me);
+  load_vec<NT>(y, md.c + (st + 1) * n, n, me);
+  zero<NT>(W);
+  add_diag<NT>(W, 0, n, me);
+  zero<NT>(D);
   if (t >= pr.p) {
-    const double* P = md.Pf + s * nn;
-    const double* x = md.xf + s * n;
-    copy_mat<NB>(U, L, P, n, false, n, n);                                   /* U = P */
-    copy_mat<NB>(M, L, F, n, false, n, n);                                   /* M = F */
-    mm<NB>(T, L, M, L, false, U, L, false, n, n, n, 1.0, 0.0);               /* T = F P */
-    mv<NB>(v1, M, L, false, x, n, n, 1.0, 0.0);
-    axpy<NB>(v1, c, n, 1.0);                                                 /* v1 = F x + c */
-    copy_mat<NB>(U, L, Q, n, false, n, n);
-    mm<NB>(U, L, T, L, false, M, L, true, n, n, n, 1.0, 1.0);                /* U = F P F^T + Q = G G^T */
-    set_identity<NB>(M, L, n, 1.0);
-    double* const B[2] = {T, M};
-    chol_forward<NB, false, false>(U, L, n, B, n, L, nullptr, 0);            /* T = Y = G^{-1} F P, M = G^{-1} */
-    mm<NB>(E, n, T, L, true, M, L, false, n, n, n, 1.0, 0.0);                /* E = Y^T G^{-1} */
-    mv<NB>(v2, M, L, false, v1, n, n, 1.0, 0.0);
-    mv<NB>(gv, T, L, true, v2, n, n, -1.0, 0.0);
-    axpy<NB>(gv, x, n, 1.0);                                                 /* g = x - E (F x + c) */
-    copy_mat<NB>(Lo, n, P, n, false, n, n);
-    mm<NB>(Lo, n, T, L, true, T, L, false, n, n, n, -1.0, 1.0);              /* L = P - Y^T Y */
+    load<NT, true>(P, md.Pf + st * nn, n, n, n, me);
+    load<NT, true>(D, F, n, n, n, me); /* F^T */
+    load_vec<NT>(x, md.xf + st * n, n, me);
+    b0.put(D, me);
+    b1.put(P, me);
+    sync<NT>();
+    zero<NT>(Y);
+    if (me.mat) {
+      tmul<NT>(b0, P, Y, n, me);              /* Y = F P */
+      as_d4 U[NT];
+      zero<NT>(U);
+      tmul<NT>(b1, D, U, n, me);              /* U = P F^T */
+      tmul<NT>(b0, U, M, n, me, 0, me.w);     /* M = F P F^T + Q = G G^T */
+    }
+    if (me.vec) tmul<NT>(b0, x, y, n, me);    /* y = F x + c */
+    add_diag<NT>(M, n, 16 * NT, me);
+    chol_forward<NT, false>(s, M, n, me, y, Y, W); /* Y = G^{-1} F P, W = G^{-1}, y = G^{-1} (F x + c) */
+    b0.put(Y, me);
+    sync<NT>();
+    if (me.mat) {
+      zero<NT>(D);
+      tmul<NT>(b0, W, D, n, me);
+      store<NT, false>(D, E, n, me);          /* E = Y^T W */
+      tmul<NT, -1>(b0, Y, P, n, me);
+      store<NT, true>(P, Lo, n, me);          /* L = P - Y^T Y */
+    }
+    if (me.vec) {
+      tmul<NT, -1>(b0, y, x, n, me);
+      store_vec<NT>(x, gv, n, me);            /* g = x - E (F x + c) */
+    }
   } else {
-    copy_mat<NB>(U, L, Q, n, false, n, n);
-    copy_mat<NB>(T, L, F, n, false, n, n);
-    copy_vec<NB>(v1, c, n);
-    set_identity<NB>(M, L, n, 1.0);
-    double* const B[2] = {T, M};
-    chol_forward<NB, false, false>(U, L, n, B, n, L, v1, 1);                 /* Q = G G^T: T = Y = G^{-1} F, M = G^{-1}, v1 = G^{-1} c */
-    mm<NB>(M, L, M, L, true, T, L, false, n, n, n, 1.0, 0.0);                /* M = Q^{-1} F */
-    copy_mat<NB>(U, L, md.Lam + s * nn, n, false, n, n);
-    mm<NB>(U, L, T, L, true, T, L, false, n, n, n, 1.0, 1.0);                /* U = Lam + F^T Q^{-1} F */
-    mv<NB>(v2, T, L, true, v1, n, n, -1.0, 0.0);
-    axpy<NB>(v2, md.eta + s * n, n, 1.0);                                    /* v2 = eta - F^T Q^{-1} c */
-    chol_inverse_factor<NB>(U, T, L, n);
-    mm<NB>(T, L, T, L, true, T, L, false, n, n, n, 1.0, 0.0);                /* T = L */
-    copy_mat<NB>(Lo, n, T, L, false, n, n);
-    mm<NB>(E, n, T, L, false, M, L, true, n, n, n, 1.0, 0.0);                /* E = L (Q^{-1} F)^T */
-    mv<NB>(gv, T, L, false, v2, n, n, 1.0, 0.0);                             /* g = L (eta - F^T Q^{-1} c) */
+    load<NT, false>(Y, F, n, n, n, me);
+    load<NT, true>(P, md.Lam + st * nn, n, n, n, me);
+    load_vec<NT>(x, md.eta + st * n, n, me);
+    add_diag<NT>(M, n, 16 * NT, me);
+    chol_forward<NT, false>(s, M, n, me, y, Y, W); /* Q = G G^T: Y = G^{-1} F, W = G^{-1}, y = G^{-1} c */
+    b0.put(Y, me);
+    sync<NT>();
+    if (me.mat) {
+      tmul<NT>(b0, W, D, n, me);              /* D = F^T Q^{-1} */
+      tmul<NT>(b0, Y, P, n, me);              /* P = Lam + F^T Q^{-1} F = H H^T */
+    }
+    if (me.vec) tmul<NT, -1>(b0, y, x, n, me); /* x = eta - F^T Q^{-1} c */
+    add_diag<NT>(P, n, 16 * NT, me);
+    zero<NT>(W);
+    add_diag<NT>(W, 0, n, me);
+    chol_forward<NT, false>(s, P, n, me, x, W, D); /* W = H^{-1}, D = H^{-1} F^T Q^{-1}, x = H^{-1} x */
+    b0.put(W, me);
+    sync<NT>();
+    if (me.mat) {
+      zero<NT>(M);
+      tmul<NT>(b0, W, M, n, me);
+      store<NT, true>(M, Lo, n, me);          /* L = W^T W */
+      zero<NT>(M);
+      tmul<NT>(b0, D, M, n, me);
+      store<NT, false>(M, E, n, me);          /* E = L F^T Q^{-1} */
+    }
+    if (me.vec) {
+      zero<NT>(y);
+      tmul<NT>(b0, x, y, n, me);
+      store_vec<NT>(y, gv, n, me);            /* g = L x */
+    }
   }
 }
 
@@ -1140,12 +1380,12 @@ int64_t make_chunks(std::vector<Chunk>& out, int64_t base, int64_t len, int dir,
   return nch;
 }
 
-/* Chunks aimed at over a batch: as many as the filtering scan's workgroups
- * that are resident at once (by its LDS: one per CU in buckets 48 and 64, two
- * in 32, ten single waves in 16). More would only add to the rounds over the
- * chunk totals. Chunks have at least 4 elements. */
+/* Chunks aimed at over a batch: as many as the scan's workgroups that are
+ * resident at once (two per CU at n = 33 .. 48, one above, ten single waves for
+ * n <= 16). More would only add to the rounds over the chunk totals. Chunks
+ * have at least 4 elements. */
 template <int NB>
-constexpr int64_t CHUNKS_TARGET = NB <= 16 ? 2560 : (NB <= 32 ? 512 : 256);
+constexpr int64_t CHUNKS_TARGET = NB <= 16 ? 2560 : (NB <= 32 ? 768 : (NB <= 48 ? 512 : 256));
 
 template <int NB>
 int run_assoc(ukhip_batch* b) {
@@ -1216,8 +1456,6 @@ int run_assoc(ukhip_batch* b) {
   const size_t o_ft0 = take(elem_bytes(ftot, true)), o_ft1 = take(elem_bytes(ftot, true));
   const size_t o_se = take(elem_bytes(S, false));
   const size_t o_st0 = take(elem_bytes(stot, false)), o_st1 = take(elem_bytes(stot, false));
-  const int64_t maxch = std::max<int64_t>((int64_t)std::max(fch.size(), sch.size()), 1);
-  const size_t o_gw = take((size_t)maxch * ScanPlan<NB, true>::WORK * 8);
   const size_t tab_bytes = probs.size() * sizeof(AsProb) + (elem_prob.size() + step_prob.size()) * 4 +
                            (fch.size() + sch.size()) * sizeof(Chunk) + 6 * 256;
   const size_t o_tab = take(tab_bytes);
@@ -1255,7 +1493,6 @@ int run_assoc(ukhip_batch* b) {
   const AsElems ft[2] = {elems_at(o_ft0, ftot, true), elems_at(o_ft1, ftot, true)};
   const AsElems se = elems_at(o_se, S, false);
   const AsElems stt[2] = {elems_at(o_st0, stot, false), elems_at(o_st1, stot, false)};
-  double* gw = (double*)(W + o_gw);
 
   /* tables */
   std::vector<char> tab(tab_bytes, 0);
@@ -1273,7 +1510,8 @@ int run_assoc(ukhip_batch* b) {
   const Chunk* d_sch = (const Chunk*)put(sch.data(), sch.size() * sizeof(Chunk));
   if (!ok(hipMemcpyAsync(W + o_tab, tab.data(), to, hipMemcpyHostToDevice, st), "upload scan tables")) return -1;
 
-  const dim3 blk(AT<NB>);
+  constexpr int NT = NB / 16;
+  const dim3 blk(AT<NB>), tblk(Geo<NT>::THREADS);
   AsTimer* tm = t_timer;
   auto mark = [&](int slot, int launches) { /* slot's launches are done: its closing event */
     if (!tm) return;
@@ -1289,20 +1527,20 @@ int run_assoc(ukhip_batch* b) {
   if (diag) ka_model_diag<<<dim3((unsigned)S), dim3(256), 0, st>>>(*raw, md, n);
   else ka_model<NB><<<dim3((unsigned)S), blk, 0, st>>>(wch, raw->first, md, n);
   mark(UKHIP_AS_MODEL, 1);
-  ka_prior<NB><<<dim3((unsigned)nprob), blk, 0, st>>>(d_probs, wch, m_obs, md, n, mr);
+  ka_prior<NT><<<dim3((unsigned)nprob), tblk, 0, st>>>(d_probs, wch, m_obs, md, n, mr);
   mark(UKHIP_AS_PRIOR, 1);
   if (ne > 0) {
     const unsigned nc = (unsigned)fch.size();
-    ka_felem<NB><<<dim3((unsigned)ne), blk, 0, st>>>(d_probs, d_elem_prob, wch, m_obs, md, fe, n, mr);
+    ka_felem<NT><<<dim3((unsigned)ne), tblk, 0, st>>>(d_probs, d_elem_prob, wch, m_obs, md, fe, n, mr);
     mark(UKHIP_AS_FELEM, 1);
-    ka_scan_reduce<NB, true><<<dim3(nc), blk, 0, st>>>(d_fch, fe, ft[0], n, gw);
+    ka_scan_reduce<NT, true><<<dim3(nc), tblk, 0, st>>>(d_fch, fe, ft[0], n);
     int cur = 0, rounds = 0;
     for (int64_t d = 1; d < maxr_f; d <<= 1) {
-      ka_scan_round<NB, true><<<dim3(nc), blk, 0, st>>>(d_fch, ft[cur], ft[cur ^ 1], (int)d, n, gw);
+      ka_scan_round<NT, true><<<dim3(nc), tblk, 0, st>>>(d_fch, ft[cur], ft[cur ^ 1], (int)d, n);
       cur ^= 1;
       ++rounds;
     }
-    ka_scan_down<NB, true><<<dim3(nc), blk, 0, st>>>(d_fch, fe, ft[cur], n, gw);
+    ka_scan_down<NT, true><<<dim3(nc), tblk, 0, st>>>(d_fch, fe, ft[cur], n);
     mark(UKHIP_AS_FSCAN, 2 + rounds);
     ka_filtered<NB><<<dim3((unsigned)ne), blk, 0, st>>>(d_probs, d_elem_prob, fe, md, n);
     mark(UKHIP_AS_FILTERED, 1);
@@ -1313,16 +1551,16 @@ int run_assoc(ukhip_batch* b) {
   }
   {
     const unsigned nc = (unsigned)sch.size();
-    ka_selem<NB><<<dim3((unsigned)S), blk, 0, st>>>(d_probs, d_step_prob, md, se, n);
+    ka_selem<NT><<<dim3((unsigned)S), tblk, 0, st>>>(d_probs, d_step_prob, md, se, n);
     mark(UKHIP_AS_SELEM, 1);
-    ka_scan_reduce<NB, false><<<dim3(nc), blk, 0, st>>>(d_sch, se, stt[0], n, gw);
+    ka_scan_reduce<NT, false><<<dim3(nc), tblk, 0, st>>>(d_sch, se, stt[0], n);
     int cur = 0, rounds = 0;
     for (int64_t d = 1; d < maxr_s; d <<= 1) {
-      ka_scan_round<NB, false><<<dim3(nc), blk, 0, st>>>(d_sch, stt[cur], stt[cur ^ 1], (int)d, n, gw);
+      ka_scan_round<NT, false><<<dim3(nc), tblk, 0, st>>>(d_sch, stt[cur], stt[cur ^ 1], (int)d, n);
       cur ^= 1;
       ++rounds;
     }
-    ka_scan_down<NB, false><<<dim3(nc), blk, 0, st>>>(d_sch, se, stt[cur], n, gw);
+    ka_scan_down<NT, false><<<dim3(nc), tblk, 0, st>>>(d_sch, se, stt[cur], n);
     mark(UKHIP_AS_SSCAN, 2 + rounds);
     ka_results<NB><<<dim3((unsigned)S), blk, 0, st>>>(se, xout, Sout, n);
     mark(UKHIP_AS_RESULTS, 1);
