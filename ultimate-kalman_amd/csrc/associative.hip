@@ -176,34 +176,6 @@ __device__ void copy_mat(double* D, int ldd, const double* S, int lds, bool t, i
   __syncthreads();
 }
 
-/* D = d I on the leading n x n block; the padding rows and columns
- * [n, NB) of the NB x NB block become the identity. */
-template <int NB>
-__device__ void set_identity(double* D, int ld, int n, double d) {
-  constexpr int PER = (NB * NB + AT<NB> - 1) / AT<NB>;
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int idx = (int)threadIdx.x + u * AT<NB>;
-    const int i = idx % NB, j = idx / NB;
-    if (idx < NB * NB) D[i + (int64_t)j * ld] = (i == j) ? (i < n ? d : 1.0) : 0.0;
-  }
-  __syncthreads();
-}
-
-/* y (m) = a x + y */
-template <int NB>
-__device__ void axpy(double* y, const double* x, int m, double a) {
-  for (int i = threadIdx.x; i < m; i += AT<NB>) y[i] = fma(a, x[i], y[i]);
-  __syncthreads();
-}
-
-/* y (m) = x */
-template <int NB>
-__device__ void copy_vec(double* y, const double* x, int m) {
-  for (int i = threadIdx.x; i < m; i += AT<NB>) y[i] = x[i];
-  __syncthreads();
-}
-
 /* Pivot keys: |v| with its low 7 mantissa bits replaced by (127 - row), so
  * that an unsigned 64-bit maximum picks the largest magnitude and, among
  * (near-)equal magnitudes, the first row. NaN sorts above every number. */
@@ -373,6 +345,13 @@ struct Geo {
   static constexpr int WAVES = NT + (SEP ? 1 : 0);
   static constexpr int THREADS = 64 * WAVES;
 };
+/* waves per SIMD the kernels over many elements are compiled for: two workgroups of four waves on a
+ * CU at NT = 3; all registers for one wave at NT = 4. (The
+ * element builds at n = 48, k = 10000: 855 -> 551 us and 840 -> 722 us with two,
+ * a few registers spilled included.) */
+template <int NT>
+constexpr int SCAN_OCC = NT == 4 ? 1 : 2;
+
 template <int NT>
 struct Who { /* of this lane */
   int li, lk, lane, w;
@@ -833,7 +812,7 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS) ka_prior(const AsProb* probs
  * (m1 if first), Z = Q (Q1), e = 0, J = 0.
  */
 template <int NT>
-__global__ void __launch_bounds__(Geo<NT>::THREADS) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
+__global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_felem(const AsProb* probs, const int32_t* elem_prob, uk_chain_t wch,
                                                              const int32_t* m_obs, AsModel md, AsElems el, int n, int mr) {
   __shared__ Lds<NT> s;
   const Who<NT> me;
@@ -1149,11 +1128,6 @@ struct Chunk {
   int32_t pad;
 };
 
-/* waves per SIMD the scans are compiled for: two workgroups of four waves on a
- * CU at NT = 3; all registers for one wave at NT = 4 */
-template <int NT>
-constexpr int SCAN_OCC = NT == 4 ? 1 : 2;
-
 /* pass 1: the total of every chunk */
 template <int NT, bool FILT>
 __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_scan_reduce(const Chunk* ch, AsElems el, AsElems tot,
@@ -1228,7 +1202,7 @@ __global__ void __launch_bounds__(AT<NB>) ka_filtered(const AsProb* probs, const
  *           L = (Lam + F^T Q^{-1} F)^{-1}, E = L F^T Q^{-1}, g = L (eta - F^T Q^{-1} c).
  */
 template <int NT>
-__global__ void __launch_bounds__(Geo<NT>::THREADS) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md,
+__global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_selem(const AsProb* probs, const int32_t* step_prob, AsModel md,
                                                              AsElems el, int n) {
   __shared__ Lds<NT> s;
   const Who<NT> me;
