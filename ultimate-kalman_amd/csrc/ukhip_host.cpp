@@ -20,6 +20,7 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -44,7 +45,7 @@ hipError_t uk_launch_cov_format(const double* S, int64_t steps, int n, int fmt, 
 hipError_t uk_launch_backsub(const uk_level_t* lv, const uk_factors_t* fac, double* xout, double* Sout,
                              const double* Xup, const double* XTup, double* Xcur, double* XTcur, int n, int cov,
                              hipStream_t st);
-int uk_assoc_smooth(struct ukhip_batch* b, uint32_t options);
+int uk_assoc_smooth(struct ukhip_batch* b, uint32_t options, hipStream_t st);
 int uk_assoc_smooth_timed(struct ukhip_batch* b, uint32_t options, double* ms, int32_t* launches);
 void uk_set_error(const char* fmt, ...);
 hipError_t uk_launch_eliminate32(const uk_level_t* lv, const uk_chain32_t* in, const uk_chain32_t* out,
@@ -217,7 +218,8 @@ struct ukhip_batch {
   double* Sout = nullptr;
   double* fix = nullptr; /* per problem: Z (n x n) and o (n) of a lone last step */
   int64_t total_evens = 0;
-  /* associative-path workspace, allocated on first use */
+  /* associative-path workspace and plan, made on first use */
+  std::shared_ptr<void> assoc_plan;
   void* d_assoc = nullptr;
   size_t assoc_bytes = 0;
   /* A batch of problems with different state dimensions is a composite: one
@@ -1358,10 +1360,12 @@ extern "C" int ukhip_batch_smooth_associative(ukhip_batch_t* b, uint32_t options
   if (!b) { uk_set_error("NULL batch"); return -1; }
   if (!ensure_stream()) return -1;
   if (!ensure_elim_all(b)) return -1; /* the covariance output */
-  if (b->parts.empty()) return uk_assoc_smooth(b, options);
-  for (auto* q : b->parts)
-    if (uk_assoc_smooth(q, options) != 0) return -1;
-  return 0;
+  const bool done = b->parts.empty()
+                        ? uk_assoc_smooth(b, options, g_stream) == 0
+                        : enqueue_parts(b, [&](ukhip_batch* q, hipStream_t st) { return uk_assoc_smooth(q, options, st) == 0; });
+  if (!done) /* a part may be refused: nothing of the others stays in flight */
+    for (auto st : b->part_streams) (void)hipStreamSynchronize(st);
+  return hip_ok(hipStreamSynchronize(g_stream), "associative smoothing") && done ? 0 : -1;
 }
 
 extern "C" int ukhip_batch_smooth_associative_timed(ukhip_batch_t* b, uint32_t options, double* ms,
@@ -1872,6 +1876,7 @@ extern "C" void uk_batch_set_assoc_ws(ukhip_batch* b, void* p, size_t bytes) {
   b->d_assoc = p;
   b->assoc_bytes = bytes;
 }
+extern "C" std::shared_ptr<void>* uk_batch_assoc_plan(ukhip_batch* b) { return &b->assoc_plan; }
 /* the level-0 chain buffers, which hold the whitened steps of the batch (B
  * and D stored in full), with the level-0 observation slots: ld mr0 and m0[s]
  * rows per step */
@@ -1929,7 +1934,7 @@ static bool smooth_equations(kalman_options_t options, kalman_step_equations_t**
   staging_free(st);
   if (!b) return false;
   const int cov = associative ? 1 : ((options & KALMAN_NO_COVARIANCE) == 0);
-  int rc = associative ? uk_assoc_smooth(b, options) : (run_oddeven(b, cov, nullptr, g_stream) ? 0 : -1);
+  int rc = associative ? uk_assoc_smooth(b, options, g_stream) : (run_oddeven(b, cov, nullptr, g_stream) ? 0 : -1);
   if (rc != 0) {
     batch_release(b);
     return false;
@@ -3004,7 +3009,7 @@ extern "C" int uk_ingest_smooth(uk_ingest* g, uint32_t options) {
             up(st.offKt, &g->Kt[j0], S) && up(st.offCt, &g->Ct[j0], S) && up(st.offm, &g->m[j0], S * 4) &&
             up(st.offfirst, first.data(), S);
   const int cov = assoc ? 1 : ((options & KALMAN_NO_COVARIANCE) == 0);
-  if (ok) ok = assoc ? uk_assoc_smooth(b, options) == 0 : run_oddeven(b, cov, nullptr, g_stream);
+  if (ok) ok = assoc ? uk_assoc_smooth(b, options, g_stream) == 0 : run_oddeven(b, cov, nullptr, g_stream);
   const bool wform = cov && (options & UKHIP_COVARIANCE_W) != 0;
   if (ok) ok = ukhip_batch_download(b, 0, &g->x[j0 * n], (cov && !wform) ? &g->S[j0 * nn] : nullptr) == 0;
   if (ok && wform) ok = ukhip_batch_download_cov(b, 0, 'W', &g->S[j0 * nn]) == 0;
