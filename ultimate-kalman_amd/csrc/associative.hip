@@ -427,36 +427,68 @@ __device__ __forceinline__ Sh<NT> sh(double* p) {
 }
 
 /* Lets the matrix products before it finish. The compiler places the wait
- * states between a product and the first read of its result, but it counts
- * them along one of the paths that lead there: where products are under a
- * condition, another path can be too short, and the read gets the sum without
- * its last term. So code with conditions on products ends with this. */
+ * states between a product and the first read of its result, but where
+ * branches follow the product it counts them along one of the paths to the
+ * read, another can be too short, and the read gets the sum without its last
+ * term. So a group of products ends with this, in the same block. */
 __device__ __forceinline__ void mfma_drain() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_nop 15\n\ts_nop 3");
   __builtin_amdgcn_sched_barrier(0);
 }
 
-/* Y += SGN P^T X over the first kk rows of P and X; LOWER: P is lower
- * triangular; rlo: X starts at tile row rlo; ihi: the last row of Y wanted */
+/* Y += SGN P^T X; LOWER: P is lower triangular. Over the whole order, or with
+ * kk >= 0 over the first kk rows of P and X (the rest is zeros) */
 template <int NT, int SGN = 1, bool LOWER = false>
-__device__ __forceinline__ void tmul(const Sh<NT>& P, const as_d4 (&X)[NT], as_d4 (&Y)[NT], int kk, const Who<NT>& me,
-                                     int rlo = 0, int ihi = NT - 1) {
+__device__ __forceinline__ void tmul(const Sh<NT>& P, const as_d4 (&X)[NT], as_d4 (&Y)[NT], const Who<NT>& me,
+                                     int kk = -1) {
+  auto rows = [&](int r) {
 #pragma unroll
-  for (int r = 0; r < NT; ++r) {
-    if (16 * r < kk && r >= rlo) {
+    for (int i = 0; i < NT; ++i) {
+      if (!LOWER || r >= i) {
+        const as_d4 p = P.tile(r, i, me);
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        if ((!LOWER || r >= i) && i <= ihi) {
-          const as_d4 p = P.tile(r, i, me);
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            if (NT > 1 || 4 * g < kk) Y[i] = as_mfma(SGN < 0 ? -p[g] : p[g], X[r][g], Y[i]);
-        }
+        for (int g = 0; g < 4; ++g) Y[i] = as_mfma(SGN < 0 ? -p[g] : p[g], X[r][g], Y[i]);
       }
     }
+  };
+  if (kk < 0) {
+#pragma unroll
+    for (int r = 0; r < NT; ++r) rows(r);
+    mfma_drain();
+  } else {
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+      if (16 * r < kk) {
+        rows(r);
+        mfma_drain();
+      }
   }
+}
+/* The same for one tile: as many of the four products as rows of P and X are
+ * not zeros (they are n here where the whole order is asked for) */
+template <int G, int SGN>
+__device__ __forceinline__ void tmul_rows(const as_d4& p, const as_d4& x, as_d4& y) {
+#pragma unroll
+  for (int g = 0; g < G; ++g) y = as_mfma(SGN < 0 ? -p[g] : p[g], x[g], y);
   mfma_drain();
+}
+template <int SGN>
+__device__ __forceinline__ void tmul_tile(const as_d4& p, const as_d4& x, as_d4& y, int kk) {
+  if (kk > 12) tmul_rows<4, SGN>(p, x, y);
+  else if (kk > 8) tmul_rows<3, SGN>(p, x, y);
+  else if (kk > 4) tmul_rows<2, SGN>(p, x, y);
+  else tmul_rows<1, SGN>(p, x, y);
+}
+template <int NT, int SGN = 1, bool LOWER = false>
+__device__ __forceinline__ void tmul_n(const Sh<NT>& P, const as_d4 (&X)[NT], as_d4 (&Y)[NT], int n, const Who<NT>& me) {
+  if constexpr (NT == 1) tmul_tile<SGN>(P.v, X[0], Y[0], n);
+  else tmul<NT, SGN, LOWER>(P, X, Y, me);
+}
+template <int NT, int SGN = 1>
+__device__ __forceinline__ void tmul_m(const Sh<NT>& P, const as_d4 (&X)[NT], as_d4 (&Y)[NT], int m, const Who<NT>& me) {
+  if constexpr (NT == 1) tmul_tile<SGN>(P.v, X[0], Y[0], m);
+  else tmul<NT, SGN>(P, X, Y, me, m);
 }
 template <int NT>
 __device__ __forceinline__ void zero(as_d4 (&X)[NT]) {
@@ -570,6 +602,19 @@ __device__ __forceinline__ void chol_forward(Lds<NT>& s, as_d4 (&M)[NT], int lim
         fl = fmax(2.2e-16 * rows_sum(d), 1e-290);
       }
   }
+  auto each = [&](auto f) {
+    f(R1);
+    if constexpr (!Geo<NT>::SEP || sizeof...(Rs) == 0) {
+      (f(Rs), ...);
+      mfma_drain();
+    } else {
+      mfma_drain();
+      if (me.mat) {
+        (f(Rs), ...);
+        mfma_drain();
+      }
+    }
+  };
 #pragma unroll
   for (int p = 0; p < NT; ++p) {
     as_d4 wt;
@@ -595,9 +640,7 @@ __device__ __forceinline__ void chol_forward(Lds<NT>& s, as_d4 (&M)[NT], int lim
 #pragma unroll
       for (int g = 0; g < 4; ++g) wt[g] = s.wt[g * 64 + me.lane];
     }
-    panel_solve<NT>(R1[p], wt);
-    if (me.mat) (panel_solve<NT>(Rs[p], wt), ...);
-    mfma_drain();
+    each([&](as_d4(&X)[NT]) { panel_solve<NT>(X[p], wt); });
     if (p + 1 < NT) {
       if (me.mat && me.w > p) {
         panel_solve<NT>(M[p], wt);
@@ -615,12 +658,11 @@ __device__ __forceinline__ void chol_forward(Lds<NT>& s, as_d4 (&M)[NT], int lim
 #pragma unroll
           for (int g = 0; g < 4; ++g) X[r] = as_mfma(t[g], X[p][g], X[r]);
         };
-        update(R1);
-        if (me.mat) {
-          (update(Rs), ...);
-          if (me.w >= r) update(M);
+        each(update);
+        if (me.mat && me.w >= r) {
+          update(M);
+          mfma_drain();
         }
-        mfma_drain();
       }
     }
   }
@@ -734,28 +776,28 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS) ka_prior(const AsProb* probs
       sync<NT>();
       zero<NT>(D);
       if (me.mat) {
-        tmul<NT>(b0, W, D, n, me); /* Y^T W */
-        tmul<NT>(b0, Y, Lm, n, me);
+        tmul_n<NT>(b0, W, D, n, me); /* Y^T W */
+        tmul_n<NT>(b0, Y, Lm, n, me);
         zero<NT>(M);
-        tmul<NT>(b1, W, M, n, me); /* Q^{-1} */
+        tmul_n<NT>(b1, W, M, n, me); /* Q^{-1} */
       }
       as_d4 ey[NT];
       zero<NT>(ey);
       if (me.vec) {
-        tmul<NT, -1>(b0, y, et, n, me);
-        tmul<NT>(b1, y, ey, n, me);
+        tmul_n<NT, -1>(b0, y, et, n, me);
+        tmul_n<NT>(b1, y, ey, n, me);
       }
       add_diag<NT>(Lm, n, 16 * NT, me);
       chol_forward<NT, false>(s, Lm, n, me, et, D);
       b0.put(D, me);
       sync<NT>();
       if (me.mat) {
-        tmul<NT, -1>(b0, D, M, n, me);
+        tmul_n<NT, -1>(b0, D, M, n, me);
 #pragma unroll
         for (int r = 0; r < NT; ++r) Lm[r] = M[r];
       }
       if (me.vec) {
-        tmul<NT>(b0, et, ey, n, me);
+        tmul_n<NT>(b0, et, ey, n, me);
 #pragma unroll
         for (int r = 0; r < NT; ++r) et[r] = ey[r];
       }
@@ -768,8 +810,8 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS) ka_prior(const AsProb* probs
       load_vec<NT>(o, wch.o + st * n, m, me);
       b0.put(C, me);
       sync<NT>();
-      if (me.mat) tmul<NT>(b0, C, Lm, m, me);
-      if (me.vec) tmul<NT>(b0, o, et, m, me);
+      if (me.mat) tmul_m<NT>(b0, C, Lm, m, me);
+      if (me.vec) tmul_m<NT>(b0, o, et, m, me);
       sync<NT>();
     }
     if (t < pr.p) {
@@ -788,12 +830,12 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS) ka_prior(const AsProb* probs
   sync<NT>();
   if (me.mat) {
     zero<NT>(P);
-    tmul<NT>(b0, W, P, n, me);
+    tmul_n<NT>(b0, W, P, n, me);
     store<NT, true>(P, md.Pf + sp * nn, n, me);
   }
   if (me.vec) {
     zero<NT>(x);
-    tmul<NT>(b0, et, x, n, me);
+    tmul_n<NT>(b0, et, x, n, me);
     store_vec<NT>(x, md.xf + sp * n, n, me);
   }
 }
@@ -843,10 +885,10 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_felem(const
     sync<NT>();
     if (me.mat) {
       zero<NT>(U);
-      tmul<NT>(b1, Ft, U, n, me);
-      tmul<NT>(b0, U, Q, n, me);
+      tmul_n<NT>(b1, Ft, U, n, me);
+      tmul_n<NT>(b0, U, Q, n, me);
     }
-    if (me.vec) tmul<NT>(b0, x, w1, n, me);
+    if (me.vec) tmul_n<NT>(b0, x, w1, n, me);
     sync<NT>();
   }
   as_d4 J[NT], e[NT];
@@ -863,12 +905,12 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_felem(const
     zero<NT>(CF);
     zero<NT>(S);
     if (me.mat) {
-      tmul<NT>(b0, Q, CQ, n, me);
-      tmul<NT>(b0, F, CF, n, me);
+      tmul_n<NT>(b0, Q, CQ, n, me);
+      tmul_n<NT>(b0, F, CF, n, me);
       as_d4 U[NT];
       zero<NT>(U);
-      tmul<NT>(b1, Ct, U, n, me);               /* Q C^T */
-      tmul<NT>(b0, U, S, n, me, 0, me.w);       /* S = C Q C^T + I */
+      tmul_n<NT>(b1, Ct, U, n, me);               /* Q C^T */
+      tmul_n<NT>(b0, U, S, n, me);       /* S = C Q C^T + I */
       add_diag<NT>(S, 0, 16 * NT, me);
     }
     if (me.vec) { /* column 0: o - C w1, the others: o - C c */
@@ -877,20 +919,20 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_felem(const
       for (int r = 0; r < NT; ++r)
 #pragma unroll
         for (int g = 0; g < 4; ++g) x[r][g] = me.li == 0 ? double(w1[r][g]) : double(c[r][g]);
-      tmul<NT, -1>(b0, x, y, n, me);
+      tmul_n<NT, -1>(b0, x, y, n, me);
     }
     chol_forward<NT, false>(s, S, m, me, y, CQ, CF); /* CQ = Y_1, CF = Y_2 */
     b0.put(CQ, me);
     b1.put(CF, me);
     sync<NT>();
     if (me.mat) {
-      tmul<NT, -1>(b0, CQ, Q, m, me);           /* Z = Q - Y_1^T Y_1 */
-      if (!firstel) tmul<NT, -1>(b0, CF, F, m, me); /* A = F - Y_1^T Y_2 */
-      tmul<NT>(b1, CF, J, m, me);               /* J = Y_2^T Y_2 */
+      tmul_m<NT, -1>(b0, CQ, Q, m, me);           /* Z = Q - Y_1^T Y_1 */
+      if (!firstel) tmul_m<NT, -1>(b0, CF, F, m, me); /* A = F - Y_1^T Y_2 */
+      tmul_m<NT>(b1, CF, J, m, me);               /* J = Y_2^T Y_2 */
     }
     if (me.vec) {
-      tmul<NT>(b0, y, w1, m, me);               /* b = w1 + Y_1^T r (column 0) */
-      tmul<NT>(b1, y, e, m, me);                /* e = Y_2^T rc (column 1) */
+      tmul_m<NT>(b0, y, w1, m, me);               /* b = w1 + Y_1^T r (column 0) */
+      tmul_m<NT>(b1, y, e, m, me);                /* e = Y_2^T rc (column 1) */
       spread<1>(e);
     }
   }
@@ -955,13 +997,13 @@ __device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsEle
   sync<NT>();
   if (me.mat) {
     zero<NT>(T2);
-    tmul<NT>(b0, a.A, T2, n, me); /* J_j A_i */
+    tmul_n<NT>(b0, a.A, T2, n, me); /* J_j A_i */
   }
   if (me.vec) { /* column 0: e_j; the others: e_j - J_j b_i */
     as_d4 u[NT];
 #pragma unroll
     for (int r = 0; r < NT; ++r) u[r] = x[r];
-    tmul<NT, -1>(b0, a.b(), u, n, me);
+    tmul_n<NT, -1>(b0, a.b(), u, n, me);
 #pragma unroll
     for (int r = 0; r < NT; ++r)
 #pragma unroll
@@ -983,14 +1025,14 @@ __device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsEle
       if (r >= me.w) Lc[r] = b1.tile(r, me.w, me);
     }
     zero<NT>(T);
-    tmul<NT>(b0, Lc, T, n, me, me.w); /* J_j L */
+    tmul_n<NT>(b0, Lc, T, n, me); /* J_j L */
     zero<NT>(M);
-    tmul<NT, 1, true>(b1, T, M, n, me, 0, me.w);
+    tmul_n<NT, 1, true>(b1, T, M, n, me);
     add_diag<NT>(M, 0, 16 * NT, me);  /* N */
     zero<NT>(C2);
-    tmul<NT, 1, true>(b1, T2, C2, n, me);
+    tmul_n<NT, 1, true>(b1, T2, C2, n, me);
     zero<NT>(T);
-    tmul<NT, 1, true>(b1, B1, T, n, me);
+    tmul_n<NT, 1, true>(b1, B1, T, n, me);
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
       T2[r] = C2[r]; /* L^T J_j A_i */
@@ -1002,7 +1044,7 @@ __device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsEle
     for (int r = 0; r < NT; ++r)
 #pragma unroll
       for (int h = 0; h < 4; ++h) a.b()[r][h] = me.li == 0 ? double(a.b()[r][h]) : 0.0;
-    tmul<NT, 1, true>(b1, x, a.b(), n, me);
+    tmul_n<NT, 1, true>(b1, x, a.b(), n, me);
   }
   if constexpr (SEP) chol_forward<NT, false>(s, M, n, me, a.A, T2, B1); /* y_0 | y_1 and Y_1, Y_2, Y_b */
   else chol_forward<NT, false>(s, M, n, me, a.b(), a.A, T2, B1);
@@ -1013,17 +1055,17 @@ __device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsEle
   b1.put(a.A, me);
   sync<NT>();
   if (me.mat) {
-    tmul<NT>(b1, T2, a.J, n, me);
-    tmul<NT>(b0, B1, a.Z, n, me);
+    tmul_n<NT>(b1, T2, a.J, n, me);
+    tmul_n<NT>(b0, B1, a.Z, n, me);
 #pragma unroll
     for (int r = 0; r < NT; ++r) T2[r] = a.A[r];
   }
   if (me.vec) {
-    tmul<NT>(b0, a.b(), bn, n, me);
+    tmul_n<NT>(b0, a.b(), bn, n, me);
     spread<0>(bn);
     as_d4 y1[NT];
     zero<NT>(y1);
-    tmul<NT>(b1, a.b(), y1, n, me);
+    tmul_n<NT>(b1, a.b(), y1, n, me);
     spread<1>(y1);
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
@@ -1033,7 +1075,7 @@ __device__ __forceinline__ void filt_combine(Acc<NT>& a, Lds<NT>& s, const AsEle
   }
   if (me.mat) {
     zero<NT>(a.A);
-    tmul<NT>(b0, T2, a.A, n, me);
+    tmul_n<NT>(b0, T2, a.A, n, me);
   }
   sync<NT>();
 }
@@ -1057,10 +1099,10 @@ __device__ __forceinline__ void smooth_combine(Acc<NT>& a, Lds<NT>& s, const AsE
   if (me.mat) {
     as_d4 U[NT];
     zero<NT>(U);
-    tmul<NT>(b1, Et, U, n, me); /* L_i E_j^T */
-    tmul<NT>(b0, U, Lj, n, me);
+    tmul_n<NT>(b1, Et, U, n, me); /* L_i E_j^T */
+    tmul_n<NT>(b0, U, Lj, n, me);
     zero<NT>(U);
-    tmul<NT>(b0, a.A, U, n, me);
+    tmul_n<NT>(b0, a.A, U, n, me);
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
       a.Z[r] = Lj[r];
@@ -1068,7 +1110,7 @@ __device__ __forceinline__ void smooth_combine(Acc<NT>& a, Lds<NT>& s, const AsE
     }
   }
   if (me.vec) {
-    tmul<NT>(b0, a.b(), gj, n, me);
+    tmul_n<NT>(b0, a.b(), gj, n, me);
 #pragma unroll
     for (int r = 0; r < NT; ++r) a.b()[r] = gj[r];
   }
@@ -1239,26 +1281,26 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_selem(const
     sync<NT>();
     zero<NT>(Y);
     if (me.mat) {
-      tmul<NT>(b0, P, Y, n, me);              /* Y = F P */
+      tmul_n<NT>(b0, P, Y, n, me);              /* Y = F P */
       as_d4 U[NT];
       zero<NT>(U);
-      tmul<NT>(b1, D, U, n, me);              /* U = P F^T */
-      tmul<NT>(b0, U, M, n, me, 0, me.w);     /* M = F P F^T + Q = G G^T */
+      tmul_n<NT>(b1, D, U, n, me);              /* U = P F^T */
+      tmul_n<NT>(b0, U, M, n, me);     /* M = F P F^T + Q = G G^T */
     }
-    if (me.vec) tmul<NT>(b0, x, y, n, me);    /* y = F x + c */
+    if (me.vec) tmul_n<NT>(b0, x, y, n, me);    /* y = F x + c */
     add_diag<NT>(M, n, 16 * NT, me);
     chol_forward<NT, false>(s, M, n, me, y, Y, W); /* Y = G^{-1} F P, W = G^{-1}, y = G^{-1} (F x + c) */
     b0.put(Y, me);
     sync<NT>();
     if (me.mat) {
       zero<NT>(D);
-      tmul<NT>(b0, W, D, n, me);
+      tmul_n<NT>(b0, W, D, n, me);
       store<NT, false>(D, E, n, me);          /* E = Y^T W */
-      tmul<NT, -1>(b0, Y, P, n, me);
+      tmul_n<NT, -1>(b0, Y, P, n, me);
       store<NT, true>(P, Lo, n, me);          /* L = P - Y^T Y */
     }
     if (me.vec) {
-      tmul<NT, -1>(b0, y, x, n, me);
+      tmul_n<NT, -1>(b0, y, x, n, me);
       store_vec<NT>(x, gv, n, me);            /* g = x - E (F x + c) */
     }
   } else {
@@ -1270,10 +1312,10 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_selem(const
     b0.put(Y, me);
     sync<NT>();
     if (me.mat) {
-      tmul<NT>(b0, W, D, n, me);              /* D = F^T Q^{-1} */
-      tmul<NT>(b0, Y, P, n, me);              /* P = Lam + F^T Q^{-1} F = H H^T */
+      tmul_n<NT>(b0, W, D, n, me);              /* D = F^T Q^{-1} */
+      tmul_n<NT>(b0, Y, P, n, me);              /* P = Lam + F^T Q^{-1} F = H H^T */
     }
-    if (me.vec) tmul<NT, -1>(b0, y, x, n, me); /* x = eta - F^T Q^{-1} c */
+    if (me.vec) tmul_n<NT, -1>(b0, y, x, n, me); /* x = eta - F^T Q^{-1} c */
     add_diag<NT>(P, n, 16 * NT, me);
     zero<NT>(W);
     add_diag<NT>(W, 0, n, me);
@@ -1282,15 +1324,15 @@ __global__ void __launch_bounds__(Geo<NT>::THREADS, SCAN_OCC<NT>) ka_selem(const
     sync<NT>();
     if (me.mat) {
       zero<NT>(M);
-      tmul<NT>(b0, W, M, n, me);
+      tmul_n<NT>(b0, W, M, n, me);
       store<NT, true>(M, Lo, n, me);          /* L = W^T W */
       zero<NT>(M);
-      tmul<NT>(b0, D, M, n, me);
+      tmul_n<NT>(b0, D, M, n, me);
       store<NT, false>(M, E, n, me);          /* E = L F^T Q^{-1} */
     }
     if (me.vec) {
       zero<NT>(y);
-      tmul<NT>(b0, x, y, n, me);
+      tmul_n<NT>(b0, x, y, n, me);
       store_vec<NT>(y, gv, n, me);            /* g = L x */
     }
   }
