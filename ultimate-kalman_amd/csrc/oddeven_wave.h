@@ -69,6 +69,30 @@ __host__ __device__ constexpr bool sm_need(int l, int NK, int G, int QF) {
 /* rows of a block that QF_HALF0 / QF_HALF1 keep */
 __host__ __device__ constexpr int sm_half_rows(int NK) { return 4 * ((NK + 1) / 2); }
 
+/* The scalars of a Householder step whose vector stays unscaled (the pivot
+ * column with ukk on its pivot row): H = I - f1 f2^2 x x^T. FP32 as FP64:
+ * rounded like exact operations, and 1 / (u^T u / 2) in one piece: with the
+ * product of tau and two rounded reciprocals of ukk the mixed path's estimates
+ * were further off, 1.40 times at n = 4 and 1.30 at n = 32 (k = 3000, one
+ * refinement). f2 is a power of two that keeps squares in range. */
+__device__ __forceinline__ void wave_scalars(double alpha, double s, double& ukk, double& f1, double& f2) {
+  house_scalars(alpha, s, ukk, f1, f2);
+}
+__device__ __forceinline__ void wave_scalars(float alpha, float s, float& ukk, float& f1, float& f2) {
+  const float t2 = fmaf(alpha, alpha, s);
+  const bool tiny = t2 < 1e-28f, big = t2 > 1e28f;
+  f2 = tiny ? 0x1p32f : big ? 0x1p-32f : 1.0f;
+  const float a = alpha * f2, t = t2 * f2 * f2, aa = fabsf(a);
+  const float y = __builtin_amdgcn_rsqf(t), h = 0.5f * y;
+  float g = t * y;
+  float w = __builtin_amdgcn_rcpf(fmaf(aa, g, t));
+  g = fmaf(fmaf(-g, g, t), h, g); /* sqrt(t) */
+  const float v = fmaf(aa, g, t);
+  w = fmaf(fmaf(-v, w, 1.0f), w, w);
+  ukk = alpha + copysignf(g * (tiny ? 0x1p-32f : big ? 0x1p32f : 1.0f), alpha);
+  f1 = s != 0.0f ? w : 0.0f;
+}
+
 /* One Householder step: pivot column K (tile K / 16, lane K % 16), target row
  * K, applied to tiles K / 16 .. TILES - 1 and, on the first step of a pivot
  * tile, to the right-hand side where it is (e before step 0, lane li = 0 of
@@ -100,7 +124,7 @@ __device__ __forceinline__ void sm_step(T (&a)[TILES][2 * NK], T (&e)[2 * NK], i
       if (l != G && sm_need(l, NK, G, QF)) d[t][l & 1] = fma(x[l], c[l], d[t][l & 1]);
   }
   T ukk, f1, f2;
-  house_scalars(alpha, s, ukk, f1, f2);
+  wave_scalars(alpha, s, ukk, f1, f2);
   const bool none = f1 == T(0);
   ukk = none ? T(0) : T(ukk);
   if (sizeof(T) == 4) f2 = none ? T(0) : T(f2);
