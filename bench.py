@@ -113,9 +113,9 @@ def kernel_label(slot, n, m, fp32=False, cov=True, all_w=True, h_ident=True, lev
     if slot == "k_weigh":
         return "k_weigh_diag<" + ("true" if fp32 else "false") + ">" if all_w else f"k_weigh<{bucket(max(n, m))}>"
     if slot == "k_backsub":
-        if nb >= 32:
-            return f"k_backsub_mfma<{nb}>" if cov else f"k_estimate<{nb}>"
-        return f"k_backsub<{nb}>"
+        if not cov:
+            return f"k_estimate<{nb}>"
+        return f"k_backsub_mfma<{nb}>" if nb >= 32 else f"k_backsub_small<{(n + 3) // 4}, *>"
     if slot == "k_solve_est":
         return f"k_solve_est<{nq}, {T}, *>"
     if slot == "k_normal":
@@ -126,11 +126,12 @@ def kernel_label(slot, n, m, fp32=False, cov=True, all_w=True, h_ident=True, lev
     if slot == "convert":
         return "k_to32 / k_to64"
     phase = int(slot[-1])
-    if nq >= 24:
-        v = device.launch_table()[f"phase{phase}<{nq}, {T}>"]
-        cpl, wg = int(v[1]), int(v[3])
-    else:
-        cpl, wg = 1, 0
+    if nb <= 16:  # the three phases of a level in one launch, timed as phase 1
+        return f"k_level_small<{(n + 3) // 4}, {T}, *>"
+    if nb == 32:  # phase 1's slot also holds k_mid_level, the short levels
+        return f"k_mid{phase}<{(n + 3) // 4}, {T}, *>"
+    v = device.launch_table()[f"phase{phase}<{nq}, {T}>"]
+    cpl, wg = int(v[1]), int(v[3])
     if cpl == 0:
         return f"k_phase2_wy<{nq}, {T}, *>"
     return f"{slot}<{nq}, {T}, {wg}, {cpl}, *>"
@@ -315,7 +316,8 @@ def accumulate_parts(b, ch, R, kern):
             slot_ms[key] = slot_ms.get(key, 0.0) + ms[slot]
             slot_launch[key] = slot_launch.get(key, 0) + nl[slot]
             if slot.startswith("k_phase"):
-                slot_flops[key] = slot_flops.get(key, 0.0) + fps["phase" + slot[-1]] * kpart
+                done = "123" if n_ <= 16 else slot[-1]  # phases that the slot's launches do
+                slot_flops[key] = slot_flops.get(key, 0.0) + sum(fps["phase" + ph] for ph in done) * kpart
             rb = refine_bytes_per_step(n_, m_, slot)
             if rb is not None:  # k_solve_est also forms the first estimates: R + 1 sweeps
                 slot_bytes[key] = slot_bytes.get(key, 0.0) + rb * kpart * (R + (slot == "k_solve_est"))
@@ -657,9 +659,9 @@ def run_long(args):
         cls = [c for c in device.AS_KERNELS if c != "total"]
         adom = max(cls, key=lambda c: ams_k[c])
         a_ach = afl[adom] / (ams_k[adom] * 1e-3) / 1e12
-        names = {"fscan": "ka_scan_reduce/round/down<48, true>", "sscan": "ka_scan_reduce/round/down<48, false>",
-                 "felem": "ka_felem<48>", "selem": "ka_selem<48>", "model": "ka_model<48>", "prior": "ka_prior<48>",
-                 "filtered": "ka_filtered", "results": "ka_results", "weigh": "k_weigh<48>"}
+        names = {"fscan": "ka_scan_reduce/round/down<3, true>", "sscan": "ka_scan_reduce/round/down<3, false>",
+                 "felem": "ka_felem<3>", "selem": "ka_selem<3>", "model": "ka_model_diag", "prior": "ka_prior<3>",
+                 "filtered": "ka_filtered", "results": "ka_results", "weigh": "k_weigh_diag<false>"}
         out["associative"] = {
             "algorithm": "associative scan (Saerkkae-Garcia-Fernandez), FP64, with covariances",
             "ms_per_step": ams, "value": pr.k / (ams * 1e-3), "unit": "timesteps/s", "steps": args.assoc_steps,
@@ -667,7 +669,7 @@ def run_long(args):
             "max_rel_err_covdiag_vs_oddeven": step_rel_err(np.einsum("kii->ki", Sa), d64),
             "kernels_ms_per_step": {c: ams_k[c] for c in device.AS_KERNELS},
             "kernels_tflops": {c: afl[c] / (ams_k[c] * 1e-3) / 1e12 for c in cls if afl[c] > 0 and ams_k[c] > 0},
-            "roofline": {"bound": "valu", "kernel": names[adom], "achieved": a_ach, "peak": FP64_PEAK_TFLOPS,
+            "roofline": {"bound": "mfma", "kernel": names[adom], "achieved": a_ach, "peak": FP64_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": a_ach / FP64_PEAK_TFLOPS, "traffic": None,
                          "algorithmic_flops_per_step": afl[adom], "launches_per_step": anl[adom],
                          "kernel_ms_per_step": ams_k[adom], "avg_launch_ms": ams_k[adom] / max(anl[adom], 1),

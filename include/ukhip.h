@@ -63,7 +63,7 @@ int ukhip_batch_smooth_oddeven(ukhip_batch_t* b, uint32_t options);
  * a captured graph (default 1). */
 void ukhip_use_graphs(int enable);
 /* 1 (default): the covariance back substitution for n > 16 runs its products on
- * the FP64 matrix cores; 0: on the vector units, as for n <= 16. Applies to
+ * the FP64 matrix cores; 0: on the vector units (n <= 16 has one form). Applies to
  * launches and graph captures made afterwards. */
 void ukhip_use_mfma(int enable);
 /* Launch table of the odd-even QR phase kernels (phase 1..3) for state
@@ -74,7 +74,8 @@ void ukhip_use_mfma(int enable);
  * CU the register allocation leaves room for: 1, 2 or 4 with one column per
  * group, 2, 3 or 4 with two, 2 or 3 with three; columns_per_group 0 (phase 2,
  * buckets 32, 48, 64, one workgroup per CU) is the blocked-WY phase 2 on the
- * matrix cores. The buckets are n in 17..24, 25..32, 33..48 and 49..64.
+ * matrix cores. The buckets are n in 17..24, 25..32, 33..48 and 49..64; the
+ * first two hold what is set, but n <= 32 has one form and reads nothing here.
  * ukhip_autotune times every variant on a synthetic problem of k steps (0:
  * 4096) per bucket up to n_max and keeps the fastest; the register variants
  * run the same operations on every column, so choosing among them does not

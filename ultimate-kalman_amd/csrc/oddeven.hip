@@ -6,22 +6,17 @@
  * :614-975, recursion :1358-1553, weighing :1620-1659) and
  * matlab/KalmanOddevenSmoother.m:21-358.
  *
- * k_weigh      whitening of one step per workgroup (c/kalman_base.c:61-175).
- * k_phase1..3  the reference's three elimination phases of one level, one
- *              workgroup per step pair (or even step), writing the
- *              back-substitution factors and the next level's chain
- *              (oddeven_qr.h; the buckets above 16 are compiled in
- *              oddeven_qr{32,48,64}.hip).
- * k_backsub    one workgroup per even step: estimate and, optionally, the
- *              selected-inversion covariance and the two cross covariances.
- *
- * Register layout of the QR kernels: every matrix column is owned by SL = 2
- * or 4 adjacent lanes. The column has two row blocks of NB rows (block 0 holds
- * the pivot rows, block 1 the stacked rows); sub-lane b holds the rows
- * r = b (mod SL) of both blocks, 2 NB / SL doubles. A Householder reflector is
- * published through double-buffered LDS by the pivot column's lanes; every
- * other lane runs branch-free loops over its rows (no dynamic register
- * indexing), combining its partial dot products with DPP quad permutations.
+ * k_weigh         whitening of one step per workgroup (c/kalman_base.c:61-175),
+ *                 k_weigh_diag for inverse standard deviations.
+ * The reference's three elimination phases of one level, which write the
+ * back-substitution factors and the next level's chain, are in
+ *   oddeven_small.hip      n <= 16, one launch a level, a wave per step pair,
+ *   oddeven_mid{20..32}    n <= 32, the same by phases or, for short levels, in
+ *                          one launch with a workgroup per step pair,
+ *   oddeven_qr{48,64}.hip  n <= 64, a workgroup per step pair and phase.
+ * k_backsub_small, k_backsub_mfma, k_estimate, k_backsub
+ *                 estimates and, except k_estimate, the selected-inversion
+ *                 covariances of a level's even steps.
  *
  * Rows that are zero in every column stay zero under all reflectors (their
  * reflector entries are zero), so padding blocks with zero rows yields an
@@ -1451,10 +1446,10 @@ extern "C" int uk_bucket(int n) {
   if (n <= 64) return 64;
   return -1;
 }
-/* The elimination's and the refinement sweeps' buckets: uk_bucket's, and 24
- * for 16 < n <= 24 (three quarters of bucket 32's rows and lanes). The other
- * kernels keep uk_bucket's; every bucket serves any n up to its size on the
- * same layouts (blocks stored n x n). */
+/* The refinement sweeps' buckets: uk_bucket's, and 24 for 16 < n <= 24 (three
+ * quarters of bucket 32's rows and lanes). The other kernels keep uk_bucket's;
+ * every bucket serves any n up to its size on the same layouts (blocks stored
+ * n x n). */
 extern "C" int uk_bucket_qr(int n) {
   if (n > 16 && n <= 24) return 24;
   return uk_bucket(n);
@@ -1533,12 +1528,13 @@ extern "C" hipError_t uk_launch_weigh_f32(const uk_raw_t* raw, const uk_chain_t*
   return hipGetLastError();
 }
 
-/* Run-time launch table of the phase kernels at NB >= 24 (FP64, and the FP32
+/* Run-time launch table of the phase kernels at n > 32 (FP64, and the FP32
  * elimination of the mixed-precision path), per precision, phase and bucket
  * (32, 48, 64, 24): the columns each lane group holds (cpl) and the workgroups per
  * CU asked of the register allocator (wg). Starts from variants measured
- * fastest on MI355X (n = 24, 32, 48 and 64, k = 200000), rewritten by
- * ukhip_autotune. */
+ * fastest on MI355X (n = 48 and 64, k = 200000), rewritten by ukhip_autotune.
+ * The entries of buckets 24 and 32 are kept as callers set them, but no kernel
+ * reads them: n <= 32 has one form. */
 struct QrLaunch {
   int cpl, wg;
 };
@@ -1668,7 +1664,7 @@ extern "C" hipError_t uk_launch_eliminate32(const uk_level_t* lv, const uk_chain
 }
 
 /* Back substitution with covariances for n > 16 on the matrix cores (default)
- * or on the vector units (k_backsub, the kernel used for n <= 16). cov: 0
+ * or on the vector units (k_backsub). cov: 0
  * estimates only, 1 covariances, 2 only the covariances' diagonals (written
  * in their places; for level 0, whose covariances no other level reads). */
 static int g_backsub_mfma = 1;

@@ -1,8 +1,9 @@
 /*
- * oddeven_qr.h -- the QR kernels of the odd-even elimination (phases 1..3),
- * shared by oddeven.hip (n <= 16, and the device helpers its other kernels
- * use) and oddeven_qr{24,32,48,64}.hip (one translation unit per bucket above
- * 16, so that their many launch variants compile in parallel).
+ * oddeven_qr.h -- the QR kernels of the odd-even elimination (phases 1..3) for
+ * 32 < n <= 64 (oddeven_qr{48,64}.hip, one translation unit per bucket, so that
+ * their many launch variants compile in parallel), and the device helpers that
+ * the other kernels of oddeven.hip use in every bucket. Smaller n:
+ * oddeven_wave.h.
  *
  * Reference: c/kalman_oddeven_smoother.c (phases :379-560, fix-last
  * :1452-1476, renaming :563-597).
@@ -287,8 +288,7 @@ __device__ __forceinline__ void block_zero(T* __restrict__ dst, int64_t nn, int 
 
 /* LDS reflector buffers: [buffer][sub][2H + 4] (the +4 skews the sub-lane
  * arrays onto different banks), then the tau of each buffer. A stride that
- * lands on bank 0 or 16 of the 32 four-byte banks (2H + 4 = 16 in bucket 24)
- * would put two sub-lanes' reads on the same banks: it is padded by 4 more. */
+ * lands on bank 0 or 16 of the 32 four-byte banks would put two sub-lanes' reads on the same banks: it is padded by 4 more. */
 template <int NB, int SL, class T = double>
 struct Refl {
   static constexpr int SUBSTRIDE0 = 2 * (NB / SL) + 4;
@@ -351,10 +351,10 @@ __host__ __device__ constexpr int qr_chunk(int nl, int cap) {
 enum { QF_TRI1 = 1, QF_DONE = 2, QF_HALF0 = 4, QF_HALF1 = 8, QF_DIAG0 = 16, QF_SWAP = 32 };
 __host__ __device__ constexpr int qr_gl(int H) { return H <= 16 ? 2 : 4; }
 /* the granules of a block that QF_HALF0 / QF_HALF1 keep: the first half,
- * rounded up (bucket 24: 2 of 3) */
+ * rounded up */
 __host__ __device__ constexpr int qr_half_granules(int H) { return (H / qr_gl(H) + 1) / 2; }
 /* rows of a block that QF_HALF0 / QF_HALF1 keep for bucket NB with SL lanes
- * per column (NB / 2, and 16 in bucket 24) */
+ * per column */
 __host__ __device__ constexpr int qr_half_rows(int NB, int SL) {
   return qr_half_granules(NB / SL) * qr_gl(NB / SL) * SL;
 }
@@ -713,7 +713,7 @@ __device__ __forceinline__ Col<NB, SL, T> swap_col0(T r00, int sub) {
  * R1 = 2n right-hand side, Bl = [2n+1,3n+1) u_{j-1}.
  */
 /* LV: the level's stacked rows (C) as structure: 0 dense, 1 at most
- * qr_half_rows rows (level 0 with m <= NB / 2; 16 in bucket 24), 2 upper
+ * qr_half_rows rows (level 0 with m <= NB / 2), 2 upper
  * triangular (the levels above 0) */
 template <int NB, class T, int WG = 0, int CPL = 1, int LV = 0>
 __global__ void __launch_bounds__((QRGeom<NB, 2 * NB + 1, 1, WG, CPL, true>::NT),
@@ -1431,36 +1431,29 @@ void phases_nb(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, 
 template <int NB, class T>
 void phase_launch_impl(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac, T* fix,
                        int n, hipStream_t st, int phase, ukqr::Launch v) {
-  if constexpr (NB >= 24) {
-    if constexpr (NB % 16 == 0) {
-      if (v.cpl == 0 && phase == 2) { /* blocked WY on the matrix cores */
-        const dim3 g((unsigned)lv->evens), b(WyGeom<NB>::NT);
-        if (in.d_diag) k_phase2_wy<NB, T, true><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
-        else k_phase2_wy<NB, T, false><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
-        return;
-      }
+  if (v.cpl == 0 && phase == 2) { /* blocked WY on the matrix cores */
+    const dim3 g((unsigned)lv->evens), b(WyGeom<NB>::NT);
+    if (in.d_diag) k_phase2_wy<NB, T, true><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
+    else k_phase2_wy<NB, T, false><<<g, b, 0, st>>>(*lv, in, out, fac, fix, n);
+    return;
+  }
+  if (v.cpl == 3) {
+    switch (v.wg) {
+      case 2: phases_nb<NB, T, 2, 3>(lv, in, out, fac, fix, n, st, phase); break;
+      default: phases_nb<NB, T, 3, 3>(lv, in, out, fac, fix, n, st, phase); break;
     }
-    if (v.cpl == 3) {
-      switch (v.wg) {
-        case 2: phases_nb<NB, T, 2, 3>(lv, in, out, fac, fix, n, st, phase); break;
-        default: phases_nb<NB, T, 3, 3>(lv, in, out, fac, fix, n, st, phase); break;
-      }
-    } else if (v.cpl == 2) {
-      switch (v.wg) {
-        case 2: phases_nb<NB, T, 2, 2>(lv, in, out, fac, fix, n, st, phase); break;
-        case 3: phases_nb<NB, T, 3, 2>(lv, in, out, fac, fix, n, st, phase); break;
-        default: phases_nb<NB, T, 4, 2>(lv, in, out, fac, fix, n, st, phase); break;
-      }
-    } else {
-      switch (v.wg) {
-        case 1: phases_nb<NB, T, 1, 1>(lv, in, out, fac, fix, n, st, phase); break;
-        case 2: phases_nb<NB, T, 2, 1>(lv, in, out, fac, fix, n, st, phase); break;
-        default: phases_nb<NB, T, 4, 1>(lv, in, out, fac, fix, n, st, phase); break;
-      }
+  } else if (v.cpl == 2) {
+    switch (v.wg) {
+      case 2: phases_nb<NB, T, 2, 2>(lv, in, out, fac, fix, n, st, phase); break;
+      case 3: phases_nb<NB, T, 3, 2>(lv, in, out, fac, fix, n, st, phase); break;
+      default: phases_nb<NB, T, 4, 2>(lv, in, out, fac, fix, n, st, phase); break;
     }
   } else {
-    (void)v;
-    phases_nb<NB, T, 0, 1>(lv, in, out, fac, fix, n, st, phase);
+    switch (v.wg) {
+      case 1: phases_nb<NB, T, 1, 1>(lv, in, out, fac, fix, n, st, phase); break;
+      case 2: phases_nb<NB, T, 2, 1>(lv, in, out, fac, fix, n, st, phase); break;
+      default: phases_nb<NB, T, 4, 1>(lv, in, out, fac, fix, n, st, phase); break;
+    }
   }
 }
 }  // namespace

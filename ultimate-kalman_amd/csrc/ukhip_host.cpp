@@ -3109,7 +3109,7 @@ extern "C" void uk_ingest_rollback(uk_ingest* g, int64_t si) {
 
 
 
-/* For every bucket (24, 32, 48, 64) up to n_max: a synthetic problem (n = bucket,
+/* For the buckets 48 and 64 up to n_max: a synthetic problem (n = bucket,
  * m = n/2, k steps, F = 0.98 times a Householder reflection, G uniform with
  * variance 1/n, 'w' covariances) is smoothed with each phase kernel in each
  * of its launch variants (1, 2, 4 workgroups per CU asked of the register
@@ -3127,8 +3127,8 @@ extern "C" int ukhip_autotune(int32_t n_max, int32_t k) {
     st ^= st >> 12; st ^= st << 25; st ^= st >> 27;
     return (double)((st * 0x2545F4914F6CDD1Dull) >> 11) * (2.0 / 9007199254740992.0) - 1.0;
   };
-  for (int nb : {24, 32, 48, 64}) {
-    if (nb > std::max(32, (int)n_max)) break;
+  for (int nb : {48, 64}) { /* n <= 32 has one form */
+    if (nb > (int)n_max) break;
     const int n = nb, m = nb / 2;
     const size_t nn = (size_t)n * n;
     std::vector<double> v(n), F(nn), K(n, 1.0), G((size_t)k * m * n), o((size_t)k * m), C((size_t)m, 1.0 / std::sqrt(0.1));
