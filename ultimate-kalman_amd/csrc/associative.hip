@@ -64,14 +64,6 @@ __device__ __forceinline__ double at(const double* A, int ld, bool t, int i, int
   return t ? A[k + (int64_t)i * ld] : A[i + (int64_t)k * ld];
 }
 
-typedef double as_d4 __attribute__((ext_vector_type(4)));
-/* D = A B + C on 16 x 16 x 4: lane (li, lk) supplies A[li][lk] and B[lk][li];
- * element r of the accumulator is D[4 r + lk][li]. So an accumulator is the
- * next product's B as it stands, and its transpose's A. */
-__device__ __forceinline__ as_d4 as_mfma(double a, double b, as_d4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 /* C (m x q, ld ldc) = alpha op(A) op(B) + beta C with op(A) m x kk and
  * op(B) kk x q, on the matrix cores: the waves deal the 16 x 16 tiles of C
  * between them. Indices are clamped into range (rows and columns beyond C are
@@ -272,55 +264,6 @@ __device__ double* inverse(const double* A, double* W1, double* W2, int ld, int 
   return gj_inverse<NB>(W1, W2, ld, n, g);
 }
 
-/*
- * One step of the Cholesky factorization of a symmetric positive definite 16 x
- * 16 tile on one wave (accumulator layout): a is reduced to D L^T (row K final
- * at step K), wt becomes the transposed inverse of the unit lower factor. The
- * pivots are kept by row (pr) and by column (pc). FLOOR: a pivot below fl (lane
- * li: of row li), the rounding error of its original diagonal entry, counts as
- * that error, so that a semidefinite matrix has a factor too (a perturbation
- * of the size of the matrix's own rounding); NaN stays NaN.
- */
-template <int K, bool FLOOR>
-__device__ __forceinline__ void chol_step(double (&a)[4], double (&wt)[4], double (&pr)[4], double& pc, double fl,
-                                          int li, int lk) {
-  constexpr int G = K / 4, KR = K % 4;
-  double x[4];
-#pragma unroll
-  for (int g = G; g < 4; ++g) x[g] = row_lane<K>(a[g]);
-  double p = one_lane(x[G], 16 * KR);
-  if (FLOOR) {
-    const double f = one_lane(fl, K);
-    p = p < f ? f : p;
-  }
-  double rp = __builtin_amdgcn_rcp(p);
-  rp = fma(fma(-p, rp, 1.0), rp, rp);
-  rp = fma(fma(-p, rp, 1.0), rp, rp);
-  const double row = rows_sum(lk == KR ? a[G] : 0.0) * rp; /* row K over the pivot, on every lane row */
-  x[G] = lk > KR ? x[G] : 0.0;
-#pragma unroll
-  for (int g = G; g < 4; ++g) a[g] = fma(-x[g], row, a[g]);
-  const double m = li > K ? row : 0.0;
-#pragma unroll
-  for (int g = 0; g <= G; ++g) wt[g] = fma(-row_lane<K>(wt[g]), m, wt[g]);
-  pr[G] = lk == KR ? p : pr[G];
-  pc = li == K ? p : pc;
-}
-template <bool FLOOR, int... K>
-__device__ __forceinline__ void chol_steps(double (&a)[4], double (&wt)[4], double (&pr)[4], double& pc,
-                                           double fl, int lim, int li, int lk,
-                                           std::integer_sequence<int, K...>) {
-  auto one = [&](auto k) {
-    if (k.value < lim) chol_step<k.value, FLOOR>(a, wt, pr, pc, fl, li, lk);
-  };
-  (one(std::integral_constant<int, K>{}), ...);
-}
-__device__ __forceinline__ double rsqrt_ulp(double p) {
-  const double y = __builtin_amdgcn_rsq(p);
-  const double y1 = fma(0.5 * y, fma(-p * y, y, 1.0), y);
-  return fma(0.5 * y1, fma(-p * y1, y1, 1.0), y1);
-}
-
 /* ------------------------------------------------------------------------ */
 /* tile columns                                                              */
 /* ------------------------------------------------------------------------ */
@@ -424,17 +367,6 @@ __device__ __forceinline__ Sh<NT> sh(double* p) {
   Sh<NT> s;
   if constexpr (NT > 1) s.p = p;
   return s;
-}
-
-/* Lets the matrix products before it finish. The compiler places the wait
- * states between a product and the first read of its result, but where
- * branches follow the product it counts them along one of the paths to the
- * read, another can be too short, and the read gets the sum without its last
- * term. So a group of products ends with this, in the same block. */
-__device__ __forceinline__ void mfma_drain() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 15\n\ts_nop 3");
-  __builtin_amdgcn_sched_barrier(0);
 }
 
 /* Y += SGN P^T X; LOWER: P is lower triangular. Over the whole order, or with

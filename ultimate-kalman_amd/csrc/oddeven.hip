@@ -25,7 +25,7 @@
  */
 #include <hip/hip_runtime.h>
 
-#include "oddeven_qr.h"
+#include "oddeven_wave.h"
 #include "ukhip_internal.h"
 
 namespace {
@@ -916,31 +916,80 @@ template <int NB>
 struct WeighShared {
   double K[NB * NB];
   double C[NB * NB];
+  double rk[NB], rc[NB]; /* reciprocals of a triangular K's and C's diagonal */
 };
 
-/* In-place lower Cholesky of an m x m matrix (ld m) in LDS, whole block. */
-template <int NT>
-__device__ void lds_cholesky(double* A, int m, int tid) {
-  for (int jj = 0; jj < m; ++jj) {
-    if (tid == 0) A[jj + jj * m] = sqrt(A[jj + jj * m]);
-    __syncthreads();
-    const double d = A[jj + jj * m];
-    for (int i = jj + 1 + tid; i < m; i += NT) A[i + jj * m] /= d;
-    __syncthreads();
-    const int rem = m - jj - 1;
-    for (int idx = tid; idx < rem * rem; idx += NT) {
-      const int i = jj + 1 + idx % rem, kk = jj + 1 + idx / rem;
-      if (i >= kk) A[i + kk * m] -= A[i + jj * m] * A[kk + jj * m];
+/* In-place lower Cholesky of an m x m matrix (ld m) in LDS by one wave, the
+ * upper tiles in its registers: row tiles by the inverse factor of the panel's
+ * diagonal tile, the tiles below updated on the matrix cores; r: the
+ * reciprocals of the factor's diagonal. A column at a time by the workgroup,
+ * with three barriers, it was most of k_weigh: 209 us for
+ * 300 steps of n = 45 with full covariances, 89 now. */
+template <int NB>
+__device__ void wave_cholesky(double* A, double* r, int m, int lane) {
+  constexpr int NT = (NB + 15) / 16;
+  const int li = lane & 15, lk = lane >> 4;
+  as_d4 M[NT][NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = i; j < NT; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) { /* the transposes of A's lower tiles */
+        const int row = 16 * j + li, col = 16 * i + 4 * g + lk;
+        const bool in = row < m && col < m;
+        const double x = A[in ? (row >= col ? row + col * m : col + row * m) : 0];
+        M[i][j][g] = in ? x : (row == col ? 1.0 : 0.0);
+      }
+#pragma unroll
+  for (int p = 0; p < NT; ++p) {
+    double a[4], t[4], pr[4], pc = 1.0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      a[g] = M[p][p][g];
+      t[g] = 4 * g + lk == li ? 1.0 : 0.0;
+      pr[g] = 1.0;
     }
-    __syncthreads();
+    chol_steps<false>(a, t, pr, pc, 0.0, m - 16 * p, li, lk, std::make_integer_sequence<int, 16>{});
+    const double sc = rsqrt_ulp(pc);
+    if (lk == 0 && 16 * p + li < m) r[16 * p + li] = sc;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      M[p][p][g] = a[g] * rsqrt_ulp(pr[g]);
+      t[g] *= sc;
+    }
+#pragma unroll
+    for (int j = p + 1; j < NT; ++j) {
+      as_d4 y = as_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int g = 0; g < 4; ++g) y = as_mfma(t[g], M[p][j][g], y);
+      M[p][j] = y;
+    }
+#pragma unroll
+    for (int i = p + 1; i < NT; ++i)
+#pragma unroll
+      for (int j = i; j < NT; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) M[i][j] = as_mfma(-M[p][i][g], M[p][j][g], M[i][j]);
+    mfma_drain();
   }
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = i; j < NT; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int row = 16 * j + li, col = 16 * i + 4 * g + lk;
+        if (row < m && col <= row) A[row + col * m] = M[i][j][g];
+      }
 }
 
-/* x <- V x for a whitening V given as (code, matrix M in LDS, diag d);
- * src is x's column in global memory (re-read by the dense product). */
+/* x <- V x for a whitening V given as (code, matrix M in LDS, diag d, r the
+ * reciprocals of a triangular M's diagonal); src is x's column in global memory
+ * (re-read by the dense product). */
 template <int NB>
 __device__ __forceinline__ void apply_weight(double (&x)[NB], int m, int code, const double* M, const double* d,
-                                             const double* src, int src_is_identity_col) {
+                                             const double* r, const double* src, int src_is_identity_col) {
   if (code == UK_COV_w) {
 #pragma unroll
     for (int i = 0; i < NB; ++i)
@@ -954,14 +1003,15 @@ __device__ __forceinline__ void apply_weight(double (&x)[NB], int m, int code, c
       for (int i = 0; i < NB; ++i)
         if (i < m) x[i] = fma(M[i + pp * m], xp, x[i]);
     }
-  } else { /* lower-triangular solve with M (Cholesky factor or given L) */
+  } else { /* lower-triangular solve with M (Cholesky factor or given L), by columns: independent updates; the
+            * quotient by the reciprocal and one correction, which rounds like a division */
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      if (i < m) {
-        double s = x[i];
+    for (int pp = 0; pp < NB; ++pp) {
+      if (pp < m) {
+        const double q = x[pp] * r[pp];
+        x[pp] = fma(fma(-M[pp + pp * m], q, x[pp]), r[pp], q);
 #pragma unroll
-        for (int pp = 0; pp < i; ++pp) s = fma(-M[i + pp * m], x[pp], s);
-        x[i] = s / M[i + i * m];
+        for (int i = pp + 1; i < NB; ++i) x[i] = fma(-M[i + pp * m], x[pp], x[i]); /* rows from m on are not used */
       }
     }
   }
@@ -1003,8 +1053,17 @@ __global__ void __launch_bounds__(((3 * NB + 2 + 63) / 64) * 64)
     }
   }
   __syncthreads();
-  if (!first && kt == UK_COV_C) lds_cholesky<NT>(sh.K, n, tid);
-  if (m > 0 && ct == UK_COV_C) lds_cholesky<NT>(sh.C, m, tid);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  if (!first && w == 0) {
+    if (kt == UK_COV_C) wave_cholesky<NB>(sh.K, sh.rk, n, lane);
+    else if (kt == UK_COV_L)
+      for (int i = lane; i < n; i += 64) sh.rk[i] = 1.0 / sh.K[i + i * n];
+  }
+  if (m > 0 && w == NT / 64 - 1) {
+    if (ct == UK_COV_C) wave_cholesky<NB>(sh.C, sh.rc, m, lane);
+    else if (ct == UK_COV_L)
+      for (int i = lane; i < m; i += 64) sh.rc[i] = 1.0 / sh.C[i + i * m];
+  }
   __syncthreads();
 
   double x[NB];
@@ -1027,7 +1086,7 @@ __global__ void __launch_bounds__(((3 * NB + 2 + 63) / 64) * 64)
     }
     const double* src = q < n ? raw.F + raw.Fidx[s] * nn + (int64_t)q * n
                         : (q < 2 * n ? (raw.H_ident ? nullptr : raw.H + s * nn + (int64_t)(q - n) * n) : raw.c + s * n);
-    apply_weight<NB>(x, n, kt, sh.K, sh.K, src, (q >= n && q < 2 * n && raw.H_ident) ? q - n : -1);
+    apply_weight<NB>(x, n, kt, sh.K, sh.K, sh.rk, src, (q >= n && q < 2 * n && raw.H_ident) ? q - n : -1);
     if (q < n) {
       double* dst = out.B + s * nn + (int64_t)q * n;
 #pragma unroll
@@ -1050,7 +1109,7 @@ __global__ void __launch_bounds__(((3 * NB + 2 + 63) / 64) * 64)
       const double* src = is_o ? raw.o + s * mr : raw.G + s * mr * n + (int64_t)qq * mr;
 #pragma unroll
       for (int i = 0; i < NB; ++i) x[i] = (i < m) ? src[i] : 0.0;
-      apply_weight<NB>(x, m, ct, sh.C, sh.C, src, -1);
+      apply_weight<NB>(x, m, ct, sh.C, sh.C, sh.rc, src, -1);
     } else {
 #pragma unroll
       for (int i = 0; i < NB; ++i) x[i] = 0.0;
@@ -1203,7 +1262,7 @@ __global__ void __launch_bounds__((QRGeom<NB, NB + 1, 3>::NT))
 template <int NB>
 __global__ void __launch_bounds__(64) k_cov_format(const double* __restrict__ S, int n, int fmt,
                                                    double* __restrict__ dst) {
-  __shared__ double L[NB * NB];
+  __shared__ double L[NB * NB], r[NB];
   const int tid = threadIdx.x;
   const int64_t s = blockIdx.x;
   const int64_t nn = (int64_t)n * n;
@@ -1214,7 +1273,8 @@ __global__ void __launch_bounds__(64) k_cov_format(const double* __restrict__ S,
   }
   for (int i = tid; i < n * n; i += 64) L[i] = Ss[i];
   __syncthreads();
-  lds_cholesky<64>(L, n, tid); /* lower factor in place, ld n (ends with a barrier) */
+  wave_cholesky<NB>(L, r, n, tid); /* lower factor in place, ld n */
+  __syncthreads();
   if (tid < n) {
     const int j = tid;
     double x[NB];
