@@ -912,6 +912,8 @@ __global__ void __launch_bounds__(256)
 /* whitening (level-0 chain)                                                  */
 /* ------------------------------------------------------------------------ */
 
+/* ld NB; the identity beyond the covariances' rows and columns, so that nothing
+ * below asks for them */
 template <int NB>
 struct WeighShared {
   double K[NB * NB];
@@ -919,14 +921,14 @@ struct WeighShared {
   double rk[NB], rc[NB]; /* reciprocals of a triangular K's and C's diagonal */
 };
 
-/* In-place lower Cholesky of an m x m matrix (ld m) in LDS by one wave, the
+/* In-place lower Cholesky of an m x m matrix (ld) in LDS by one wave, the
  * upper tiles in its registers: row tiles by the inverse factor of the panel's
  * diagonal tile, the tiles below updated on the matrix cores; r: the
  * reciprocals of the factor's diagonal. A column at a time by the workgroup,
  * with three barriers, it was most of k_weigh: 209 us for
- * 300 steps of n = 45 with full covariances, 89 now. */
+ * 300 steps of n = 45 with full covariances. */
 template <int NB>
-__device__ void wave_cholesky(double* A, double* r, int m, int lane) {
+__device__ void wave_cholesky(double* A, int ld, double* r, int m, int lane) {
   constexpr int NT = (NB + 15) / 16;
   const int li = lane & 15, lk = lane >> 4;
   as_d4 M[NT][NT];
@@ -938,7 +940,7 @@ __device__ void wave_cholesky(double* A, double* r, int m, int lane) {
       for (int g = 0; g < 4; ++g) { /* the transposes of A's lower tiles */
         const int row = 16 * j + li, col = 16 * i + 4 * g + lk;
         const bool in = row < m && col < m;
-        const double x = A[in ? (row >= col ? row + col * m : col + row * m) : 0];
+        const double x = A[in ? (row >= col ? row + col * ld : col + row * ld) : 0];
         M[i][j][g] = in ? x : (row == col ? 1.0 : 0.0);
       }
 #pragma unroll
@@ -980,39 +982,36 @@ __device__ void wave_cholesky(double* A, double* r, int m, int lane) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int row = 16 * j + li, col = 16 * i + 4 * g + lk;
-        if (row < m && col <= row) A[row + col * m] = M[i][j][g];
+        if (row < m && col <= row) A[row + col * ld] = M[i][j][g];
       }
 }
 
-/* x <- V x for a whitening V given as (code, matrix M in LDS, diag d, r the
- * reciprocals of a triangular M's diagonal); src is x's column in global memory
- * (re-read by the dense product). */
+/* x <- V x for a whitening V given as (code, matrix M in LDS or its diagonal in
+ * M's first column, r the reciprocals of a triangular M's diagonal), x zero
+ * from row m on; src is x's column in global memory (re-read by the dense
+ * product), or idcol >= 0 the column of the identity that x is. */
 template <int NB>
-__device__ __forceinline__ void apply_weight(double (&x)[NB], int m, int code, const double* M, const double* d,
-                                             const double* r, const double* src, int src_is_identity_col) {
+__device__ __forceinline__ void apply_weight(double (&x)[NB], int m, int code, const double* M, const double* r,
+                                             const double* src, int idcol) {
   if (code == UK_COV_w) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (i < m) x[i] *= d[i];
+    for (int i = 0; i < NB; ++i) x[i] *= M[i];
   } else if (code == UK_COV_W) {
 #pragma unroll
     for (int i = 0; i < NB; ++i) x[i] = 0.0;
     for (int pp = 0; pp < m; ++pp) {
-      const double xp = src_is_identity_col >= 0 ? (pp == src_is_identity_col ? 1.0 : 0.0) : src[pp];
+      const double xp = idcol >= 0 ? (pp == idcol ? 1.0 : 0.0) : src[pp];
 #pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i < m) x[i] = fma(M[i + pp * m], xp, x[i]);
+      for (int i = 0; i < NB; ++i) x[i] = fma(M[i + pp * NB], xp, x[i]);
     }
   } else { /* lower-triangular solve with M (Cholesky factor or given L), by columns: independent updates; the
             * quotient by the reciprocal and one correction, which rounds like a division */
 #pragma unroll
     for (int pp = 0; pp < NB; ++pp) {
-      if (pp < m) {
-        const double q = x[pp] * r[pp];
-        x[pp] = fma(fma(-M[pp + pp * m], q, x[pp]), r[pp], q);
+      const double q = x[pp] * r[pp];
+      x[pp] = fma(fma(-M[pp + pp * NB], q, x[pp]), r[pp], q);
 #pragma unroll
-        for (int i = pp + 1; i < NB; ++i) x[i] = fma(-M[i + pp * m], x[pp], x[i]); /* rows from m on are not used */
-      }
+      for (int i = pp + 1; i < NB; ++i) x[i] = fma(-M[i + pp * NB], x[pp], x[i]);
     }
   }
 }
@@ -1038,87 +1037,73 @@ __global__ void __launch_bounds__(((3 * NB + 2 + 63) / 64) * 64)
   const bool first = raw.first[s] != 0;
   const int kt = raw.Kt[s], ct = raw.Ct[s];
 
-  if (!first) {
-    if (raw.K_full) {
-      for (int i = tid; i < n * n; i += NT) sh.K[i] = raw.K[s * nn + i];
-    } else {
-      for (int i = tid; i < n; i += NT) sh.K[i] = raw.K[s * n + i];
-    }
-  }
-  if (m > 0) {
-    if (raw.C_full) {
-      for (int i = tid; i < m * m; i += NT) sh.C[i] = raw.C[s * mr * mr + (i % m) + (int64_t)(i / m) * mr];
-    } else {
-      for (int i = tid; i < m; i += NT) sh.C[i] = raw.C[s * mr + i];
-    }
-  }
-  __syncthreads();
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  if (!first && w == 0) {
-    if (kt == UK_COV_C) wave_cholesky<NB>(sh.K, sh.rk, n, lane);
-    else if (kt == UK_COV_L)
-      for (int i = lane; i < n; i += 64) sh.rk[i] = 1.0 / sh.K[i + i * n];
+  constexpr int NW = NT / 64;
+#pragma unroll
+  for (int u = 0; u < (NB * NB + NT - 1) / NT; ++u) {
+    const int idx = tid + u * NT, i = idx % NB, c = idx / NB;
+    if (idx < NB * NB) {
+      double kv = i == c ? 1.0 : 0.0, cv = kv;
+      if (!first && i < n && c < n) kv = raw.K_full ? raw.K[s * nn + i + c * n] : (c == 0 ? raw.K[s * n + i] : 0.0);
+      if (i < m && c < m) cv = raw.C_full ? raw.C[s * mr * mr + i + c * mr] : (c == 0 ? raw.C[s * mr + i] : 0.0);
+      sh.K[idx] = kv;
+      sh.C[idx] = cv;
+    }
   }
-  if (m > 0 && w == NT / 64 - 1) {
-    if (ct == UK_COV_C) wave_cholesky<NB>(sh.C, sh.rc, m, lane);
-    else if (ct == UK_COV_L)
-      for (int i = lane; i < m; i += 64) sh.rc[i] = 1.0 / sh.C[i + i * m];
+  if (tid < NB) sh.rk[tid] = sh.rc[tid] = 1.0;
+  __syncthreads();
+  /* K on the first wave, C on the last: the same code, which the instruction
+   * cache holds once (both inlined, and a copy of the columns' loads, weights
+   * and stores per kind of column: 89 us for 300 steps of n = 45, 64 like this) */
+  if (w == 0 || w == NW - 1) {
+#pragma unroll 1
+    for (int role = w == 0 ? 0 : 1; role < 2; role += NW) {
+      double *A = role ? sh.C : sh.K, *r = role ? sh.rc : sh.rk;
+      const int dim = role ? m : (first ? 0 : n), code = role ? ct : kt;
+      if (dim > 0 && code == UK_COV_C) wave_cholesky<NB>(A, NB, r, dim, lane);
+      if (code == UK_COV_L)
+        for (int i = lane; i < dim; i += 64) r[i] = 1.0 / A[i * (NB + 1)];
+    }
   }
   __syncthreads();
 
-  double x[NB];
   const int q = tid;
-  if (q < 2 * n + 1) {
-    if (first) { /* no evolution equation on a chain's first step */
-      return;
-    }
-    if (q < n) {
-      const double* src = raw.F + raw.Fidx[s] * nn + (int64_t)q * n;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) x[i] = (i < n) ? src[i] : 0.0;
-    } else if (q < 2 * n) {
-      const int qq = q - n;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) x[i] = (i < n) ? (raw.H_ident ? (i == qq ? 1.0 : 0.0) : raw.H[s * nn + (int64_t)qq * n + i]) : 0.0;
-    } else {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) x[i] = (i < n) ? raw.c[s * n + i] : 0.0;
-    }
-    const double* src = q < n ? raw.F + raw.Fidx[s] * nn + (int64_t)q * n
-                        : (q < 2 * n ? (raw.H_ident ? nullptr : raw.H + s * nn + (int64_t)(q - n) * n) : raw.c + s * n);
-    apply_weight<NB>(x, n, kt, sh.K, sh.K, sh.rk, src, (q >= n && q < 2 * n && raw.H_ident) ? q - n : -1);
-    if (q < n) {
-      double* dst = out.B + s * nn + (int64_t)q * n;
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i < n) dst[i] = -x[i];
-    } else if (q < 2 * n) {
-      double* dst = out.D + s * nn + (int64_t)(q - n) * n;
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i < n) dst[i] = x[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i < n) out.c[s * n + i] = x[i];
-    }
-  } else if (q < 3 * n + 2) {
-    const bool is_o = q == 3 * n + 1;
-    const int qq = q - 2 * n - 1;
-    if (m > 0) {
-      const double* src = is_o ? raw.o + s * mr : raw.G + s * mr * n + (int64_t)qq * mr;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) x[i] = (i < m) ? src[i] : 0.0;
-      apply_weight<NB>(x, m, ct, sh.C, sh.C, sh.rc, src, -1);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NB; ++i) x[i] = 0.0;
-    }
-    double* dst = is_o ? out.o + s * ost : out.C + s * cst + (int64_t)qq * mr;
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (i < mr) dst[i] = (i < m) ? x[i] : 0.0;
+  const bool evo = q < 2 * n + 1;
+  if (q >= 3 * n + 2 || (evo && first)) return; /* no evolution equation on a chain's first step */
+  const int dim = evo ? n : m, rows = evo ? n : mr, code = evo ? kt : ct;
+  const double *M = evo ? sh.K : sh.C, *r = evo ? sh.rk : sh.rc;
+  const int idcol = q >= n && q < 2 * n && raw.H_ident ? q - n : -1;
+  const double* src;
+  double* dst;
+  if (q < n) {
+    src = raw.F + raw.Fidx[s] * nn + (int64_t)q * n;
+    dst = out.B + s * nn + (int64_t)q * n;
+  } else if (q < 2 * n) {
+    src = raw.H_ident ? raw.c + s * n : raw.H + s * nn + (int64_t)(q - n) * n;
+    dst = out.D + s * nn + (int64_t)(q - n) * n;
+  } else if (evo) {
+    src = raw.c + s * n;
+    dst = out.c + s * n;
+  } else if (q < 3 * n + 1) {
+    src = raw.G + s * mr * n + (int64_t)(q - 2 * n - 1) * mr;
+    dst = out.C + s * cst + (int64_t)(q - 2 * n - 1) * mr;
+  } else {
+    src = raw.o + s * mr;
+    dst = out.o + s * ost;
   }
+  double x[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) x[i] = 0.0;
+  if (dim > 0) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) x[i] = src[i < dim ? i : dim - 1];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) x[i] = i < dim ? (idcol >= 0 ? (i == idcol ? 1.0 : 0.0) : x[i]) : 0.0;
+    apply_weight<NB>(x, dim, code, M, r, src, idcol);
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    if (i < rows) dst[i] = i < dim ? (q < n ? -x[i] : x[i]) : 0.0;
 }
 
 /*
@@ -1273,7 +1258,7 @@ __global__ void __launch_bounds__(64) k_cov_format(const double* __restrict__ S,
   }
   for (int i = tid; i < n * n; i += 64) L[i] = Ss[i];
   __syncthreads();
-  wave_cholesky<NB>(L, r, n, tid); /* lower factor in place, ld n */
+  wave_cholesky<NB>(L, n, r, n, tid); /* lower factor in place, ld n */
   __syncthreads();
   if (tid < n) {
     const int j = tid;

@@ -39,7 +39,7 @@ def base_name(name):
     """The kernel without its launch-variant template arguments
     ("k_phase1<48, double, 2, 2, true>" -> "k_phase1<48, double>"): the
     variants move the same bytes, so traffic is keyed by the base name."""
-    m = re.match(r"^(k_phase\d<\d+, (?:double|float))(?:, [^>]*)?>$", name)
+    m = re.match(r"^((?:k_phase\d|k_mid\d|k_level_small)<\d+, (?:double|float))(?:, [^>]*)?>$", name)
     return m.group(1) + ">" if m else name
 
 
