@@ -164,21 +164,25 @@ def headline_traffic(kernel, specs, sample=600):
     if t is None:
         return None
     nb = int(base.split("<")[1].split(",")[0])
-    k_sample = sum(sp["k"] for sp in P.batch_specs(count=sample) if bucket_qr(sp["n"]) == nb)
-    k_all = sum(sp["k"] for sp in specs if bucket_qr(sp["n"]) == nb)
+    if base.startswith(("k_mid", "k_level_small")):  # compiled by row granules of four
+        group = lambda sp: (sp["n"] + 3) // 4 == nb
+    else:
+        group = lambda sp: bucket_qr(sp["n"]) == nb
+    k_sample = sum(sp["k"] for sp in P.batch_specs(count=sample) if group(sp))
+    k_all = sum(sp["k"] for sp in specs if group(sp))
     if k_sample == 0:
         return None
     f = k_all / k_sample
     alg = None
-    if base.startswith("k_phase2<") and ", float>" in base:
+    if base.startswith(("k_phase2<", "k_mid2<")) and ", float>" in base:
         # the FP32 levels (0-7) of the mixed path; level 0 with D diagonal and B formed on load (K, C given as 'w')
         alg = sum(flops.oddeven_phase2_bytes(sp["n"], sp["k"], fp32_levels=8, level0_diag_synth=True)
-                  for sp in specs if bucket_qr(sp["n"]) == nb)
+                  for sp in specs if group(sp))
     meas = t["bytes_per_step"] * f
     return {"bytes_per_step": meas, "fetch_bytes": t["fetch_bytes"] * f,
             "write_bytes": t["write_bytes"] * f, "algorithmic_bytes_per_step": alg,
             "measured_over_algorithmic": (meas / alg) if alg else None,
-            "source": f"profiles/traffic.json, batch_mixed_chunk{sample} ({base}), x{f:.3f}: bucket-{nb} time steps "
+            "source": f"profiles/traffic.json, batch_mixed_chunk{sample} ({base}), x{f:.3f}: its time steps "
                       f"of the workload over the sample's"}
 
 

@@ -27,11 +27,8 @@ constexpr int MID_WAVES = 4; /* waves (work items) per workgroup */
  * fetching of their straight-line code leave a lone wave's SIMD idle more than
  * half of the time, so a second or third wave is worth a few spilled
  * registers. */
-#ifndef UK_MID_D2
-#define UK_MID_D2 2
-#endif
 __host__ __device__ constexpr int mid_occ(int NK, int phase, bool fp32) {
-  if (phase == 2) return fp32 ? (NK <= 6 ? 4 : 3) : (NK <= 6 ? 2 : UK_MID_D2);
+  if (phase == 2) return fp32 ? (NK <= 6 ? 4 : 3) : 2;
   return fp32 ? (phase == 1 ? 4 : 5) : 2;
 }
 
@@ -431,11 +428,12 @@ __global__ void __launch_bounds__(64 * MidLevel<NK>::WAVES)
   if (has_lone) __syncthreads();
 }
 
-/* Levels of at most this many pairs take k_mid_level: two workgroups per CU. */
-#ifndef UK_MID_SPLIT
-#define UK_MID_SPLIT 512
-#endif
-constexpr int64_t MID_SPLIT = UK_MID_SPLIT;
+/* Levels of at most this many pairs take k_mid_level: two workgroups per CU.
+ * Smoothing n = 32 without covariances, never / up to this line / always: k =
+ * 500 679 / 501 / 499 us, k = 4000 1011 / 768 / 804, k = 16000 1804 / 1557 / 1962
+ * (FP32 elimination 1529 / 1290 / 1686); n = 24: k = 500 375 / 290 / 290, k =
+ * 16000 959 / 836 / 938. */
+constexpr int64_t MID_SPLIT = 512;
 
 template <class T>
 bool mid_one_launch(const uk_level_t* lv, const ChainT<T>& in) {

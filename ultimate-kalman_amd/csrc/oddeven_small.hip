@@ -177,12 +177,12 @@ __global__ void __launch_bounds__(256)
   if (split && has_lone && wave != 1) __syncthreads(); /* wave 1 waits for it in phase 3 */
 }
 
-/* A level of at most this many pairs gives each pair three waves: it then has
- * at most as many waves as the chip has SIMDs. */
-#ifndef UK_SM_SPLIT
-#define UK_SM_SPLIT 1024
-#endif
-constexpr int64_t SM_SPLIT = UK_SM_SPLIT;
+/* A level of at most this many pairs gives each pair three waves: beyond, the
+ * pairs alone give every SIMD of the chip (1,024) a wave. Smoothing n = 16
+ * without covariances, never / up to this line / always three waves: k = 500
+ * 226 / 155 / 155 us, k = 4000 324 / 260 / 270, k = 16000 485 / 421 / 495 (FP32
+ * elimination 469 / 399 / 453). */
+constexpr int64_t SM_SPLIT = 1024;
 
 template <int NK, class T>
 void launch_nk(const uk_level_t* lv, const ChainT<T>& in, const ChainT<T>& out, const FactorsT<T>& fac, int n,

@@ -1,8 +1,10 @@
 /*
  * oddeven_wave.h -- Householder QR of a stacked pair of blocks on one wave
  * (n <= 32), shared by oddeven_small.hip (n <= 16, the three phases of a step
- * pair in one kernel) and oddeven_wave{20,24,28,32}.hip (16 < n <= 32, a kernel
- * per phase).
+ * pair in one kernel), oddeven_mid{20,24,28,32}.hip (16 < n <= 32, a kernel per
+ * phase or per short level) and filter_small.hip; and a Cholesky factorization
+ * of matrix-core tiles (n <= 64), shared by associative.hip and the dense
+ * whitening of oddeven.hip.
  *
  * Layout: 16 matrix columns are a tile; lane (li, lk) = (lane % 16, lane / 16)
  * holds rows 4 g + lk, g = 0 .. NK - 1, of the tile's column li in NK = ceil(n
